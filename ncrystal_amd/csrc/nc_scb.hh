@@ -128,31 +128,57 @@ NCD double gci_sum(const SCBView& v, const GCI& g, unsigned n, double off, doubl
   do { sum += gci_f(v, g, gr.c); } while (gr.step());
   return sum;
 }
-// Romberg integration of the mosaic density along the circle, t in [a,b]
-__device__ __noinline__ double gci_integrate(const SCBView& v, const GCI& g, double a, double b) {
+// Romberg integration of the mosaic density along the circle, t in [a,b].
+// The 17 points of the first five rows are added to their groups (ends, eighth
+// point, quarters, eighths, sixteenths; pairwise, in the order of the
+// reference's expressions) as they come: an array of them would hold 34
+// registers in every kernel that can meet this integral.
+NCD double gci_integrate(const SCBView& v, const GCI& g, double a, double b) {
   double h = (b - a);
-  double fv[17];
+  double s_end = 0.0, s_mid = 0.0, s_q = 0.0, s_e = 0.0, s_s = 0.0;
   {
     CSGrid gr;
     gr.init(17, a, h * 0.0625);
-    unsigned i = 0;
-    do { fv[i++] = gci_f(v, g, gr.c); } while (gr.step());
+    double x0 = 0.0, e0 = 0.0;
+#pragma nounroll
+    for (int k = 0; k < 4; ++k) {  // points 4k .. 4k+3
+      const double p = gci_f(v, g, gr.c);
+      if (k == 0) s_end = p;
+      else if (k == 2) s_mid = p;
+      else s_q = k == 1 ? p : s_q + p;
+      gr.step();
+      double x = gci_f(v, g, gr.c);
+      gr.step();
+      double e = gci_f(v, g, gr.c);
+      gr.step();
+      x += gci_f(v, g, gr.c);
+      gr.step();
+      if (k & 1) {
+        x = x0 + x;
+        e = e0 + e;
+        s_s = k == 1 ? x : s_s + x;
+        s_e = k == 1 ? e : s_e + e;
+      }
+      x0 = x;
+      e0 = e;
+    }
+    s_end += gci_f(v, g, gr.c);  // 16
   }
   h *= 0.5;
-  const double R00 = (fv[0] + fv[16]) * h;
-  const double R10 = h * fv[8] + 0.5 * R00;
+  const double R00 = s_end * h;
+  const double R10 = h * s_mid + 0.5 * R00;
   const double R11 = (4. / 3.) * R10 + (-1. / 3.) * R00;
   h *= 0.5;
-  const double R20 = h * (fv[4] + fv[12]) + 0.5 * R10;
+  const double R20 = h * s_q + 0.5 * R10;
   const double R21 = (4. / 3.) * R20 + (-1. / 3.) * R10;
   const double R22 = (16. / 15.) * R21 + (-1. / 15.) * R11;
   h *= 0.5;
-  const double R30 = h * ((fv[2] + fv[6]) + (fv[10] + fv[14])) + 0.5 * R20;
+  const double R30 = h * s_e + 0.5 * R20;
   const double R31 = (4. / 3.) * R30 + (-1. / 3.) * R20;
   const double R32 = (16. / 15.) * R31 + (-1. / 15.) * R21;
   const double R33 = (64. / 63.) * R32 + (-1. / 63.) * R22;
   h *= 0.5;
-  const double R40 = h * (((fv[1] + fv[3]) + (fv[5] + fv[7])) + ((fv[9] + fv[11]) + (fv[13] + fv[15]))) + 0.5 * R30;
+  const double R40 = h * s_s + 0.5 * R30;
   const double R41 = (4. / 3.) * R40 + (-1. / 3.) * R30;
   const double R42 = (16. / 15.) * R41 + (-1. / 15.) * R31;
   const double R43 = (64. / 63.) * R42 + (-1. / 63.) * R32;

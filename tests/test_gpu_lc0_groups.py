@@ -1,0 +1,73 @@
+"""Layered-crystal kernel (lcmode=0) at the edges of its work split: the
+neutrons per workgroup follow from the batch size, the ranges are integrated in
+rounds of a workgroup's list, and sampling finds its range in the round or, for
+more plane sets than a round's masks hold, in a second pass.  None of that may
+change a neutron's value."""
+import math
+
+import numpy as np
+import pytest
+
+from test_lcbragg_checker import FIX, WL2EKIN, checker_crystal, graphite_inputs, lchelper
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def core():
+    from ncrystal_amd import _capi, core
+    if _capi.lib().ncamd_device_count() < 1:
+        pytest.fail("no GPU visible to libncrystal_amd")
+    return core
+
+
+def _layered(core, dcutoff, mosaic):
+    def msd(e, d, T, m):
+        return core.vdos_analyse((e, d), T, m)["msd"]
+    cell, sp, v0n = graphite_inputs(msd)
+    _, _, dsp, fsq, moff, mh = core.hkl_spacegroup_members(FIX["spacegroup"], cell, sp, dcutoff)
+    return core.create_lcbragg(v0n, dsp, fsq, moff, mh, core.reci_lattice(cell), np.eye(3), FIX["lcaxis"],
+                               math.radians(mosaic))
+
+
+def _neutrons(n, lo, hi, seed):
+    rng = np.random.default_rng(seed)
+    d = rng.normal(size=(n, 3))
+    return WL2EKIN / rng.uniform(lo, hi, n) ** 2, d / np.linalg.norm(d, axis=1)[:, None]
+
+
+# 0.5-0.7 Aa: all plane sets in reach, several rounds per workgroup and, at 5
+# degrees, ranges with backscattering points; 2.2-7 Aa: mostly none or a few
+@pytest.mark.parametrize("lo,hi,mosaic", [(0.5, 0.7, 1.0), (0.5, 0.7, 5.0), (2.2, 7.0, 4.0)])
+def test_batch_size_changes_nothing(core, lo, hi, mosaic):
+    lc = _layered(core, 0.5, mosaic)
+    n = 33000  # 64 neutrons per workgroup; the calls below use 4, 8, 16 and 32
+    e, d = _neutrons(n, lo, hi, 3)
+    xs = lc.crossSection(e, d)
+    lc.setRNGState(17, 0)
+    oe, od = lc.sampleScatter(e, d)
+    assert np.array_equal(oe, e) and np.allclose(np.linalg.norm(od, axis=1), 1.0, atol=1e-12)
+    for m in (1, 3, 63, 65, 2049, 5000, 9001, 20000):
+        assert np.array_equal(lc.crossSection(e[:m], d[:m]), xs[:m])
+        lc.setRNGState(17, 0)
+        assert np.array_equal(lc.sampleScatter(e[:m], d[:m])[1], od[:m])
+
+
+def test_more_plane_sets_than_a_round(core, oracle):
+    """dcutoff 0.2 Aa gives the crystal over 256 plane sets; neutrons that
+    reach only those down to 0.5 Aa see the same crystal as without the rest
+    (same sums: identical), others are compared with the checker"""
+    small, large = _layered(core, 0.5, 4.0), _layered(core, 0.2, 4.0)
+    e, d = _neutrons(3000, 1.01, 3.0, 5)
+    assert np.array_equal(small.crossSection(e, d), large.crossSection(e, d))
+    for lc in (small, large):
+        lc.setRNGState(4, 0)
+    assert np.array_equal(small.sampleScatter(e, d)[1], large.sampleScatter(e, d)[1])
+    o, fam = checker_crystal(oracle, 0.2)
+    e, d = _neutrons(40, 0.41, 0.6, 6)
+    got, want = large.crossSection(e, d), lchelper(oracle, o, fam).xs_dir(e, d)
+    # the bound of the checker comparison of this model: device cosines in
+    # ranges that lose up to 1e5 of their argument's precision
+    assert np.max(np.abs(got - want) / want) < 1e-10
+    gd = large.sampleScatter(e, d)[1]
+    assert np.allclose(np.linalg.norm(gd, axis=1), 1.0, atol=1e-12)
