@@ -1717,10 +1717,12 @@ Proc* create_scb(double v0n, int64_t nfam, const double* dsp, const double* fsq,
   v.nrec = b_nrec->as<double4>();
   v.nrec32 = b_nrec32->as<float4>();
   v.nfx = b_nfx->as<double2>();
-  // |sin(phi) - sin(theta)| <= |phi - theta| < truncation angle for every
-  // contributing normal; the margins cover the rounding of cos(truncation)
-  // (~1e-14) and of the FP32 records and products of the pre-filter (< 3e-6)
-  v.band32 = (float)(trunc * (1.0 + 1e-6) + 1e-5);
+  // pre-filter of the scan (scb_prefilter); the factor covers the rounding of
+  // cos(truncation) (~1e-14) and of these constants
+  const double T = trunc * (1.0 + 1e-6);
+  v.band_hT2 = (float)(0.5 * T * T);
+  v.band_T2 = (float)(T * T);
+  v.band_T2c = (float)(T * T * (1.0 + 1e-6));
   {
     const double w = maxd * 2.0, w2 = w * w;
     v.threshold = w2 ? kWl2Ekin / w2 : __builtin_huge_val();
