@@ -1703,6 +1703,13 @@ Proc* create_scb(double v0n, int64_t nfam, const double* dsp, const double* fsq,
   DevBuf* b_inv2d = p->newbuf(); b_inv2d->upload(inv2d.data(), inv2d.size());
   DevBuf* b_xsf = p->newbuf(); b_xsf->upload(xsf.data(), xsf.size());
   DevBuf* b_off = p->newbuf(); b_off->upload(off32.data(), off32.size());
+  const double f_scale = kScbGuide / inv2d[nf - 1];
+  std::vector<int> f_guide(kScbGuide + 1, nf);
+  for (int g = 0, f = 0; g < kScbGuide; ++g) {
+    while (f < nf && inv2d[f] < g / f_scale) ++f;
+    f_guide[g] = f;
+  }
+  DevBuf* b_guide = p->newbuf(); b_guide->upload(f_guide.data(), f_guide.size());
   DevBuf* b_nrec = p->newbuf(); b_nrec->upload(nrec.data(), nrec.size());
   DevBuf* b_nrec32 = p->newbuf(); b_nrec32->upload(nrec32.data(), nrec32.size());
   DevBuf* b_nfx = p->newbuf(); b_nfx->upload(nfx.data(), nfx.size());
@@ -1714,6 +1721,8 @@ Proc* create_scb(double v0n, int64_t nfam, const double* dsp, const double* fsq,
   v.inv2d = b_inv2d->as<double>();
   v.xsf = b_xsf->as<double>();
   v.off = b_off->as<int>();
+  v.f_guide = b_guide->as<int>();
+  v.f_scale = f_scale;
   v.nrec = b_nrec->as<double4>();
   v.nrec32 = b_nrec32->as<float4>();
   v.nfx = b_nfx->as<double2>();

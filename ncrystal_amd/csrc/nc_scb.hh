@@ -43,6 +43,8 @@ struct SCBView {
   const double* __restrict__ inv2d;     // [nfam] 1/(2d), non-decreasing
   const double* __restrict__ xsf;       // [nfam] |F|^2/(V0 n) * 0.5
   const int* __restrict__ off;          // [nfam+1] demi-normal offsets
+  const int* __restrict__ f_guide;      // [kScbGuide+1] lower_bound(inv2d, g / f_scale), last entry nfam
+  double f_scale;                       // kScbGuide / inv2d[nfam-1]
   // one record per demi-normal in scan order: lab-frame unit normal and the
   // family's 1/(2d) rounded to 1e-15 (GaussMos cache rounding)
   const double4* __restrict__ nrec;     // [nnormals + kScbPad]
@@ -55,6 +57,8 @@ struct SCBView {
   float band_hT2, band_T2, band_T2c;
   SplineView lt_evalcosx, lt_sofcosd;
 };
+
+constexpr int kScbGuide = 4096;
 
 // scan group size; the record arrays carry this many padding entries so
 // that a group never reads past the end
@@ -492,7 +496,7 @@ struct ScbLane {
 // order and accumulates them; all lanes of the wave call this together.
 // Select=false: count and cumulative total.  Select=true: stop at the
 // contribution picked by pickRandIdxByWeight for (n_select, target).
-template <bool Select, bool AllowSlow>
+template <bool Select>
 NCD void scb_eval_list(const SCBView& v, ScbLane& L, ScbAcc& a, bool& alive, const uint16_t* __restrict__ list,
                        int base, int n, double w, double wl3, int n_select, double target) {
   const int lane = (int)__lane_id();
@@ -509,7 +513,7 @@ NCD void scb_eval_list(const SCBView& v, ScbLane& L, ScbAcc& a, bool& alive, con
       a.xssum = 0.0;
     }
     double xs2[2];
-    if (!scb_candidate<AllowSlow>(v, r, fx.x, w, wl3, L.u.x, L.u.y, L.u.z, xs2[0], xs2[1])) {
+    if (!scb_candidate<false>(v, r, fx.x, w, wl3, L.u.x, L.u.y, L.u.z, xs2[0], xs2[1])) {
       L.slow = true;
       alive = false;
       continue;
@@ -586,12 +590,9 @@ constexpr double kScbCoarseChord = 0.2;
 //    The normals left are broadcast (readlane) and pre-filtered per lane.
 //  - dense: every lane pre-filters every normal, in groups of kScbGroup with
 //    a wave-uniform index (scalar loads of the FP32 records).
-// `complete` is set (wave-uniform) when the list held every candidate of the
-// scan, so that a second pass can evaluate it without scanning again.  All
-// lanes of the wavefront must call this together.
-template <bool Select, bool AllowSlow>
-NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uint16_t* __restrict__ list,
-                  int& nlist, bool& complete) {
+// All lanes of the wavefront must call this together.
+template <bool Select>
+NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uint16_t* __restrict__ list) {
   L.count = 0;
   L.total = 0.0;
   L.slow = false;
@@ -604,7 +605,6 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
   const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
   ScbAcc a{-1, 0.0, 0.0, 0.0};
   int n = 0, base = 0;
-  complete = true;
   // bounds of the wave: mean direction, chord, wavelength range
   const double mx0 = wave_sum_d(alive ? L.u.x : 0.0), my0 = wave_sum_d(alive ? L.u.y : 0.0),
                mz0 = wave_sum_d(alive ? L.u.z : 0.0);
@@ -633,10 +633,9 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
       uint64_t M = __ballot(pass);
       if (!M) continue;
       if (__any(n + __popcll(M) > kScbListCap) || jb + 64 - base > kScbListSpan) {
-        scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
+        scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
         n = 0;
         base = jb;
-        complete = false;
         if (!__any(alive)) break;
       }
       while (M) {
@@ -654,10 +653,9 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
   } else {
     for (int jb = 0; jb < jmax; jb += kScbGroup) {
       if (__any(n > kScbListCap - kScbGroup) || jb + kScbGroup - base > kScbListSpan) {
-        scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
+        scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
         n = 0;
         base = jb;
-        complete = false;
         if (!__any(alive)) break;
       }
       unsigned cand = 0u;
@@ -677,24 +675,8 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
       }
     }
   }
-  scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
-  nlist = n;
+  scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
   L.total = a.commul_last;
-}
-
-// Second pass over a complete list (scb_walk set `complete`): the same
-// contributions as scb_walk<Select> without scanning again.
-template <bool AllowSlow>
-NCD void scb_select_list(const SCBView& v, ScbLane& L, int n_select, double target, const uint16_t* __restrict__ list,
-                         int nlist) {
-  L.count = 0;
-  L.slow = false;
-  L.found = false;
-  bool alive = L.jlim > 0;
-  const double w = gm_round(L.wl);
-  const double wl3 = w * w * w;
-  ScbAcc a{-1, 0.0, 0.0, 0.0};
-  scb_eval_list<true, AllowSlow>(v, L, a, alive, list, 0, alive ? nlist : 0, w, wl3, n_select, target);
 }
 
 // per-lane set-up of a neutron (NCSCBragg.cc:233-259): returns false when
@@ -709,7 +691,12 @@ NCD bool scb_lane_setup(const SCBView& v, double E, double dx, double dy, double
   L.wl = wl;
   L.u = v3normalise(V3{dx, dy, dz});
   const double inv2dcut = (1.0 - 2 * 2.220446049250313080847263336181640625e-16) / wl;
-  L.jlim = v.off[lower_bound_d(v.inv2d, 0, v.nfam, inv2dcut)];
+  // lower_bound over all families: the guide's bracket, with one bucket of
+  // margin for the rounding of the scaled value, contains it
+  const double gs = inv2dcut * v.f_scale;
+  const int g = gs < (double)(kScbGuide - 1) ? (int)gs : kScbGuide - 1;
+  const int lo = v.f_guide[g > 0 ? g - 1 : 0], hi = v.f_guide[g + 2 < kScbGuide ? g + 2 : kScbGuide];
+  L.jlim = v.off[lower_bound_d(v.inv2d, lo, hi, inv2dcut)];
   return true;
 }
 

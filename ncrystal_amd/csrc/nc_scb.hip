@@ -12,7 +12,7 @@
 // Each kernel pair is a main kernel without the Romberg circle integral and
 // a queue kernel that redoes, with it, the neutrons whose scan met a
 // contribution outside the spline's validity (backscattering within the
-// mosaic spread).  Cross sections involve no random numbers and sampling
+// mosaic spread), one wave per neutron.  Cross sections involve no random numbers and sampling
 // draws from the neutron's own Philox stream from its first draw, so the
 // split does not change any result either.
 //
@@ -25,7 +25,6 @@ namespace ncamd {
 
 namespace {
 
-template <bool AllowSlow>
 NCD void scb_xs_one(const SCBView& v, bool valid, int64_t i, const double* __restrict__ ekin,
                     const double* __restrict__ dirs, double* __restrict__ out, int64_t* __restrict__ queue,
                     unsigned long long* __restrict__ qcount, uint16_t* __restrict__ list) {
@@ -35,11 +34,9 @@ NCD void scb_xs_one(const SCBView& v, bool valid, int64_t i, const double* __res
   L.jlim = 0;
   bool can = false;
   if (valid) can = scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
-  int nlist;
-  bool complete;
-  scb_walk<false, AllowSlow>(v, L, 0, 0.0, list, nlist, complete);
+  scb_walk<false>(v, L, 0, 0.0, list);
   if (!valid) return;
-  if (!AllowSlow && L.slow) {
+  if (L.slow) {
     const unsigned long long slot = atomicAdd(qcount, 1ull);
     queue[slot] = i;
     return;
@@ -47,60 +44,87 @@ NCD void scb_xs_one(const SCBView& v, bool valid, int64_t i, const double* __res
   out[i] = (can && L.count) ? L.total : 0.0;
 }
 
-template <bool AllowSlow>
-NCD void scb_sample_one(const SCBView& v, bool valid, int64_t i, const double* __restrict__ ekin,
-                        const double* __restrict__ dirs, uint64_t seed, uint32_t stream, double* __restrict__ oE,
-                        double* __restrict__ oD, int64_t* __restrict__ queue,
-                        unsigned long long* __restrict__ qcount, uint16_t* __restrict__ list,
-                        const int64_t* __restrict__ idmap, int skip) {
-  double E = 0.0;
-  V3 din{0.0, 0.0, 1.0};
-  ScbLane L;
-  L.wl = 1.0;
-  L.u = din;
-  L.jlim = 0;
-  bool can = false;
-  if (valid) {
-    E = ekin[i];
-    din = V3{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
-    can = scb_lane_setup(v, E, din.x, din.y, din.z, L);
+// Contributions of one neutron evaluated by a whole wave, with the Romberg
+// circle integral: lane t tests demi-normal jb + t; the candidates collect in
+// order in the wave's list and are evaluated 64 at a time, one per lane; every
+// lane then adds up the contributions in order (the sums and the selection of
+// scb_eval_list).  The queue holds few neutrons (0.2 % of a beam on a 30
+// arcmin crystal), each with a long scan and some integrals: one lane per
+// neutron left 60 waves to run 0.8 ms (cross sections of 2e6 neutrons) and 1.8
+// ms (two passes, sampling).
+constexpr int kScbWaveList = 128;
+template <bool Select>
+NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target, int* __restrict__ list) {
+  const int lane = (int)__lane_id();
+  const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
+  L.count = 0;
+  L.total = 0.0;
+  L.slow = false;
+  L.found = false;
+  const double w = gm_round(L.wl);
+  const double wl3 = w * w * w;
+  const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
+  ScbAcc a{-1, 0.0, 0.0, 0.0};
+  int n = 0;
+  for (int jb = 0; jb < L.jlim; jb += 64) {
+    const int j = jb + lane;
+    bool cand = false;
+    if (j < L.jlim) {
+      const float4 r = v.nrec32[j];
+      cand = scb_prefilter(v, r.x, r.y, r.z, r.w, fx, fy, fz, fw);
+    }
+    const uint64_t M = __ballot(cand);
+    if (cand) list[n + __popcll(M & below)] = j;
+    n += __popcll(M);
+    // evaluate full sets of 64, and what is left at the end
+    while (n >= 64 || (n > 0 && jb + 64 >= L.jlim)) {
+      const int m = n < 64 ? n : 64;
+      __builtin_amdgcn_wave_barrier();
+      const int jj = lane < m ? list[lane] : 0;
+      const int rest = 64 + lane < n ? list[64 + lane] : 0;
+      __builtin_amdgcn_wave_barrier();
+      if (64 + lane < n) list[lane] = rest;
+      n -= m;
+      double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
+      double xs0 = 0.0, xs1 = 0.0;
+      int f = 0;
+      if (lane < m) {
+        r = v.nrec[jj];
+        const double2 nf = v.nfx[jj];
+        f = (int)nf.y;
+        scb_candidate<true>(v, r, nf.x, w, wl3, L.u.x, L.u.y, L.u.z, xs0, xs1);
+      }
+      uint64_t C = __ballot(xs0 != 0.0 || xs1 != 0.0);
+      while (C) {
+        const int t = __builtin_ctzll(C);
+        C &= C - 1ull;
+        const int ft = __builtin_amdgcn_readlane(f, t);
+        if (ft != a.cur_f) {
+          a.cur_f = ft;
+          a.xsoffset = a.commul_last;
+          a.xssum = 0.0;
+        }
+        for (int side = 0; side < 2; ++side) {
+          const double xs = __shfl(side ? xs1 : xs0, t, 64);
+          if (!xs) continue;
+          const double cm = a.xsoffset + (a.xssum += xs);
+          a.commul_last = cm;
+          if constexpr (Select) {
+            const bool hit = n_select < 5 ? (cm > target) : !(cm < target);
+            if (hit || L.count == n_select - 1) {
+              const double nx = __shfl(r.x, t, 64), ny = __shfl(r.y, t, 64), nz = __shfl(r.z, t, 64);
+              L.found = true;
+              L.sel_inv2d_r = __shfl(r.w, t, 64);
+              L.sel_normal = side == 0 ? V3{-nx, -ny, -nz} : V3{nx, ny, nz};
+              return;
+            }
+          }
+          L.count++;
+        }
+      }
+    }
   }
-  // pass 1: number of contributions and their cumulative total
-  int nlist;
-  bool complete;
-  scb_walk<false, AllowSlow>(v, L, 0, 0.0, list, nlist, complete);
-  bool queued = false;
-  if (valid && !AllowSlow && L.slow) {
-    const unsigned long long slot = atomicAdd(qcount, 1ull);
-    queue[slot] = i;
-    queued = true;
-  }
-  const bool scatter = valid && can && !queued && L.count > 0 && L.total > 0.0;
-  const int64_t o = idmap && valid ? idmap[i] : i;  // output slot and Philox index
-  Rng rng;
-  rng.init(seed, stream, (uint64_t)o);
-  for (int q = 0; q < skip; ++q) (void)rng.gen();
-  double target = 0.0;
-  if (scatter && L.count > 1) target = L.total * rng.gen();
-  // pass 2: the contribution whose cumulative value passes the target, from
-  // the candidate list of pass 1 when it held them all (wave-uniform), else
-  // by a new scan
-  ScbLane S = L;
-  if (!scatter) S.jlim = 0;
-  if (complete) {
-    scb_select_list<AllowSlow>(v, S, L.count, target, list, nlist);
-  } else {
-    int nl2;
-    bool c2;
-    scb_walk<true, AllowSlow>(v, S, L.count, target, list, nl2, c2);
-  }
-  if (!valid || queued) return;
-  V3 d = din;
-  if (scatter && S.found) d = gm_genscat(v, rng, S.sel_normal, S.sel_inv2d_r, L.wl, L.u);
-  oE[o] = E;
-  oD[3 * o] = d.x;
-  oD[3 * o + 1] = d.y;
-  oD[3 * o + 2] = d.z;
+  L.total = a.commul_last;
 }
 
 }  // namespace
@@ -117,7 +141,11 @@ __global__ void __launch_bounds__(256) k_scb_keys(SCBView v, const double* __res
     ScbLane L;
     L.jlim = 0;
     scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
-    const unsigned b = (unsigned)(((int64_t)L.jlim * kScbBuckets) / ((int64_t)v.nnormals + 1));
+    // the scan length grows as the cube of the wave number: buckets of equal
+    // wave-number width, which a batch of any spectrum fills evenly enough
+    // that the counters below are not all taken at one place
+    const unsigned c = (unsigned)(cbrtf((float)L.jlim / (float)(v.nnormals + 1)) * (float)kScbBuckets);
+    const unsigned b = c < (unsigned)kScbBuckets ? c : (unsigned)kScbBuckets - 1u;
     keys[i] = b;
     atomicAdd(&lh[b], 1u);
   }
@@ -196,21 +224,23 @@ __global__ void __launch_bounds__(256) k_scb_xs_main(SCBView v, const double* __
   for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride) {
     const int64_t k = base + threadIdx.x;
     const bool valid = k < n;
-    scb_xs_one<false>(v, valid, valid ? perm[k] : 0, ekin, dirs, out, queue, qcount, list);
+    scb_xs_one(v, valid, valid ? perm[k] : 0, ekin, dirs, out, queue, qcount, list);
   }
 }
 __global__ void __launch_bounds__(256) k_scb_xs_slow(SCBView v, const double* __restrict__ ekin,
                                                      const double* __restrict__ dirs, double* __restrict__ out,
                                                      const int64_t* __restrict__ queue,
                                                      const unsigned long long* __restrict__ qcount) {
-  __shared__ uint16_t lists[4 * kScbListWave];
-  uint16_t* list = lists + (threadIdx.x >> 6) * kScbListWave;
+  __shared__ int lists[4 * kScbWaveList];
+  int* list = lists + (threadIdx.x >> 6) * kScbWaveList;
   const int64_t nq = (int64_t)*qcount;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nq; base += stride) {
-    const int64_t q = base + threadIdx.x;
-    const bool valid = q < nq;
-    scb_xs_one<true>(v, valid, valid ? queue[q] : 0, ekin, dirs, out, nullptr, nullptr, list);
+  const int64_t nwaves = (int64_t)gridDim.x * 4;
+  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < nq; q += nwaves) {
+    const int64_t i = queue[q];
+    ScbLane L;
+    const bool can = scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
+    scb_wave_walk<false>(v, L, 0, 0.0, list);
+    if ((threadIdx.x & 63) == 0) out[i] = (can && L.count) ? L.total : 0.0;
   }
 }
 // Sampling in three kernels over the sorted batch (fewer registers each
@@ -247,9 +277,7 @@ __global__ void __launch_bounds__(256) k_scb_sample_count(SCBView v, const doubl
       din = V3{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
       can = scb_lane_setup(v, E, din.x, din.y, din.z, L);
     }
-    int nlist;
-    bool complete;
-    scb_walk<false, false>(v, L, 0, 0.0, list, nlist, complete);
+    scb_walk<false>(v, L, 0, 0.0, list);
     if (!valid) continue;
     if (L.slow) {
       const unsigned long long slot = atomicAdd(qcount, 1ull);
@@ -298,9 +326,7 @@ __global__ void __launch_bounds__(256) k_scb_sample_pick(SCBView v, const double
     for (int q = 0; q < skip; ++q) (void)rng.gen();
     double target = 0.0;
     if (c > 1) target = tot[k] * rng.gen();
-    int nl;
-    bool complete;
-    scb_walk<true, false>(v, L, c, target, list, nl, complete);
+    scb_walk<true>(v, L, c, target, list);
     if (c <= 0) continue;
     sel[k] = L.found ? make_double4(L.sel_normal.x, L.sel_normal.y, L.sel_normal.z, L.sel_inv2d_r)
                      : make_double4(0.0, 0.0, 0.0, 0.0);
@@ -342,15 +368,34 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
                                                          double* __restrict__ oD, const int64_t* __restrict__ queue,
                                                          const unsigned long long* __restrict__ qcount,
                                                          const int64_t* __restrict__ idmap, int skip) {
-  __shared__ uint16_t lists[4 * kScbListWave];
-  uint16_t* list = lists + (threadIdx.x >> 6) * kScbListWave;
+  __shared__ int lists[4 * kScbWaveList];
+  int* list = lists + (threadIdx.x >> 6) * kScbWaveList;
   const int64_t nq = (int64_t)*qcount;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nq; base += stride) {
-    const int64_t q = base + threadIdx.x;
-    const bool valid = q < nq;
-    scb_sample_one<true>(v, valid, valid ? queue[q] : 0, ekin, dirs, seed, stream, oE, oD, nullptr, nullptr, list,
-                         idmap, skip);
+  const int64_t nwaves = (int64_t)gridDim.x * 4;
+  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < nq; q += nwaves) {
+    const int64_t i = queue[q];
+    const double E = ekin[i];
+    const V3 din{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
+    ScbLane L;
+    const bool can = scb_lane_setup(v, E, din.x, din.y, din.z, L);
+    scb_wave_walk<false>(v, L, 0, 0.0, list);
+    const int64_t o = idmap ? idmap[i] : i;  // output slot and Philox index
+    V3 d = din;
+    if (can && L.count > 0 && L.total > 0.0) {  // the same for every lane
+      Rng rng;
+      rng.init(seed, stream, (uint64_t)o);
+      for (int s = 0; s < skip; ++s) (void)rng.gen();
+      const int n = L.count;
+      const double target = n > 1 ? L.total * rng.gen() : 0.0;
+      scb_wave_walk<true>(v, L, n, target, list);
+      if (L.found) d = gm_genscat(v, rng, L.sel_normal, L.sel_inv2d_r, L.wl, L.u);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      oE[o] = E;
+      oD[3 * o] = d.x;
+      oD[3 * o + 1] = d.y;
+      oD[3 * o + 2] = d.z;
+    }
   }
 }
 
@@ -362,11 +407,22 @@ static inline unsigned scb_grid(int64_t n) {
   return (unsigned)g;
 }
 
+// queue kernels: a wave per queued neutron, at most as many workgroups as the
+// chip holds at once
+static inline unsigned scb_slow_grid(int64_t n) { return (unsigned)(n < 4096 ? (n + 3) / 4 : 1024); }
+
+// every workgroup of k_scb_keys adds its LDS counters to the global ones:
+// eight neutrons per lane at least, and at most four workgroups per CU
+static inline unsigned scb_keys_grid(int64_t n) {
+  const int64_t g = (n + 2047) / 2048;
+  return (unsigned)(g < 1 ? 1 : (g > 1024 ? 1024 : g));
+}
+
 // sorts the batch by scan length into w.perm and clears the queue counter
 static void scb_order(const SCBView& v, const double* ekin, const double* dirs, int64_t n, const ScbWork& w,
                       hipStream_t st) {
   hipLaunchKernelGGL(k_scb_clear, dim3(1), dim3(256), 0, st, w.hist, w.qcount);
-  hipLaunchKernelGGL(k_scb_keys, dim3(scb_grid(n)), dim3(256), 0, st, v, ekin, dirs, n, w.keys, w.hist);
+  hipLaunchKernelGGL(k_scb_keys, dim3(scb_keys_grid(n)), dim3(256), 0, st, v, ekin, dirs, n, w.keys, w.hist);
   hipLaunchKernelGGL(k_scb_offsets, dim3(1), dim3(kScbBuckets), 0, st, w.hist, w.cursor);
   hipLaunchKernelGGL(k_scb_scatter, dim3(scb_grid((n + kScbScatterItems - 1) / kScbScatterItems)), dim3(256), 0, st,
                      w.keys, n, w.cursor, w.perm);
@@ -378,7 +434,7 @@ void launch_scb_xs(const SCBView& v, const double* ekin, const double* dirs, int
   scb_order(v, ekin, dirs, n, w, st);
   hipLaunchKernelGGL(k_scb_xs_main, dim3(scb_grid(n)), dim3(256), 0, st, v, ekin, dirs, n, w.perm, out, w.queue,
                      w.qcount);
-  hipLaunchKernelGGL(k_scb_xs_slow, dim3(256), dim3(256), 0, st, v, ekin, dirs, out, w.queue, w.qcount);
+  hipLaunchKernelGGL(k_scb_xs_slow, dim3(scb_slow_grid(n)), dim3(256), 0, st, v, ekin, dirs, out, w.queue, w.qcount);
 }
 
 // gathers the neutrons listed in q (count *qc, at most nmax) into compact
@@ -416,7 +472,7 @@ void launch_scb_sample(const SCBView& v, const double* ekin, const double* dirs,
                      w.cnt, w.tot, w.sel, idmap, skip);
   hipLaunchKernelGGL(k_scb_sample_scatter, dim3(scb_grid(n)), dim3(256), 0, st, v, ekin, dirs, n, w.perm, seed,
                      stream, oE, oD, w.cnt, w.sel, idmap, skip);
-  hipLaunchKernelGGL(k_scb_sample_slow, dim3(256), dim3(256), 0, st, v, ekin, dirs, seed, stream, oE, oD, w.queue,
+  hipLaunchKernelGGL(k_scb_sample_slow, dim3(scb_slow_grid(n)), dim3(256), 0, st, v, ekin, dirs, seed, stream, oE, oD, w.queue,
                      w.qcount, idmap, skip);
 }
 
