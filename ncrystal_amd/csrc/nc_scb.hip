@@ -52,9 +52,62 @@ NCD void scb_xs_one(const SCBView& v, bool valid, int64_t i, const double* __res
 // arcmin crystal), each with a long scan and some integrals: one lane per
 // neutron left 60 waves to run 0.8 ms (cross sections of 2e6 neutrons) and 1.8
 // ms (two passes, sampling).
-constexpr int kScbWaveList = 128;
+// The scan keeps four loads in flight (a scan of 15000 demi-normals, 1 Aa, is
+// otherwise one load's latency per 64 of them), and the selection reads the
+// candidates from the list where it held them all.
+constexpr int kScbWaveList = 1024;
+constexpr int kScbWaveLoads = 4;
 template <bool Select>
-NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target, int* __restrict__ list) {
+NCD bool scb_wave_eval(const SCBView& v, ScbLane& L, ScbAcc& a, int n_select, double target, double w, double wl3,
+                       const int* __restrict__ list, int n) {
+  const int lane = (int)__lane_id();
+  for (int b = 0; b < n; b += 64) {
+    double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
+    double xs0 = 0.0, xs1 = 0.0;
+    int f = 0;
+    if (b + lane < n) {
+      const int j = list[b + lane];
+      r = v.nrec[j];
+      const double2 nf = v.nfx[j];
+      f = (int)nf.y;
+      scb_candidate<true>(v, r, nf.x, w, wl3, L.u.x, L.u.y, L.u.z, xs0, xs1);
+    }
+    uint64_t C = __ballot(xs0 != 0.0 || xs1 != 0.0);
+    while (C) {
+      const int t = __builtin_ctzll(C);
+      C &= C - 1ull;
+      const int ft = __builtin_amdgcn_readlane(f, t);
+      if (ft != a.cur_f) {
+        a.cur_f = ft;
+        a.xsoffset = a.commul_last;
+        a.xssum = 0.0;
+      }
+      for (int side = 0; side < 2; ++side) {
+        const double xs = __shfl(side ? xs1 : xs0, t, 64);
+        if (!xs) continue;
+        const double cm = a.xsoffset + (a.xssum += xs);
+        a.commul_last = cm;
+        if constexpr (Select) {
+          const bool hit = n_select < 5 ? (cm > target) : !(cm < target);
+          if (hit || L.count == n_select - 1) {
+            const double nx = __shfl(r.x, t, 64), ny = __shfl(r.y, t, 64), nz = __shfl(r.z, t, 64);
+            L.found = true;
+            L.sel_inv2d_r = __shfl(r.w, t, 64);
+            L.sel_normal = side == 0 ? V3{-nx, -ny, -nz} : V3{nx, ny, nz};
+            return true;
+          }
+        }
+        L.count++;
+      }
+    }
+  }
+  return false;
+}
+// complete: the list holds all candidates (set by the first pass and taken by
+// the second); nlist: their number
+template <bool Select>
+NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target, int* __restrict__ list, int& nlist,
+                       bool& complete) {
   const int lane = (int)__lane_id();
   const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
   L.count = 0;
@@ -63,67 +116,40 @@ NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target
   L.found = false;
   const double w = gm_round(L.wl);
   const double wl3 = w * w * w;
-  const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
   ScbAcc a{-1, 0.0, 0.0, 0.0};
+  if (Select && complete) {
+    scb_wave_eval<Select>(v, L, a, n_select, target, w, wl3, list, nlist);
+    return;
+  }
+  const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
   int n = 0;
-  for (int jb = 0; jb < L.jlim; jb += 64) {
-    const int j = jb + lane;
-    bool cand = false;
-    if (j < L.jlim) {
-      const float4 r = v.nrec32[j];
-      cand = scb_prefilter(v, r.x, r.y, r.z, r.w, fx, fy, fz, fw);
+  complete = true;
+  for (int jb = 0; jb < L.jlim; jb += 64 * kScbWaveLoads) {
+    if (n > kScbWaveList - 64 * kScbWaveLoads) {
+      __builtin_amdgcn_wave_barrier();
+      if (scb_wave_eval<Select>(v, L, a, n_select, target, w, wl3, list, n)) return;
+      __builtin_amdgcn_wave_barrier();
+      n = 0;
+      complete = false;
     }
-    const uint64_t M = __ballot(cand);
-    if (cand) list[n + __popcll(M & below)] = j;
-    n += __popcll(M);
-    // evaluate full sets of 64, and what is left at the end
-    while (n >= 64 || (n > 0 && jb + 64 >= L.jlim)) {
-      const int m = n < 64 ? n : 64;
-      __builtin_amdgcn_wave_barrier();
-      const int jj = lane < m ? list[lane] : 0;
-      const int rest = 64 + lane < n ? list[64 + lane] : 0;
-      __builtin_amdgcn_wave_barrier();
-      if (64 + lane < n) list[lane] = rest;
-      n -= m;
-      double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
-      double xs0 = 0.0, xs1 = 0.0;
-      int f = 0;
-      if (lane < m) {
-        r = v.nrec[jj];
-        const double2 nf = v.nfx[jj];
-        f = (int)nf.y;
-        scb_candidate<true>(v, r, nf.x, w, wl3, L.u.x, L.u.y, L.u.z, xs0, xs1);
-      }
-      uint64_t C = __ballot(xs0 != 0.0 || xs1 != 0.0);
-      while (C) {
-        const int t = __builtin_ctzll(C);
-        C &= C - 1ull;
-        const int ft = __builtin_amdgcn_readlane(f, t);
-        if (ft != a.cur_f) {
-          a.cur_f = ft;
-          a.xsoffset = a.commul_last;
-          a.xssum = 0.0;
-        }
-        for (int side = 0; side < 2; ++side) {
-          const double xs = __shfl(side ? xs1 : xs0, t, 64);
-          if (!xs) continue;
-          const double cm = a.xsoffset + (a.xssum += xs);
-          a.commul_last = cm;
-          if constexpr (Select) {
-            const bool hit = n_select < 5 ? (cm > target) : !(cm < target);
-            if (hit || L.count == n_select - 1) {
-              const double nx = __shfl(r.x, t, 64), ny = __shfl(r.y, t, 64), nz = __shfl(r.z, t, 64);
-              L.found = true;
-              L.sel_inv2d_r = __shfl(r.w, t, 64);
-              L.sel_normal = side == 0 ? V3{-nx, -ny, -nz} : V3{nx, ny, nz};
-              return;
-            }
-          }
-          L.count++;
-        }
-      }
+    float4 r[kScbWaveLoads];
+#pragma unroll
+    for (int q = 0; q < kScbWaveLoads; ++q) {
+      const int j = jb + 64 * q + lane;
+      r[q] = v.nrec32[j < L.jlim ? j : L.jlim - 1];
+    }
+#pragma unroll
+    for (int q = 0; q < kScbWaveLoads; ++q) {
+      const int j = jb + 64 * q + lane;
+      const bool cand = j < L.jlim && scb_prefilter(v, r[q].x, r[q].y, r[q].z, r[q].w, fx, fy, fz, fw);
+      const uint64_t M = __ballot(cand);
+      if (cand) list[n + __popcll(M & below)] = j;
+      n += __popcll(M);
     }
   }
+  __builtin_amdgcn_wave_barrier();
+  nlist = n;
+  if (scb_wave_eval<Select>(v, L, a, n_select, target, w, wl3, list, n)) return;
   L.total = a.commul_last;
 }
 
@@ -239,7 +265,9 @@ __global__ void __launch_bounds__(256) k_scb_xs_slow(SCBView v, const double* __
     const int64_t i = queue[q];
     ScbLane L;
     const bool can = scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
-    scb_wave_walk<false>(v, L, 0, 0.0, list);
+    int nlist = 0;
+    bool complete = false;
+    scb_wave_walk<false>(v, L, 0, 0.0, list, nlist, complete);
     if ((threadIdx.x & 63) == 0) out[i] = (can && L.count) ? L.total : 0.0;
   }
 }
@@ -378,7 +406,9 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
     const V3 din{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
     ScbLane L;
     const bool can = scb_lane_setup(v, E, din.x, din.y, din.z, L);
-    scb_wave_walk<false>(v, L, 0, 0.0, list);
+    int nlist = 0;
+    bool complete = false;
+    scb_wave_walk<false>(v, L, 0, 0.0, list, nlist, complete);
     const int64_t o = idmap ? idmap[i] : i;  // output slot and Philox index
     V3 d = din;
     if (can && L.count > 0 && L.total > 0.0) {  // the same for every lane
@@ -387,7 +417,7 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
       for (int s = 0; s < skip; ++s) (void)rng.gen();
       const int n = L.count;
       const double target = n > 1 ? L.total * rng.gen() : 0.0;
-      scb_wave_walk<true>(v, L, n, target, list);
+      scb_wave_walk<true>(v, L, n, target, list, nlist, complete);
       if (L.found) d = gm_genscat(v, rng, L.sel_normal, L.sel_inv2d_r, L.wl, L.u);
     }
     if ((threadIdx.x & 63) == 0) {
