@@ -9,6 +9,7 @@
 // that the tail of the launch is made of short tiles); the tile size, the
 // number of resident workgroups and the order are the autotuned parameters.
 #include "nc_kernels.hh"
+#include "nc_sabstream.hh"
 
 namespace ncamd {
 
@@ -17,9 +18,10 @@ namespace ncamd {
 // alone would hold the occupancy at one wave per SIMD):
 //   k_batch_pick  picks the component, samples PowderBragg / ElInc in place
 //                 and lists each tile's S(alpha,beta) neutrons (block-wide
-//                 compaction, so each list is in neutron order);
+//                 compaction, so each list is in neutron order), those above
+//                 the table's Emax in a queue;
 //   k_batch_sab   samples the listed neutrons tile by tile (one material per
-//                 workgroup), leaving those above the table's Emax in a queue;
+//                 workgroup);
 //   k_batch_highe samples that queue with the free-gas extender.
 // The S(alpha,beta) stages restart the neutron's Philox stream and replay the
 // pick's draw (one draw when the material has several components), so every
@@ -55,9 +57,12 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_pick(const BatchMat* __re
                                                             const double* __restrict__ ekin, double* __restrict__ o1,
                                                             double* __restrict__ o2, unsigned* __restrict__ next,
                                                             int64_t* __restrict__ sab, int* __restrict__ tcount,
+                                                            int64_t* __restrict__ highe,
+                                                            unsigned long long* __restrict__ hcount,
                                                             unsigned long long* __restrict__ nerr) {
   __shared__ int s_tile;
-  __shared__ int s_wave[kBatchBlock / 64];
+  __shared__ int s_wave[kBatchBlock / 64], s_high[kBatchBlock / 64];
+  __shared__ unsigned long long s_base;
   const int lane = (int)(threadIdx.x & 63), wid = (int)(threadIdx.x >> 6);
   const uint64_t below = (1ull << lane) - 1ull;
   while (true) {
@@ -66,31 +71,41 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_pick(const BatchMat* __re
     const BatchTile tile = tiles[t];
     const BatchMat& m = mats[tile.mat];
     const BatchRng r = rngs[tile.mat];
-    int run = 0;  // S(alpha,beta) neutrons listed so far in this tile
+    // a batch material has at most one staged component, its S(alpha,beta) one
+    const double emax = m.view.nstaged ? m.view.sab[0].egrid[m.view.sab[0].ne - 1] : 0.0;
+    int run = 0;  // S(alpha,beta) neutrons below emax listed so far in this tile
     for (int64_t start = tile.begin; start < tile.end; start += blockDim.x) {
       const int64_t k = start + threadIdx.x;
-      bool to_sab = false;
+      bool to_sab = false, to_high = false;
       if (k < tile.end) {
         Rng rng;
         rng.init(r.seed, (uint32_t)r.stream, (uint64_t)k);
         double Ef, mu;
-        int slot = 0;  // a batch material has at most one staged component, its S(alpha,beta) one
-        const int rc = comp_pick_sample<false>(m.view, rng, ekin[m.offset + k], Ef, mu, slot);
+        int slot = 0;
+        const double E = ekin[m.offset + k];
+        const int rc = comp_pick_sample<false>(m.view, rng, E, Ef, mu, slot);
         if (rc == kCompToStage) {
-          to_sab = true;
+          to_sab = E < emax;
+          to_high = !to_sab;
         } else {
           if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
           o1[m.offset + k] = Ef;
           o2[m.offset + k] = mu;
         }
       }
-      const uint64_t bal = __ballot(to_sab);
-      if (lane == 0) s_wave[wid] = __popcll(bal);
+      const uint64_t bal = __ballot(to_sab), balh = __ballot(to_high);
+      if (lane == 0) { s_wave[wid] = __popcll(bal); s_high[wid] = __popcll(balh); }
       __syncthreads();
-      int off = run, sum = 0;
+      int off = run, sum = 0, offh = 0, sumh = 0;
       for (int w = 0; w < kBatchBlock / 64; ++w) {
-        if (w < wid) off += s_wave[w];
+        if (w < wid) { off += s_wave[w]; offh += s_high[w]; }
         sum += s_wave[w];
+        sumh += s_high[w];
+      }
+      if (sumh) {  // (uniform) one append per step of the workgroup
+        if (threadIdx.x == 0) s_base = atomicAdd(hcount, (unsigned long long)sumh);
+        __syncthreads();
+        if (to_high) highe[s_base + offh + __popcll(balh & below)] = ((int64_t)t << 40) | k;
       }
       if (to_sab) sab[m.offset + tile.begin + off + __popcll(bal & below)] = k;
       __syncthreads();  // s_wave is rewritten by the next chunk
@@ -100,6 +115,7 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_pick(const BatchMat* __re
   }
 }
 
+template <bool Lds>
 __global__ void __launch_bounds__(kBatchBlock) k_batch_sab(const BatchMat* __restrict__ mats,
                                                            const BatchRng* __restrict__ rngs,
                                                            const BatchTile* __restrict__ tiles, int ntiles,
@@ -107,10 +123,9 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_sab(const BatchMat* __res
                                                            double* __restrict__ o2, unsigned* __restrict__ next,
                                                            const int64_t* __restrict__ sab,
                                                            const int* __restrict__ tcount,
-                                                           int64_t* __restrict__ highe,
-                                                           unsigned long long* __restrict__ hcount,
                                                            unsigned long long* __restrict__ nerr) {
   __shared__ int s_tile;
+  __shared__ double lds[Lds ? kSabLds : 1];
   while (true) {
     const int t = batch_next_tile(next, &s_tile);
     if (t >= ntiles) break;
@@ -120,23 +135,24 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_sab(const BatchMat* __res
     if (cnt == 0) continue;
     const BatchRng r = rngs[tile.mat];
     const int skip = m.view.n > 1 ? 1 : 0;
-    const double emax = m.view.sab[0].egrid[m.view.sab[0].ne - 1];
-    for (int j = threadIdx.x; j < cnt; j += blockDim.x) {
-      const int64_t k = sab[m.offset + tile.begin + j];
-      const double E = ekin[m.offset + k];
-      if (!(E < emax)) {
-        highe[atomicAdd(hcount, 1ull)] = ((int64_t)t << 40) | k;
-        continue;
-      }
-      Rng rng;
-      rng.init(r.seed, (uint32_t)r.stream, (uint64_t)k);
-      if (skip) rng.gen();
-      double Ef, mu;
-      const int rc = sab_sample_iso<false>(m.view.sab[0], rng, E, Ef, mu);
-      if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
-      o1[m.offset + k] = Ef;
-      o2[m.offset + k] = mu;
-    }
+    const SABView& view = m.view.sab[0];
+    const SabSmall<Lds> small(view, lds);
+    int64_t begin, end;
+    sab_share(cnt, threadIdx.x >> 6, kBatchBlock / 64, begin, end);
+    sab_stream<false>(
+        view, small, r.seed, (uint32_t)r.stream, skip, begin, end,
+        [&](int64_t p, int64_t& k, double& E) {
+          k = sab[m.offset + tile.begin + p];
+          E = ekin[m.offset + k];
+          return true;
+        },
+        [](bool) {},
+        [&](int64_t k, int rc, double Ef, double mu) {
+          if (rc) atomicAdd(nerr, 1ull);
+          o1[m.offset + k] = rc ? -1.0 : Ef;
+          o2[m.offset + k] = rc ? -999.0 : mu;
+        },
+        [](int64_t, double, double, double, double) {}, [](int64_t, double&, double&, double&) {});
   }
 }
 
@@ -175,7 +191,7 @@ __global__ void k_batch_reset(unsigned* next, unsigned long long* hcount) {
 
 void launch_batch(const BatchMat* mats, const BatchRng* rngs, const BatchTile* tiles, int ntiles, int nblocks,
                   int mode, const double* ekin, double* o1, double* o2, const BatchWork& w,
-                  unsigned long long* nerr, hipStream_t st) {
+                  unsigned long long* nerr, bool small_fit, hipStream_t st) {
   if (ntiles <= 0) return;
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(1), 0, st, w.next, w.hcount);
   if (mode == 0) {
@@ -183,9 +199,9 @@ void launch_batch(const BatchMat* mats, const BatchRng* rngs, const BatchTile* t
     return;
   }
   hipLaunchKernelGGL(k_batch_pick, dim3(nblocks), dim3(kBatchBlock), 0, st, mats, rngs, tiles, ntiles, ekin, o1, o2,
-                     w.next, w.sab, w.tcount, nerr);
-  hipLaunchKernelGGL(k_batch_sab, dim3(nblocks), dim3(kBatchBlock), 0, st, mats, rngs, tiles, ntiles, ekin, o1, o2,
-                     w.next + 1, w.sab, w.tcount, w.highe, w.hcount, nerr);
+                     w.next, w.sab, w.tcount, w.highe, w.hcount, nerr);
+  hipLaunchKernelGGL(small_fit ? k_batch_sab<true> : k_batch_sab<false>, dim3(nblocks), dim3(kBatchBlock), 0, st,
+                     mats, rngs, tiles, ntiles, ekin, o1, o2, w.next + 1, w.sab, w.tcount, nerr);
   hipLaunchKernelGGL(k_batch_highe, dim3(nblocks), dim3(kBatchBlock), 0, st, mats, rngs, tiles, ekin, o1, o2,
                      w.highe, w.hcount, nerr);
 }

@@ -29,6 +29,7 @@
 #include "../../include/ncrystal_amd.h"
 #include "../../include/ncrystal_dropin.h"
 #include "nc_kernels.hh"
+#include "nc_sabstream.hh"
 #include "nc_math.hh"
 #include "nc_vdos.hh"
 
@@ -1007,10 +1008,20 @@ Proc* create_sab(int na, int nb, const double* alpha, const double* beta, const 
     if (nb + 1 > 65535) raise("BadInput", "beta grid too large (at most 65534 points)");
     launch_sab_guides(s, bcg->as<unsigned short>(), brg->as<unsigned short>(), brs->as<double>(), 0);
     NCAMD_HIP(hipGetLastError());
-    NCAMD_HIP(hipDeviceSynchronize());
     s.cdf_guide = bcg->as<unsigned short>();
     s.row_guide = brg->as<unsigned short>();
     s.row_scale = brs->as<double>();
+    DevBuf* bpt = p->newbuf(); bpt->alloc(sizeof(SabPt) * (size_t)nb * na);
+    DevBuf* bhd = p->newbuf(); bhd->alloc(sizeof(SabHead) * (size_t)ne * nb);
+    DevBuf* bbn = p->newbuf(); bbn->alloc(sizeof(SabBin) * (size_t)ne * (nb + 1));
+    DevBuf* bst = p->newbuf(); bst->alloc(sizeof(double) * (size_t)(na + 2 * nb + 3 * ne));
+    launch_sab_pack(s, bpt->as<SabPt>(), bhd->as<SabHead>(), bbn->as<SabBin>(), bst->as<double>(), 0);
+    NCAMD_HIP(hipGetLastError());
+    NCAMD_HIP(hipDeviceSynchronize());
+    s.pt = bpt->as<SabPt>();
+    s.head = bhd->as<SabHead>();
+    s.bin = bbn->as<SabBin>();
+    s.small = bst->as<double>();
   }
   p->sab_egrid_h = egrid;
   p->sab_xs_h = xs;
@@ -1769,6 +1780,7 @@ struct Batch {
   DevBuf d_mats, d_rngs, d_tiles, d_next, d_err;
   DevBuf d_sab, d_tcount, d_highe, d_hcount;  // staged sampling (BatchWork)
   std::vector<BatchRng> h_rngs;
+  bool small_fit = true;  // sab_small_fits for every material
   int tile = 4096, nblocks = 1024, ordering = 1;
   int ntiles = 0;
   bool tiles_valid = false;
@@ -1863,7 +1875,7 @@ void batch_run(Batch* b, int mode, const double* in, double* o1, double* o2, hip
     w.highe = b->d_highe.as<int64_t>();
     w.hcount = b->d_hcount.as<unsigned long long>();
     launch_batch(b->d_mats.as<BatchMat>(), b->d_rngs.as<BatchRng>(), b->d_tiles.as<BatchTile>(), b->ntiles,
-                 b->nblocks, mode, in, o1, o2, w, b->d_err.as<unsigned long long>(), b->cap_stream);
+                 b->nblocks, mode, in, o1, o2, w, b->d_err.as<unsigned long long>(), b->small_fit, b->cap_stream);
     const hipError_t e1 = hipGetLastError();
     const hipError_t e2 = hipStreamEndCapture(b->cap_stream, &g);
     NCAMD_HIP(e1);
@@ -2274,21 +2286,17 @@ unsigned long long read_reset_err(Proc* p, hipStream_t st) {
   return n;
 }
 
-// isotropic sampling dispatch: S(alpha,beta)-only handles take the split
-// main/high-energy kernels, everything else the composition kernel
-// two queues of up to `total` neutrons (and their counters) for the staged
-// composition kernels
-// queues of a staged composition: one per staged component and the
-// high-energy queue, total neutrons each; kMaxStaged + 1 counters
+// queues of a staged composition: one per staged component, total neutrons
+// each; 2 kMaxStaged counters
 void comp_queues(Proc* p, int64_t total, hipStream_t st) {
   const int nst = make_view(p).nstaged;
-  const size_t need = (size_t)(nst + 1) * sizeof(int64_t) * (size_t)std::max<int64_t>(total, 1);
+  const size_t need = (size_t)nst * sizeof(int64_t) * (size_t)std::max<int64_t>(total, 1);
   if (p->q_idx.bytes < need) {
     NCAMD_HIP(hipStreamSynchronize(st));  // the old queue may still be in use on this stream
     p->q_idx.alloc(need);
   }
-  if (p->q_count.bytes < (kMaxStaged + 1) * sizeof(unsigned long long))
-    p->q_count.alloc((kMaxStaged + 1) * sizeof(unsigned long long));
+  if (p->q_count.bytes < 2 * kMaxStaged * sizeof(unsigned long long))
+    p->q_count.alloc(2 * kMaxStaged * sizeof(unsigned long long));
 }
 
 void check_fp32(Proc* p) {
@@ -2490,8 +2498,10 @@ void sample_dirs_dispatch(Proc* p, const double* ekin, const double* dirs, int64
                      p->q_idx.as<int64_t>(), p->q_count.as<unsigned long long>(), st);
 }
 
-// ext_q / ext_qc: caller-provided queue (2 x n x repeat entries) and two
-// counters; then no device memory is allocated here
+// isotropic sampling dispatch: S(alpha,beta)-only handles take the split
+// main/high-energy kernels, everything else the composition kernel
+// ext_q / ext_qc: caller-provided queue (2 x n x repeat entries) and 2
+// kMaxStaged counters; then no device memory is allocated here
 void sample_iso_dispatch(Proc* p, const double* ekin, int64_t n, int64_t repeat, double* oE, double* oMu,
                          hipStream_t st, int64_t* ext_q = nullptr, unsigned long long* ext_qc = nullptr) {
   if (p->oriented_comp) raise("BadInput", "oriented process: use the calls with neutron directions");
@@ -3426,6 +3436,7 @@ ncamd_batch_t ncamd_batch_create(int nmat, const ncamd_process_t* procs, const i
     b->counts.push_back(counts[i]);
     b->offsets.push_back(off);
     b->cost.push_back(batch_cost(v));
+    if (v.nstaged) b->small_fit = b->small_fit && sab_small_fits(v.sab[0]);
     hm[(size_t)i].view = v;
     hm[(size_t)i].offset = off;
     off += counts[i];

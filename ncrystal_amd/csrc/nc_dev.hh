@@ -142,6 +142,41 @@ NCD unsigned long long block_append(unsigned long long* counter, bool want, unsi
   return pos;
 }
 
+// Two such queues at once (a thread wants at most one of them): position in
+// its own.  With `packed` one counter holds both numbers, 32 bits each, so that
+// one atomic serves both; otherwise counter[stride] is the second one's.
+template <int NW>
+NCD unsigned long long block_append2(unsigned long long* counter, int stride, bool packed, bool want0, bool want1,
+                                     unsigned long long* lds) {
+  const unsigned long long m0 = __ballot(want0), m1 = __ballot(want1);
+  const int lane = (int)__lane_id(), w = (int)(threadIdx.x >> 6);
+  if (lane == 0) lds[w] = (unsigned long long)__popcll(m0) | (unsigned long long)__popcll(m1) << 32;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long tot = 0;
+    for (int j = 0; j < NW; ++j) {
+      const unsigned long long c = lds[j];
+      lds[j] = tot;
+      tot += c;
+    }
+    const unsigned long long n0 = tot & 0xFFFFFFFFull, n1 = tot >> 32;
+    if (packed) {
+      const unsigned long long b = tot ? atomicAdd(counter, tot) : 0ull;
+      lds[NW] = b & 0xFFFFFFFFull;
+      lds[NW + 1] = b >> 32;
+    } else {
+      lds[NW] = n0 ? atomicAdd(counter, n0) : 0ull;
+      lds[NW + 1] = n1 ? atomicAdd(counter + stride, n1) : 0ull;
+    }
+  }
+  __syncthreads();
+  const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
+  const unsigned long long pos = want1 ? lds[NW + 1] + (lds[w] >> 32) + (unsigned long long)__popcll(m1 & below)
+                                       : lds[NW] + (lds[w] & 0xFFFFFFFFull) + (unsigned long long)__popcll(m0 & below);
+  __syncthreads();  // lds is free for the next call
+  return pos;
+}
+
 // ---------------------------------------------------------------------------
 // Position of this lane's entry in a queue that the active lanes with `want`
 // append to: one atomic per wave (the first such lane adds their count) and
@@ -388,6 +423,22 @@ struct AInfo {
 };
 static_assert(sizeof(AInfo) == 72, "AInfo layout");
 
+// The same tables as the sampler reads them (nc_sabstream.hh).
+struct SabPt {                // table point
+  double s, logs, cumul;      // S, log S, cumulative alpha integral of its row
+};
+struct alignas(16) SabHead {  // alpha sampler of a row: AInfo's probabilities, the row's cumul at its
+  double prob_front, prob_notback, cl, cu;  // indices
+};
+struct SabBin {               // point of a beta distribution
+  double cdf, x, y;
+};
+// small tables, one after the other: alpha grid [na], beta grid [nb], guide
+// scales of the rows [nb], energy grid [ne], and per energy-grid point the
+// first-bin endpoint and two ints (first beta row; points, or -1 for alpha =
+// beta = 0, -2 for no sampler) [2 ne]
+constexpr int kSabLds = 4096;  // values of them that a workgroup can keep in LDS
+
 struct SABView {
   int na, nb, ne;
   const double* alpha;    // [na]
@@ -411,11 +462,28 @@ struct SABView {
   int eg_nbkt, eg_shift;
   long long eg_base;               // bucket b = (bits(E) >> eg_shift) - eg_base
   const unsigned short* cdf_guide; // [ne][kCdfGuide+1]: lower_bound(cdf, g/kCdfGuide)
-  const unsigned short* row_guide; // [nb][kRowGuide+1]: upper_bound(cumul row, g/row_scale)
+  const unsigned short* row_guide; // [nb][kRowGuide+1]: points of the row with row_bucket below g
   const double* row_scale;         // [nb]: kRowGuide / cumul[row][na-1] (0: row without area)
+  const SabPt* pt;                 // [nb*na]
+  const SabHead* head;             // [ne*nb]
+  const SabBin* bin;               // [ne*(nb+1)]
+  const double* small;             // [na + 2 nb + 3 ne]
 };
-constexpr int kCdfGuide = 256;  // power of two: p*kCdfGuide is exact
-constexpr int kRowGuide = 64;
+constexpr int kCdfGuide = 4096;  // power of two: p*kCdfGuide is exact
+constexpr int kRowGuide = 1024;
+// bucket of a cumulative value of a row; monotone, so the upper_bound of x is
+// between the numbers of points in buckets below x's and up to x's
+NCD int row_bucket(double x, double scale) {
+  const int g = (int)(x * scale);
+  return g < 0 ? 0 : (g < kRowGuide ? g : kRowGuide - 1);
+}
+// two consecutive guide entries (any 2-byte address) by one load
+NCD void guide_pair(const unsigned short* __restrict__ g, int& lo, int& hi) {
+  unsigned v;
+  __builtin_memcpy(&v, g, 4);
+  lo = (int)(v & 0xFFFFu);
+  hi = (int)(v >> 16);
+}
 
 NCD double sab_fg_xs(const SABView& s, double E) { return s.sigma_free * freegas_xs_shape(s.fg_ca * E); }
 
@@ -490,14 +558,10 @@ NCD double alg1_sample_alpha(const SABView& s, int ie, int ibl, int ibeta, doubl
     int e;
     const double rs = s.row_scale[ibeta];
     if (rs > 0.0) {
-      // the global upper_bound of sel lies in the guide bracket (one bucket of
-      // margin either side absorbs rounding of sel*rs); clamping it to iu+1
-      // equals the bounded search of the reference (cumul[il] <= sel)
-      int g = (int)(sel * rs);
-      g = g < 0 ? 0 : (g > kRowGuide ? kRowGuide : g);
-      const unsigned short* rg = s.row_guide + (size_t)ibeta * (kRowGuide + 1);
-      const int lo = rg[g > 0 ? g - 1 : 0];
-      const int hi = rg[g + 2 <= kRowGuide ? g + 2 : kRowGuide];
+      // the global upper_bound of sel lies in the guide bracket; clamping it
+      // to iu+1 equals the bounded search of the reference (cumul[il] <= sel)
+      int lo, hi;
+      guide_pair(s.row_guide + (size_t)ibeta * (kRowGuide + 1) + row_bucket(sel, rs), lo, hi);
       e = upper_bound_d(cumul, lo, hi, sel);
       if (e > iu + 1) e = iu + 1;
     } else {

@@ -176,9 +176,9 @@ NCHD bool comp_has_gas(const CompView& c) {
 // per-neutron kernels (nc_kernels.hip)
 void launch_xs_iso(const CompView&, const double* ekin, int64_t n, int64_t repeat, double* out, bool fp32,
                    hipStream_t);
-// queues: [(nstaged + 1) x n*repeat] neutron indices (one queue per staged
-// component and the high-energy queue), qcount: [kMaxStaged + 1] counters
-// (used by compositions with an S(alpha,beta) part)
+// queues: [nstaged x n*repeat] neutron indices (one queue per staged
+// component, filled from both ends), qcount: [2 kMaxStaged] counters (used by
+// compositions with an S(alpha,beta) part)
 void launch_sample_iso(const CompView&, const double* ekin, int64_t n, int64_t repeat, uint64_t seed,
                        uint32_t stream, double* oE, double* oMu, unsigned long long* nerr, int64_t* queues,
                        unsigned long long* qcount, hipStream_t);
@@ -200,6 +200,7 @@ void launch_sab_sample_iso(const SABView&, const double* ekin, int64_t n, int64_
                            unsigned long long* qcount, int domain_check, hipStream_t);
 void launch_sab_guides(const SABView&, unsigned short* cdf_guide, unsigned short* row_guide, double* row_scale,
                        hipStream_t);
+void launch_sab_pack(const SABView&, SabPt* pt, SabHead* head, SabBin* bin, double* small, hipStream_t);
 
 // box-envelope sampler of S(alpha,beta) (nc_kb.hip)
 void launch_kb_bounds(const SABView&, const double4* node_par, int nn, int nbox, int64_t total, KBBox* box,
@@ -300,10 +301,11 @@ struct BatchWork {
   int64_t* highe;              // [total] (tile << 40 | neutron) above the table's Emax
   unsigned long long* hcount;  // [1]
 };
+// small_fit: sab_small_fits for every material's S(alpha,beta)
 // mode 0: cross sections into o1; mode 1: isotropic sampling into (o1=E', o2=mu)
 void launch_batch(const BatchMat* mats, const BatchRng* rngs, const BatchTile* tiles, int ntiles, int nblocks,
                   int mode, const double* ekin, double* o1, double* o2, const BatchWork& w,
-                  unsigned long long* nerr, hipStream_t);
+                  unsigned long long* nerr, bool small_fit, hipStream_t);
 
 // single-crystal Bragg, oriented (nc_scb.hip): counting sort of the batch by
 // scan length, main kernel, Romberg queue kernel

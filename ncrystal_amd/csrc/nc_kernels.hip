@@ -6,6 +6,8 @@
 // (cumulative component xs), :353-362 (xs), :379-389 (component pick +
 // sampling); batched layout: ncrystal_core/src/cinterface/ncrystal.cc:1107-1246.
 #include "nc_kernels.hh"
+#include "nc_sabstream.hh"
+#include <algorithm>
 
 namespace ncamd {
 
@@ -110,9 +112,8 @@ __global__ void __launch_bounds__(256) k_fg_sample(FGView g, const double* __res
 
 // Compositions with an S(alpha,beta) part, in stages so that no kernel
 // carries every sampler: k_comp_pick samples PowderBragg / ElInc picks in
-// place and queues the neutrons that pick S(alpha,beta); k_comp_sab<false>
-// samples those below the table's Emax and queues the rest for
-// k_comp_sab<true> (free-gas extender).  The S(alpha,beta) stages restart
+// place and queues the neutrons that pick S(alpha,beta), those below the
+// table's Emax and those above it apart; k_comp_sab samples both.  The S(alpha,beta) stages restart
 // the neutron's Philox stream and replay the pick's draw (`skip`), so every
 // neutron gets what one kernel doing all of it would give.
 // outputs of one neutron: (E', mu), or (E', direction) for the oriented call
@@ -133,72 +134,116 @@ NCD void comp_store(int64_t k, int rc, double Ef, double mu, Rng& rng, const dou
   }
 }
 
+// Appends to one counter run one after the other, about 13 ns each whatever
+// workgroup they come from, and paced this kernel (1e6 neutrons, two queues:
+// 107 us with an append per queue and 256 neutrons): large workgroups, both ends
+// of a queue by one atomic.
+constexpr int kPickThreads = 1024;
 template <bool Dirs, bool Gas>
-__global__ void __launch_bounds__(256) k_comp_pick(CompView c, const double* __restrict__ ekin,
+__global__ void __launch_bounds__(kPickThreads) k_comp_pick(CompView c, const double* __restrict__ ekin,
                                                    const double* __restrict__ dirs, int64_t n, int64_t total,
                                                    uint64_t seed, uint32_t stream, double* __restrict__ oE,
                                                    double* __restrict__ o2, unsigned long long* __restrict__ nerr,
                                                    int64_t* __restrict__ sq, unsigned long long* __restrict__ sqc,
                                                    const double* __restrict__ ext, int64_t* __restrict__ cq,
                                                    unsigned long long* __restrict__ cqc) {
-  __shared__ unsigned long long s_app[5];
+  constexpr int NW = kPickThreads / 64;
+  __shared__ unsigned long long s_app[NW + 2];
+  const bool packed = total < ((int64_t)1 << 32);
   const int64_t gstride = (int64_t)gridDim.x * blockDim.x;
   // workgroup-uniform loop: the queue appends synchronise the workgroup
   for (int64_t k0 = (int64_t)blockIdx.x * blockDim.x; k0 < total; k0 += gstride) {
     const int64_t k = k0 + threadIdx.x;
     const bool valid = k < total;
     Rng rng;
-    double Ef = 0.0, mu = 0.0;
+    double E = 0.0, Ef = 0.0, mu = 0.0;
     int slot = 0, rc = kCompToStage + kCompToSCB + 1;  // neither queue
     if (valid) {
       const int64_t i = (total == n) ? k : (k % n);
+      E = ekin[i];
       rng.init(seed, stream, (uint64_t)k);
-      rc = comp_pick_sample<Gas>(c, rng, ekin[i], Ef, mu, slot, ext ? ext[k] : 0.0);
+      rc = comp_pick_sample<Gas>(c, rng, E, Ef, mu, slot, ext ? ext[k] : 0.0);
     }
     // queue appends, one atomic per workgroup and queue: one queue per
     // staged component, and the SCBragg queue
     const bool staged = valid && rc == kCompToStage;
+    // (a component's neutrons above its table's Emax from the back of its queue)
     for (int s = 0; s < c.nstaged; ++s) {
       const bool want = staged && slot == s;
-      const unsigned long long pos = block_append<4>(&sqc[s], want, s_app);
-      if (want) sq[(int64_t)s * total + (int64_t)pos] = k;
+      const bool high = want && c.kind[c.stage_comp[s]] == kKindSAB && !(E < c.sab[s].egrid[c.sab[s].ne - 1]);
+      const int64_t pos = (int64_t)block_append2<NW>(&sqc[s], kMaxStaged, packed, want && !high, high, s_app);
+      if (want) sq[(int64_t)s * total + (high ? total - 1 - pos : pos)] = k;
     }
     const bool to_scb = valid && rc == kCompToSCB;
     if (cqc) {
-      const unsigned long long pos = block_append<4>(cqc, to_scb, s_app);
+      const unsigned long long pos = block_append<NW>(cqc, to_scb, s_app);
       if (to_scb) cq[pos] = k;
     }
     if (valid && !staged && !to_scb) comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
   }
 }
 
-template <bool HighE, bool Dirs>
-__global__ void __launch_bounds__(256) k_comp_sab(SABView s, const double* __restrict__ ekin,
-                                                  const double* __restrict__ dirs, int64_t n, int64_t total,
-                                                  uint64_t seed, uint32_t stream, int skip, double* __restrict__ oE,
-                                                  double* __restrict__ o2, unsigned long long* __restrict__ nerr,
-                                                  const int64_t* __restrict__ inq,
-                                                  const unsigned long long* __restrict__ inqc,
-                                                  int64_t* __restrict__ hq, unsigned long long* __restrict__ hqc) {
-  const int64_t gstride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t nq = (int64_t)*inqc;
-  const double emax = s.egrid[s.ne - 1];
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nq; q += gstride) {
-    const int64_t k = inq[q];
-    const double E = ekin[(total == n) ? k : (k % n)];
-    if constexpr (!HighE) {
-      if (!(E < emax)) {
-        hq[atomicAdd(hqc, 1ull)] = k;
-        continue;
-      }
+// entries at the front (0) or back (1) of a staged component's queue
+NCD int64_t queue_count(const unsigned long long* __restrict__ count, int back, int64_t total) {
+  if (total < ((int64_t)1 << 32)) return (int64_t)(back ? *count >> 32 : *count & 0xFFFFFFFFull);
+  return (int64_t)count[back * kMaxStaged];
+}
+// One launch per component: workgroups from nhigh on stream their waves' shares
+// of the queue's front (sab_stream), the first nhigh sample the neutrons above
+// the table's Emax at its back (free-gas extender).  Together the two hide each
+// other's latencies, and the pick has parted them: told apart here, each refill
+// of a wave appended to the extender's queue by an atomic of its own.
+template <bool Dirs, bool Lds>
+__global__ void __launch_bounds__(256, 4) k_comp_sab(SABView s, const double* __restrict__ ekin,
+                                                     const double* __restrict__ dirs, int64_t n, int64_t total,
+                                                     uint64_t seed, uint32_t stream, int skip,
+                                                     double* __restrict__ oE, double* __restrict__ o2,
+                                                     unsigned long long* __restrict__ nerr,
+                                                     const int64_t* __restrict__ q,
+                                                     const unsigned long long* __restrict__ count, unsigned nhigh) {
+  __shared__ double lds[Lds ? kSabLds : 1];
+  if (blockIdx.x < nhigh) {
+    const int64_t m = queue_count(count, 1, total);
+    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < m; j += (int64_t)nhigh * blockDim.x) {
+      const int64_t k = q[total - 1 - j];
+      Rng rng;
+      rng.init(seed, stream, (uint64_t)k);
+      if (skip) rng.gen();
+      double Ef, mu;
+      const int rc = sab_sample_iso<true>(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
+      comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
     }
-    Rng rng;
-    rng.init(seed, stream, (uint64_t)k);
-    if (skip) rng.gen();
-    double Ef, mu;
-    const int rc = sab_sample_iso<HighE>(s, rng, E, Ef, mu);
-    comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
+    return;
   }
+  const int64_t m = queue_count(count, 0, total);
+  if (m == 0) return;
+  const SabSmall<Lds> small(s, lds);
+  int64_t begin, end;
+  sab_share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4, begin, end);
+  sab_stream<Dirs>(
+      s, small, seed, stream, skip, begin, end,
+      [&](int64_t p, int64_t& k, double& E) {
+        k = q[p];
+        E = ekin[(total == n) ? k : (k % n)];
+        return true;
+      },
+      [](bool) {},
+      [&](int64_t k, int rc, double Ef, double mu) {
+        if (rc) atomicAdd(nerr, 1ull);
+        oE[k] = rc ? -1.0 : Ef;
+        if constexpr (Dirs) {  // errors only
+          o2[3 * k] = 0.0; o2[3 * k + 1] = 0.0; o2[3 * k + 2] = 0.0;
+        } else {
+          o2[k] = rc ? -999.0 : mu;
+        }
+      },
+      [&](int64_t k, double Ef, double ox, double oy, double oz) {
+        oE[k] = Ef;
+        o2[3 * k] = ox; o2[3 * k + 1] = oy; o2[3 * k + 2] = oz;
+      },
+      [&](int64_t k, double& ix, double& iy, double& iz) {
+        ix = dirs[3 * k]; iy = dirs[3 * k + 1]; iz = dirs[3 * k + 2];
+      });
 }
 
 // stage kernel of a FreeGas component beside S(alpha,beta) components: the
@@ -212,7 +257,7 @@ __global__ void __launch_bounds__(256) k_comp_fg(FGView g, const double* __restr
                                                  const int64_t* __restrict__ inq,
                                                  const unsigned long long* __restrict__ inqc) {
   const int64_t gstride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t nq = (int64_t)*inqc;
+  const int64_t nq = queue_count(inqc, 0, total);
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nq; q += gstride) {
     const int64_t k = inq[q];
     Rng rng;
@@ -244,37 +289,63 @@ __global__ void __launch_bounds__(256) k_sab_ab(SABView s, const double* __restr
 // register-hungry, so the main kernel leaves those neutrons in a queue that a
 // second kernel drains.  Both draw from the neutron's own Philox stream from
 // its first draw, so the split does not change any result.
-__global__ void __launch_bounds__(256) k_sab_sample_iso_main(SABView s, const double* __restrict__ ekin,
-                                                             int64_t n, int64_t total, uint64_t seed,
-                                                             uint32_t stream, double* __restrict__ oE,
-                                                             double* __restrict__ oMu,
-                                                             unsigned long long* __restrict__ nerr,
-                                                             int64_t* __restrict__ queue,
-                                                             unsigned long long* __restrict__ qcount,
-                                                             int domain_check) {
-  const int64_t gstride = (int64_t)gridDim.x * blockDim.x;
+template <bool Lds>
+__global__ void __launch_bounds__(256, 4) k_sab_sample_iso_main(SABView s, const double* __restrict__ ekin,
+                                                                int64_t n, int64_t total, uint64_t seed,
+                                                                uint32_t stream, double* __restrict__ oE,
+                                                                double* __restrict__ oMu,
+                                                                unsigned long long* __restrict__ nerr,
+                                                                int64_t* __restrict__ queue,
+                                                                unsigned long long* __restrict__ qcount,
+                                                                int domain_check) {
+  __shared__ double lds[Lds ? kSabLds : 1];
+  // neutrons for the high-energy queue, kept until there is a wave of them:
+  // one atomic each would pace a batch that has many
+  __shared__ int64_t bufs[4][128];
+  __shared__ int counts[4];
+  const int lane = (int)(threadIdx.x & 63);
+  int64_t* buf = bufs[threadIdx.x >> 6];
+  int* have = counts + (threadIdx.x >> 6);
+  if (lane == 0) *have = 0;
+  __syncthreads();
+  const SabSmall<Lds> small(s, lds);
+  int64_t begin, end;
+  sab_share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4, begin, end);
   const double emax = s.egrid[s.ne - 1];
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < total; k += gstride) {
-    const int64_t i = (total == n) ? k : (k % n);
-    const double E = ekin[i];
-    double Ef, mu;
-    if (domain_check && !(E >= 0.0 && E <= __builtin_huge_val())) {
-      // a composition outside its energy domain does not scatter
-      Ef = E; mu = 1.0;
-    } else if (!(E < emax)) {
-      // the free-gas kernel, and the sampler's own handling of non-finite E
-      const unsigned long long slot = atomicAdd(qcount, 1ull);
-      queue[slot] = k;
-      continue;
-    } else {
-      Rng rng;
-      rng.init(seed, stream, (uint64_t)k);
-      const int rc = sab_sample_iso<false>(s, rng, E, Ef, mu);
-      if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
-    }
-    oE[k] = Ef;
-    oMu[k] = mu;
-  }
+  sab_stream<false>(
+      s, small, seed, stream, 0, begin, end,
+      [&](int64_t p, int64_t& k, double& E) {
+        k = p;
+        E = ekin[(total == n) ? k : (k % n)];
+        if (domain_check && !(E >= 0.0 && E <= __builtin_huge_val())) {
+          // a composition outside its energy domain does not scatter
+          oE[k] = E;
+          oMu[k] = 1.0;
+          return false;
+        }
+        if (E < emax) return true;
+        // the free-gas kernel, and the sampler's own handling of non-finite E
+        buf[atomicAdd(have, 1)] = k;
+        return false;
+      },
+      [&](bool last) {  // at most 63 kept and 64 new ones
+        __builtin_amdgcn_wave_barrier();
+        const int c = *(volatile int*)have;
+        if (c < (last ? 1 : 64)) return;
+        unsigned long long at = 0ull;
+        if (lane == 0) at = atomicAdd(qcount, (unsigned long long)c);
+        at = __shfl(at, 0, 64);
+        for (int j = lane; j < c; j += 64) queue[at + j] = buf[j];
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) *(volatile int*)have = 0;
+        __builtin_amdgcn_wave_barrier();
+      },
+      [&](int64_t k, int rc, double Ef, double mu) {
+        if (rc) atomicAdd(nerr, 1ull);
+        oE[k] = rc ? -1.0 : Ef;
+        oMu[k] = rc ? -999.0 : mu;
+      },
+      [](int64_t, double, double, double, double) {}, [](int64_t, double&, double&, double&) {});
 }
 
 __global__ void __launch_bounds__(256) k_sab_sample_iso_highe(SABView s, const double* __restrict__ ekin,
@@ -322,10 +393,48 @@ __global__ void k_sab_row_guides(SABView s, unsigned short* __restrict__ guide, 
   const double rmax = row[s.na - 1];
   const double rs = rmax > 0.0 ? (double)kRowGuide / rmax : 0.0;
   if (g == 0) scale[ib] = rs;
-  // the last bucket is closed by na itself so that values at or above the
-  // row maximum always have their answer inside the bracket
-  const int r = (g == kRowGuide) ? s.na : upper_bound_d(row, 0, s.na, (double)g / rs);
-  guide[t] = rs > 0.0 ? (unsigned short)r : (unsigned short)0;
+  int lo = g == kRowGuide ? s.na : 0, n = s.na - lo;  // the last entry is na
+  while (n > 0) {
+    const int h = n >> 1, m = lo + h;
+    if (row_bucket(row[m], rs) < g) { lo = m + 1; n -= h + 1; } else n = h;
+  }
+  guide[t] = rs > 0.0 ? (unsigned short)lo : (unsigned short)0;
+}
+// the sampler's layout of the tables (built once, after the guides)
+__global__ void k_sab_pack(SABView s, SabPt* __restrict__ pt, SabHead* __restrict__ head, SabBin* __restrict__ bin,
+                           double* __restrict__ small) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < (int64_t)s.nb * s.na) {
+    const double2 q = s.sl[t];
+    pt[t] = SabPt{q.x, q.y, s.cumul[t]};
+  }
+  if (t < (int64_t)s.ne * s.nb) {
+    const int ie = (int)(t / s.nb), row = s.shdr[ie].y + (int)(t % s.nb);
+    const AInfo i = s.sinfo[t];
+    SabHead h{i.prob_front, i.prob_notback, 0.0, 0.0};
+    if (row < s.nb) {  // (the records past the last row are not used)
+      h.cl = s.cumul[(size_t)row * s.na + i.f_idx];
+      h.cu = s.cumul[(size_t)row * s.na + i.b_idx];
+    }
+    head[t] = h;
+  }
+  if (t < (int64_t)s.ne * (s.nb + 1)) {
+    const double2 q = s.sxy[t];
+    bin[t] = SabBin{s.scdf[t], q.x, q.y};
+  }
+  if (t < s.na) small[t] = s.alpha[t];
+  if (t < s.nb) {
+    small[s.na + t] = s.beta[t];
+    small[s.na + s.nb + t] = s.row_scale[t];
+  }
+  if (t < s.ne) {
+    double* e = small + s.na + 2 * s.nb;
+    e[t] = s.egrid[t];
+    const int4 h = s.shdr[t];
+    const int nv = h.x == 1 ? h.z : (h.x == 0 ? -1 : -2);
+    e[s.ne + 2 * t] = s.sfirst[t];
+    e[s.ne + 2 * t + 1] = __longlong_as_double((long long)(((unsigned long long)(unsigned)nv << 32) | (unsigned)h.y));
+  }
 }
 
 static inline unsigned grid_for(int64_t n, int bs) {
@@ -337,6 +446,12 @@ static inline unsigned grid_for(int64_t n, int bs) {
   return (unsigned)g;
 }
 
+// persistent kernels: four workgroups (of four waves) per CU
+static inline unsigned stream_grid(int64_t n) {
+  const int64_t g = (n + 255) / 256;
+  return (unsigned)(g < 1 ? 1 : (g > 1024 ? 1024 : g));
+}
+
 __global__ void k_zero_u64(unsigned long long* p) { *p = 0ull; }
 
 __global__ void k_zero_u64_n(unsigned long long* p, int n) {
@@ -344,29 +459,28 @@ __global__ void k_zero_u64_n(unsigned long long* p, int n) {
 }
 
 // the stage launches of a composition with an S(alpha,beta) part, after the
-// pick kernel filled one queue per staged component (queues + s * total,
-// counter qcount[s]); the high-energy queue after them (counter
-// qcount[kMaxStaged]) is reused by each S(alpha,beta) component in turn
+// pick kernel filled one queue per staged component from both ends (queues +
+// s * total, counters at qcount + s)
 template <bool Dirs>
 void launch_stages(const CompView& c, const double* ekin, const double* dirs, int64_t n, int64_t total,
                    uint64_t seed, uint32_t stream, double* oE, double* o2, unsigned long long* nerr,
                    int64_t* queues, unsigned long long* qcount, hipStream_t st) {
   const int skip = c.n > 1 ? 1 : 0;
-  int64_t* hq = queues + (int64_t)c.nstaged * total;
-  unsigned long long* hqc = qcount + kMaxStaged;
-  const dim3 g(grid_for(total, 256)), b(256);
+  const dim3 b(256);
+  const unsigned gs = stream_grid(total), nhigh = gs < 512 ? gs : 512;
   for (int sl = 0; sl < c.nstaged; ++sl) {
     const int comp = c.stage_comp[sl];
     int64_t* q = queues + (int64_t)sl * total;
     if (c.kind[comp] == kKindSAB) {
-      hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, hqc);
-      hipLaunchKernelGGL((k_comp_sab<false, Dirs>), g, b, 0, st, c.sab[sl], ekin, dirs, n, total, seed, stream, skip,
-                         oE, o2, nerr, q, qcount + sl, hq, hqc);
-      hipLaunchKernelGGL((k_comp_sab<true, Dirs>), g, b, 0, st, c.sab[sl], ekin, dirs, n, total, seed, stream, skip,
-                         oE, o2, nerr, hq, hqc, nullptr, nullptr);
+      if (sab_small_fits(c.sab[sl]))
+        hipLaunchKernelGGL((k_comp_sab<Dirs, true>), dim3(gs + nhigh), b, 0, st, c.sab[sl], ekin, dirs, n, total, seed,
+                           stream, skip, oE, o2, nerr, q, qcount + sl, nhigh);
+      else
+        hipLaunchKernelGGL((k_comp_sab<Dirs, false>), dim3(gs + nhigh), b, 0, st, c.sab[sl], ekin, dirs, n, total,
+                           seed, stream, skip, oE, o2, nerr, q, qcount + sl, nhigh);
     } else {
-      hipLaunchKernelGGL(k_comp_fg<Dirs>, g, b, 0, st, c.fg[comp], ekin, dirs, n, total, seed, stream, skip, oE, o2,
-                         nerr, q, qcount + sl);
+      hipLaunchKernelGGL(k_comp_fg<Dirs>, dim3(grid_for(total, 256)), b, 0, st, c.fg[comp], ekin, dirs, n, total, seed,
+                         stream, skip, oE, o2, nerr, q, qcount + sl);
     }
   }
 }
@@ -440,8 +554,8 @@ void launch_sample_iso(const CompView& c, const double* ekin, int64_t n, int64_t
                          seed, stream, oE, oMu, nerr);
       break;
     default: {
-      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, kMaxStaged + 1);
-      const dim3 g(grid_for(total, 256)), b(256);
+      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, 2 * kMaxStaged);
+      const dim3 g(grid_for(total, kPickThreads)), b(kPickThreads);
       if (comp_has_gas(c))
         hipLaunchKernelGGL((k_comp_pick<false, true>), g, b, 0, st, c, ekin, (const double*)nullptr, n, total, seed,
                            stream, oE, oMu, nerr, queues, qcount, (const double*)nullptr, (int64_t*)nullptr,
@@ -486,8 +600,8 @@ void launch_sample_dirs(const CompView& c, const double* ekin, const double* dir
                          seed, stream, oE, oD, nerr);
       break;
     default: {
-      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, kMaxStaged + 1);
-      const dim3 g(grid_for(n, 256)), b(256);
+      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, 2 * kMaxStaged);
+      const dim3 g(grid_for(n, kPickThreads)), b(kPickThreads);
       if (comp_has_gas(c))
         hipLaunchKernelGGL((k_comp_pick<true, true>), g, b, 0, st, c, ekin, dirs, n, n, seed, stream, oE, oD, nerr,
                            queues, qcount, ext, cq, cqc);
@@ -511,8 +625,12 @@ void launch_sab_sample_iso(const SABView& s, const double* ekin, int64_t n, int6
   if (total <= 0) return;
   // kernel instead of a memset node, so that callers may capture this in a graph
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, qcount);
-  hipLaunchKernelGGL(k_sab_sample_iso_main, dim3(grid_for(total, 256)), dim3(256), 0, st, s, ekin, n, total, seed,
-                     stream, oE, oMu, nerr, queue, qcount, domain_check);
+  if (sab_small_fits(s))
+    hipLaunchKernelGGL(k_sab_sample_iso_main<true>, dim3(stream_grid(total)), dim3(256), 0, st, s, ekin, n, total,
+                       seed, stream, oE, oMu, nerr, queue, qcount, domain_check);
+  else
+    hipLaunchKernelGGL(k_sab_sample_iso_main<false>, dim3(stream_grid(total)), dim3(256), 0, st, s, ekin, n, total,
+                       seed, stream, oE, oMu, nerr, queue, qcount, domain_check);
   hipLaunchKernelGGL(k_sab_sample_iso_highe, dim3(grid_for(total, 256)), dim3(256), 0, st, s, ekin, n, total, seed,
                      stream, oE, oMu, nerr, queue, qcount);
 }
@@ -532,6 +650,10 @@ void launch_sab_guides(const SABView& s, unsigned short* cdf_guide, unsigned sho
   const int64_t n2 = (int64_t)s.nb * (kRowGuide + 1);
   hipLaunchKernelGGL(k_sab_row_guides, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, st, s, row_guide,
                      row_scale);
+}
+void launch_sab_pack(const SABView& s, SabPt* pt, SabHead* head, SabBin* bin, double* small, hipStream_t st) {
+  const int64_t n = std::max((int64_t)s.nb * s.na, (int64_t)s.ne * (s.nb + 1));
+  hipLaunchKernelGGL(k_sab_pack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, s, pt, head, bin, small);
 }
 void launch_fill_loguniform(double* out, int64_t n, double lemin, double lemax, uint64_t seed, hipStream_t st) {
   if (n <= 0) return;
