@@ -269,6 +269,111 @@ __global__ void __launch_bounds__(256) k_comp_fg(FGView g, const double* __restr
   }
 }
 
+// The stages of a composition within one workgroup: its `per` neutrons are
+// picked, listed in LDS by component (below the table's Emax from the front of
+// its list, above it from the back) and sampled there, without queues in memory,
+// counters to clear or launches to wait for.  Such small batches are bound by
+// the latency of their longest rejection (a step of sab_stream takes about 5 us
+// on its own), so the neutrons are spread over the chip first, down to 16 a
+// workgroup, and the lists over its waves.
+template <bool Dirs, bool Gas, bool Lds>
+__global__ void __launch_bounds__(256, 4) k_comp_local(CompView c, const double* __restrict__ ekin,
+                                                       const double* __restrict__ dirs, int64_t n, int64_t total,
+                                                       uint64_t seed, uint32_t stream, double* __restrict__ oE,
+                                                       double* __restrict__ o2,
+                                                       unsigned long long* __restrict__ nerr,
+                                                       const double* __restrict__ ext, int64_t* __restrict__ cq,
+                                                       unsigned long long* __restrict__ cqc, int per) {
+  constexpr int kList = 256;
+  __shared__ double lds[Lds ? kSabLds : 1];
+  __shared__ unsigned char list[kMaxStaged][kList];
+  __shared__ int count[2 * kMaxStaged];
+  __shared__ unsigned long long s_app[5];
+  const int tid = (int)threadIdx.x;
+  if (tid < 2 * kMaxStaged) count[tid] = 0;
+  __syncthreads();
+  const int64_t k0 = (int64_t)blockIdx.x * per;
+  {
+    const int64_t k = k0 + tid;
+    const bool valid = tid < per && k < total;
+    Rng rng;
+    double Ef = 0.0, mu = 0.0;
+    int slot = 0, rc = kCompToStage + kCompToSCB + 1;  // neither list
+    if (valid) {
+      const double E = ekin[(total == n) ? k : (k % n)];
+      rng.init(seed, stream, (uint64_t)k);
+      rc = comp_pick_sample<Gas>(c, rng, E, Ef, mu, slot, ext ? ext[k] : 0.0);
+      if (rc == kCompToStage) {
+        const bool high = c.kind[c.stage_comp[slot]] == kKindSAB && !(E < c.sab[slot].egrid[c.sab[slot].ne - 1]);
+        const int pos = atomicAdd(&count[high ? kMaxStaged + slot : slot], 1);
+        list[slot][high ? kList - 1 - pos : pos] = (unsigned char)tid;
+      }
+    }
+    const bool to_scb = valid && rc == kCompToSCB;
+    if (cqc) {
+      const unsigned long long pos = block_append<4>(cqc, to_scb, s_app);
+      if (to_scb) cq[pos] = k;
+    }
+    if (valid && rc != kCompToStage && !to_scb) comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
+  }
+  __syncthreads();
+  const int skip = c.n > 1 ? 1 : 0;
+  for (int sl = 0; sl < c.nstaged; ++sl) {
+    const int low = count[sl], high = count[kMaxStaged + sl];
+    if (Gas && c.kind[c.stage_comp[sl]] == kKindFG) {
+      for (int j = tid; j < low; j += 256) {
+        const int64_t k = k0 + list[sl][j];
+        Rng rng;
+        rng.init(seed, stream, (uint64_t)k);
+        if (skip) rng.gen();
+        double Ef, mu;
+        const int rc = fg_sample_demu(c.fg[c.stage_comp[sl]], rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
+        comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
+      }
+      continue;
+    }
+    const SABView& s = c.sab[sl];
+    if (low > 0) {
+      const SabSmall<Lds> small(s, lds);
+      int64_t begin, end;
+      sab_share(low, tid >> 6, 4, begin, end, 32);
+      sab_stream<Dirs>(
+          s, small, seed, stream, skip, begin, end,
+          [&](int64_t p, int64_t& k, double& E) {
+            k = k0 + list[sl][p];
+            E = ekin[(total == n) ? k : (k % n)];
+            return true;
+          },
+          [](bool) {},
+          [&](int64_t k, int rc, double Ef, double mu) {
+            if (rc) atomicAdd(nerr, 1ull);
+            oE[k] = rc ? -1.0 : Ef;
+            if constexpr (Dirs) {  // errors only
+              o2[3 * k] = 0.0; o2[3 * k + 1] = 0.0; o2[3 * k + 2] = 0.0;
+            } else {
+              o2[k] = rc ? -999.0 : mu;
+            }
+          },
+          [&](int64_t k, double Ef, double ox, double oy, double oz) {
+            oE[k] = Ef;
+            o2[3 * k] = ox; o2[3 * k + 1] = oy; o2[3 * k + 2] = oz;
+          },
+          [&](int64_t k, double& ix, double& iy, double& iz) {
+            ix = dirs[3 * k]; iy = dirs[3 * k + 1]; iz = dirs[3 * k + 2];
+          });
+    }
+    for (int j = 255 - tid; j < high; j += 256) {  // from the waves that had the least above
+      const int64_t k = k0 + list[sl][kList - 1 - j];
+      Rng rng;
+      rng.init(seed, stream, (uint64_t)k);
+      if (skip) rng.gen();
+      double Ef, mu;
+      const int rc = sab_sample_iso<true>(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
+      comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
+    }
+  }
+}
+
 __global__ void __launch_bounds__(256) k_sab_ab(SABView s, const double* __restrict__ ekin, int64_t n,
                                                 uint64_t seed, uint32_t stream, double* __restrict__ oa,
                                                 double* __restrict__ ob,
@@ -486,6 +591,39 @@ void launch_stages(const CompView& c, const double* ekin, const double* dirs, in
 }
 
 
+// Batches of at most 512 workgroups of 256 neutrons are staged within workgroups
+// (rock salt, two S(alpha,beta) components, isotropic call of 100003 neutrons: 67
+// against 99 us; powder, 1000 neutrons: 31 against 52 us through the queues; 1e6: 227 against 195 us, where full waves
+// count more).
+constexpr int64_t kLocalMax = 512 * 256;
+template <bool Dirs>
+void launch_staged(const CompView& c, const double* ekin, const double* dirs, int64_t n, int64_t total, uint64_t seed,
+                   uint32_t stream, double* oE, double* o2, unsigned long long* nerr, int64_t* queues,
+                   unsigned long long* qcount, hipStream_t st, const double* ext, int64_t* cq,
+                   unsigned long long* cqc) {
+  const bool gas = comp_has_gas(c);
+  if (total <= kLocalMax) {
+    bool fits = true;
+    for (int sl = 0; sl < c.nstaged; ++sl)
+      if (c.kind[c.stage_comp[sl]] == kKindSAB) fits = fits && sab_small_fits(c.sab[sl]);
+    const int64_t spread = (total + 767) / 768;  // three workgroups per CU
+    const int per = (int)(spread < 16 ? 16 : (spread > 256 ? 256 : spread));
+    const dim3 g((unsigned)((total + per - 1) / per)), b(256);
+    const auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, g, b, 0, st, c, ekin, dirs, n, total, seed, stream, oE, o2, nerr, ext, cq, cqc, per);
+    };
+    if (gas) fits ? go(k_comp_local<Dirs, true, true>) : go(k_comp_local<Dirs, true, false>);
+    else fits ? go(k_comp_local<Dirs, false, true>) : go(k_comp_local<Dirs, false, false>);
+    return;
+  }
+  hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, 2 * kMaxStaged);
+  const dim3 g(grid_for(total, kPickThreads)), b(kPickThreads);
+  hipLaunchKernelGGL((gas ? k_comp_pick<Dirs, true> : k_comp_pick<Dirs, false>), g, b, 0, st, c, ekin, dirs, n, total,
+                     seed, stream, oE, o2, nerr, queues, qcount, ext, cq, cqc);
+  launch_stages<Dirs>(c, ekin, dirs, n, total, seed, stream, oE, o2, nerr, queues, qcount, st);
+}
+
+
 // synthetic neutron energies, log-uniform, from a dedicated Philox stream
 __global__ void __launch_bounds__(256) k_fill_loguniform(double* __restrict__ out, int64_t n, double lemin,
                                                          double lemax, uint64_t seed) {
@@ -553,19 +691,9 @@ void launch_sample_iso(const CompView& c, const double* ekin, int64_t n, int64_t
       hipLaunchKernelGGL(k_sample_iso<kCompFG>, dim3(grid_for(total, 256)), dim3(256), 0, st, c, ekin, n, total,
                          seed, stream, oE, oMu, nerr);
       break;
-    default: {
-      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, 2 * kMaxStaged);
-      const dim3 g(grid_for(total, kPickThreads)), b(kPickThreads);
-      if (comp_has_gas(c))
-        hipLaunchKernelGGL((k_comp_pick<false, true>), g, b, 0, st, c, ekin, (const double*)nullptr, n, total, seed,
-                           stream, oE, oMu, nerr, queues, qcount, (const double*)nullptr, (int64_t*)nullptr,
-                           (unsigned long long*)nullptr);
-      else
-        hipLaunchKernelGGL((k_comp_pick<false, false>), g, b, 0, st, c, ekin, (const double*)nullptr, n, total,
-                           seed, stream, oE, oMu, nerr, queues, qcount, (const double*)nullptr, (int64_t*)nullptr,
-                           (unsigned long long*)nullptr);
-      launch_stages<false>(c, ekin, nullptr, n, total, seed, stream, oE, oMu, nerr, queues, qcount, st);
-    }
+    default:
+      launch_staged<false>(c, ekin, nullptr, n, total, seed, stream, oE, oMu, nerr, queues, qcount, st, nullptr,
+                           nullptr, nullptr);
   }
 }
 __global__ void __launch_bounds__(256) k_xs_ext(CompView c, const double* __restrict__ ekin,
@@ -599,17 +727,8 @@ void launch_sample_dirs(const CompView& c, const double* ekin, const double* dir
       hipLaunchKernelGGL(k_sample_dirs<kCompFG>, dim3(grid_for(n, 256)), dim3(256), 0, st, c, ekin, dirs, n,
                          seed, stream, oE, oD, nerr);
       break;
-    default: {
-      hipLaunchKernelGGL(k_zero_u64_n, dim3(1), dim3(64), 0, st, qcount, 2 * kMaxStaged);
-      const dim3 g(grid_for(n, kPickThreads)), b(kPickThreads);
-      if (comp_has_gas(c))
-        hipLaunchKernelGGL((k_comp_pick<true, true>), g, b, 0, st, c, ekin, dirs, n, n, seed, stream, oE, oD, nerr,
-                           queues, qcount, ext, cq, cqc);
-      else
-        hipLaunchKernelGGL((k_comp_pick<true, false>), g, b, 0, st, c, ekin, dirs, n, n, seed, stream, oE, oD, nerr,
-                           queues, qcount, ext, cq, cqc);
-      launch_stages<true>(c, ekin, dirs, n, n, seed, stream, oE, oD, nerr, queues, qcount, st);
-    }
+    default:
+      launch_staged<true>(c, ekin, dirs, n, n, seed, stream, oE, oD, nerr, queues, qcount, st, ext, cq, cqc);
   }
 }
 void launch_sab_ab(const SABView& s, const double* ekin, int64_t n, uint64_t seed, uint32_t stream, double* oa,

@@ -403,11 +403,11 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
   after(true);
 }
 
-// positions of a wave's share of a list of n among nw waves: at least 64 each,
-// so that a wave is filled before the next one is begun
-NCD void sab_share(int64_t n, int64_t w, int64_t nw, int64_t& begin, int64_t& end) {
+// positions of a wave's share of a list of n among nw waves: at least `fill`
+// each (64: a wave is filled before the next one is begun)
+NCD void sab_share(int64_t n, int64_t w, int64_t nw, int64_t& begin, int64_t& end, int fill = 64) {
   int64_t per = (n + nw - 1) / nw;
-  per = per < 64 ? 64 : per;
+  per = per < fill ? fill : per;
   begin = w * per < n ? w * per : n;
   end = begin + per < n ? begin + per : n;
 }
