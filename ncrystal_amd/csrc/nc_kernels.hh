@@ -176,6 +176,8 @@ NCHD bool comp_has_gas(const CompView& c) {
 // per-neutron kernels (nc_kernels.hip)
 void launch_xs_iso(const CompView&, const double* ekin, int64_t n, int64_t repeat, double* out, bool fp32,
                    hipStream_t);
+// whether a staged composition's call of `total` neutrons needs no queues
+bool staged_locally(int64_t total);
 // queues: [nstaged x n*repeat] neutron indices (one queue per staged
 // component, filled from both ends), qcount: [2 kMaxStaged] counters (used by
 // compositions with an S(alpha,beta) part)

@@ -593,16 +593,17 @@ void launch_stages(const CompView& c, const double* ekin, const double* dirs, in
 
 // Batches of at most 512 workgroups of 256 neutrons are staged within workgroups
 // (rock salt, two S(alpha,beta) components, isotropic call of 100003 neutrons: 67
-// against 99 us; powder, 1000 neutrons: 31 against 52 us through the queues; 1e6: 227 against 195 us, where full waves
-// count more).
+// against 99 us through the queues; powder, 1000 neutrons: 31 against 52 us; rock
+// salt, 1e6: 227 against 195 us, where full waves count more).
 constexpr int64_t kLocalMax = 512 * 256;
+bool staged_locally(int64_t total) { return total <= kLocalMax; }
 template <bool Dirs>
 void launch_staged(const CompView& c, const double* ekin, const double* dirs, int64_t n, int64_t total, uint64_t seed,
                    uint32_t stream, double* oE, double* o2, unsigned long long* nerr, int64_t* queues,
                    unsigned long long* qcount, hipStream_t st, const double* ext, int64_t* cq,
                    unsigned long long* cqc) {
   const bool gas = comp_has_gas(c);
-  if (total <= kLocalMax) {
+  if (staged_locally(total)) {
     bool fits = true;
     for (int sl = 0; sl < c.nstaged; ++sl)
       if (c.kind[c.stage_comp[sl]] == kKindSAB) fits = fits && sab_small_fits(c.sab[sl]);
