@@ -474,47 +474,51 @@ __global__ void __launch_bounds__(kCumulBlock) k_fp32_cumul_scan(const double* _
   }
 }
 
-// search guides of a PowderBragg table: IEEE-bit buckets of the energy
-// axis for the threshold search and equal-value buckets of the cumulative
-// sum for the plane pick.  Each bucket stores the search answer at its lower
-// edge, so a bracket [bucket, next bucket] (widened by one bucket for the
-// rounding of target*scale) always contains the plain binary-search answer.
+// search guides of a PowderBragg table: equal-width buckets of the energy for
+// the threshold search (the number of planes up to E grows as E^1.5, so their
+// density changes little along it) and of the cumulative sum for the plane
+// pick.  A bucket holds the planes that a plain binary search can end at.
+// kPBBuckets buckets per plane at most, and bounded where a finer guide would
+// take more of a die's L2 cache than its shorter searches give back: at 262k
+// planes (figures at PBView's lookups) 2^17 energy buckets cost 1.38 ms for
+// 1.27 with 2^18, and 2^19 the same as 2^18; 2^18 cumulative ones 1.14 ms for 1.12
+// with 2^16
+constexpr int kPBGuideE = 1 << 18, kPBGuideC = 1 << 16, kPBBuckets = 16;
+
 void pb_guides(Proc* p, const std::vector<double>& e2d, const std::vector<double>& fdm) {
   const int n = (int)e2d.size();
-  auto bits = [](double x) { unsigned long long u; std::memcpy(&u, &x, 8); return u; };
-  auto fromb = [](unsigned long long u) { double x; std::memcpy(&x, &u, 8); return x; };
-  // about 4 buckets per plane over the [e2d[0], e2d[n-1]] range, at most 2^20
-  int shift = 52, m = 0;
-  long long base = 0, nbkt = 1;
-  for (m = 20; m >= 0; --m) {
-    shift = 52 - m;
-    base = (long long)(bits(e2d.front()) >> shift);
-    nbkt = (long long)(bits(e2d.back()) >> shift) - base + 1;
-    if (nbkt <= std::max<long long>(64, 4LL * n) && nbkt <= (1 << 20)) break;
+  // lo, hi of every bucket: the planes in buckets below it and up to it
+  auto guide = [n](const std::vector<double>& x, int nb, double scale, std::vector<PBGuide>& out) {
+    out.resize((size_t)nb);
+    for (int g = 0, i = 0; g < nb; ++g) {
+      const int lo = i;
+      while (i < n && pb_bucket(x[(size_t)i], scale, nb) <= g) ++i;
+      out[(size_t)g] = {lo, i, 0.0};
+    }
+  };
+  std::vector<PBGuide> eg, cg;
+  PBView& v = p->pb;
+  const long long want = std::max<long long>(64, (long long)kPBBuckets * n);
+  v.e_n = (int)std::min<long long>(kPBGuideE, want);
+  v.c_n = (int)std::min<long long>(kPBGuideC, want);
+  v.e_scale = (double)v.e_n / v.top;
+  v.c_scale = (double)v.c_n / v.all;
+  guide(e2d, v.e_n, v.e_scale, eg);
+  for (PBGuide& g : eg) {  // E >= the first energy: a plane before is always there
+    const int lo = std::max(1, g.lo), hi = std::max(1, g.cnt);
+    g = {lo, hi - lo, fdm[(size_t)lo - 1]};
   }
-  if (m < 0) { m = 0; shift = 52; base = (long long)(bits(e2d.front()) >> shift);
-               nbkt = (long long)(bits(e2d.back()) >> shift) - base + 1; }
-  std::vector<int> eb((size_t)nbkt + 1);
-  for (long long b = 0; b <= nbkt; ++b) {
-    const double edge = fromb((unsigned long long)(base + b) << shift);
-    eb[(size_t)b] = (int)(std::upper_bound(e2d.begin(), e2d.end(), edge) - e2d.begin());
+  guide(fdm, v.c_n, v.c_scale, cg);
+  for (PBGuide& g : cg) {  // a target is at most the last value: its plane is below n
+    const int lo = std::min(g.lo, n - 1), hi = std::min(g.cnt, n - 1);
+    g = {lo, hi - lo, e2d[(size_t)lo]};
   }
-  eb[(size_t)nbkt] = n;
-  const int cn = (int)std::min<long long>(1 << 20, std::max<long long>(64, 4LL * n));
-  const double scale = (double)cn / fdm.back();
-  std::vector<int> cg((size_t)cn + 1);
-  for (int g = 0; g < cn; ++g)
-    cg[(size_t)g] = (int)(std::lower_bound(fdm.begin(), fdm.end(), (double)g / scale) - fdm.begin());
-  cg[(size_t)cn] = n;
-  DevBuf* b1 = p->newbuf(); b1->upload(eb.data(), eb.size());
-  DevBuf* b2 = p->newbuf(); b2->upload(cg.data(), cg.size());
-  p->pb.e_bucket = b1->as<int>();
-  p->pb.e_base = base;
-  p->pb.e_shift = shift;
-  p->pb.e_nbkt = (int)nbkt;
-  p->pb.c_guide = b2->as<int>();
-  p->pb.c_n = cn;
-  p->pb.c_scale = scale;
+  DevBuf* be = p->newbuf();
+  be->upload(eg.data(), eg.size());
+  v.eg = be->as<PBGuide>();
+  DevBuf* bc = p->newbuf();
+  bc->upload(cg.data(), cg.size());
+  v.cg = bc->as<PBGuide>();
 }
 
 void pb_upload(Proc* p, const std::vector<double>& e2d, const std::vector<double>& fdm,
@@ -567,12 +571,13 @@ void pb_upload(Proc* p, const std::vector<double>& e2d, const std::vector<double
                const std::vector<double>& contrib, bool fp32) {
   p->pb.n = (int)fdm.size();
   p->pb.threshold = fdm.empty() ? __builtin_huge_val() : e2d.front();
-  DevBuf* be = p->newbuf();
-  be->upload(e2d.data(), e2d.size());
-  DevBuf* bf = p->newbuf();
-  bf->upload(fdm.data(), fdm.size());
-  p->pb.e2d = be->as<double>();
-  p->pb.fdm = bf->as<double>();
+  std::vector<double2> ef(fdm.size());
+  for (size_t i = 0; i < ef.size(); ++i) ef[i] = make_double2(e2d[i], fdm[i]);
+  DevBuf* bef = p->newbuf();
+  bef->upload(ef.data(), ef.size());
+  p->pb.ef = bef->as<double2>();
+  p->pb.top = fdm.empty() ? 0.0 : e2d.back();
+  p->pb.all = fdm.empty() ? 0.0 : fdm.back();
   p->pb.fdm32 = nullptr;
   if (!fdm.empty()) pb_guides(p, e2d, fdm);
   p->pb_e2d_h = e2d;

@@ -237,51 +237,104 @@ NCD int pick_idx(Rng& rng, const double* commul, int n) {
 
 // ---------------------------------------------------------------------------
 // PowderBragg
-struct PBView {
-  const double* e2d;    // [n] 2d-spacing thresholds in energy units, descending d
-  const double* fdm;    // [n] cumulative d*|F|^2*mult*c (FP64)
-  const float* fdm32;   // [n] same, FP32 (compensated build), may be null
-  int n;
-  double threshold;     // e2d[0]
-  // search guides (exact: every bracket contains the plain binary-search answer)
-  const int* e_bucket;  // [e_nbkt+1] upper_bound(e2d, bucket lower edge), IEEE-bit buckets of E
-  long long e_base;     // bits(e2d[0]) >> e_shift
-  int e_shift, e_nbkt;
-  const int* c_guide;   // [c_n+1] lower_bound(fdm, g / c_scale), last entry n
-  int c_n;
-  double c_scale;       // c_n / fdm[n-1]
+// one bucket of a search guide: the answer is in [lo, lo + cnt], v belongs to
+// the answer lo
+struct PBGuide {
+  int lo, cnt;
+  double v;
 };
-// index of the last plane with 2d >= wavelength (E >= threshold assumed)
-NCD int pb_last_valid(const PBView& pb, double E) {
-  if (!(E < pb.e2d[pb.n - 1])) return pb.n - 1;
-  const long long b = (long long)((unsigned long long)__double_as_longlong(E) >> pb.e_shift) - pb.e_base;
-  const int lo = max(pb.e_bucket[b], 1), hi = pb.e_bucket[b + 1];
-  return upper_bound_d(pb.e2d, lo, hi, E) - 1;
+struct PBView {
+  const double2* ef;    // [n] 2d-spacing thresholds in energy units, descending d, and
+                        //     the cumulative d*|F|^2*mult*c there (FP64)
+  const float* fdm32;   // [n] the latter in FP32 (compensated build), may be null
+  int n;
+  double threshold;     // first energy
+  double top;           // last energy
+  double all;           // last cumulative value
+  const PBGuide* eg;    // [e_n] buckets pb_bucket of the energy: upper_bound, v the cumulative
+                        //       value of the plane before (from the first plane on)
+  const PBGuide* cg;    // [c_n] buckets pb_bucket of the cumulative value: lower_bound, v its energy
+  int e_n, c_n;
+  double e_scale;       // e_n / top
+  double c_scale;       // c_n / all
+};
+// The lookups are bound by their loads, each lane's at a place of its own: the
+// address unit is busy 85% of the time.  So a bucket carries the value that
+// belongs to its first answer, which most lanes need nothing beyond, a search
+// keeps the partner of the value it ends at, and each is one 16-byte load (the
+// vector types: of a struct the compiler makes two).  262k planes, 5e7 neutrons,
+// E log-uniform 0.1 meV to 1 eV: cross sections 574 -> 430 us, sampling 1015 ->
+// 690 us against a guide of indices into two arrays.
+// bucket of a value; monotone, so its lower and upper bound among the planes'
+// are between the numbers of planes in buckets below its own and up to its own
+NCHD int pb_bucket(double x, double scale, int n) {
+  const long long g = (long long)(x * scale);
+  return (int)(g < 0 ? 0 : (g < n ? g : n - 1));
 }
-// lower_bound over fdm[0..idx) of a target in [0, fdm[idx]]
-NCD int pb_pick_plane(const PBView& pb, int idx, double target) {
-  long long g = (long long)(target * pb.c_scale);
-  g = g < 0 ? 0 : (g >= pb.c_n ? pb.c_n - 1 : g);
-  const int lo = pb.c_guide[g > 0 ? g - 1 : 0];
-  int hi = pb.c_guide[g + 2 <= pb.c_n ? g + 2 : pb.c_n];
-  hi = hi < idx ? hi : idx;
-  return lower_bound_d(pb.fdm, lo < hi ? lo : hi, hi, target);
+typedef int pb_int4 __attribute__((ext_vector_type(4)));
+typedef double pb_double2 __attribute__((ext_vector_type(2)));
+NCD PBGuide pb_guide(const PBGuide* __restrict__ g) {
+  const pb_int4 q = *reinterpret_cast<const pb_int4*>(g);
+  return {q.x, q.y, __hiloint2double(q.w, q.z)};
+}
+NCD pb_double2 pb_plane(const PBView& pb, int i) { return reinterpret_cast<const pb_double2*>(pb.ef)[i]; }
+// index of the last plane with 2d >= wavelength (E >= threshold assumed) and
+// the planes' cumulative value there
+NCD int pb_last_valid(const PBView& pb, double E, double& fdm) {
+  fdm = pb.all;
+  if (!(E < pb.top)) return pb.n - 1;
+  const PBGuide g = pb_guide(pb.eg + pb_bucket(E, pb.e_scale, pb.e_n));
+  int lo = g.lo, hi = g.lo + g.cnt;
+  fdm = g.v;
+  while (lo < hi) {  // upper_bound
+    const int m = (lo + hi) >> 1;
+    const pb_double2 q = pb_plane(pb, m);
+    if (!(E < q.x)) {
+      lo = m + 1;
+      fdm = q.y;
+    } else {
+      hi = m;
+    }
+  }
+  return lo - 1;
+}
+// threshold energy of the plane lower_bound(fdm, target), target in
+// [0, fdm[n-1]]
+NCD double pb_pick_plane(const PBView& pb, double target) {
+  const PBGuide g = pb_guide(pb.cg + pb_bucket(target, pb.c_scale, pb.c_n));
+  if (g.cnt == 0) return g.v;
+  int lo = g.lo, hi = g.lo + g.cnt;
+  double e = 0.0;
+  bool have = false;  // e is the energy at hi
+  while (lo < hi) {   // lower_bound
+    const int m = (lo + hi) >> 1;
+    const pb_double2 q = pb_plane(pb, m);
+    if (q.y < target) {
+      lo = m + 1;
+    } else {
+      hi = m;
+      e = q.x;
+      have = true;
+    }
+  }
+  return have ? e : pb.ef[hi].x;
 }
 NCD bool pb_active(const PBView& pb, double E) {
   return pb.n > 0 && !(E < pb.threshold) && isfinite(E);
 }
 NCD double pb_xs(const PBView& pb, double E) {
   if (!pb_active(pb, E)) return 0.0;
-  const int idx = pb_last_valid(pb, E);
+  double fdm;
+  pb_last_valid(pb, E, fdm);
   const double inv = 1.0 / E;
-  return pb.fdm[idx] * inv;
+  return fdm * inv;
 }
 NCD double pb_sample_mu(const PBView& pb, Rng& rng, double E) {
   if (!pb_active(pb, E)) return 1.0;
-  const int idx = pb_last_valid(pb, E);
+  double fdm;
+  pb_last_valid(pb, E, fdm);
   const double u = rng.gen();
-  const int i = pb_pick_plane(pb, idx, u * pb.fdm[idx]);
-  const double s2 = pb.e2d[i] / E;
+  const double s2 = pb_pick_plane(pb, u * fdm) / E;
   return 1.0 - 2.0 * s2;
 }
 

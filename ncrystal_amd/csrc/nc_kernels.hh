@@ -53,7 +53,8 @@ template <bool FP32PB>
 NCD double pb_xs_sel(const PBView& pb, double E) {
   if constexpr (FP32PB) {
     if (!pb_active(pb, E)) return 0.0;
-    const int idx = pb_last_valid(pb, E);
+    double fdm;
+    const int idx = pb_last_valid(pb, E, fdm);
     const double inv = 1.0 / E;
     return (double)pb.fdm32[idx] * inv;
   } else {

@@ -12,20 +12,22 @@
 namespace ncamd {
 
 // Variant kCompPBOnly: a single PowderBragg component (the same sum as
-// comp_xs: 0 + scale * xs); kCompFG: FreeGas / absorption components
+// comp_xs: 0 + scale * xs); kCompFG: FreeGas / absorption components.  The
+// neutrons and results pass by the caches, which are left to the tables
+// (PowderBragg, 262k planes, 5e7 neutrons, both kernels: 1341 -> 1279 us)
 template <bool FP32PB, int Variant>
 __global__ void __launch_bounds__(256) k_xs_iso(CompView c, const double* __restrict__ ekin,
                                                 int64_t n, int64_t repeat, double* __restrict__ out) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const double E = ekin[i];
+    const double E = __builtin_nontemporal_load(ekin + i);
     double xs;
     if constexpr (Variant == kCompPBOnly) {
       xs = comp_outside(c, E) ? 0.0 : 0.0 + c.scale[0] * (pb_active(c.pb, E) ? pb_xs_sel<FP32PB>(c.pb, E) : 0.0);
     } else {
       xs = comp_xs<FP32PB, Variant == kCompFG>(c, E, nullptr);  // kCompFG: any composition with gas components
     }
-    for (int64_t r = 0; r < repeat; ++r) out[r * n + i] = xs;
+    for (int64_t r = 0; r < repeat; ++r) __builtin_nontemporal_store(xs, out + r * n + i);
   }
 }
 
@@ -41,10 +43,10 @@ __global__ void __launch_bounds__(256) k_sample_iso(CompView c, const double* __
     Rng rng;
     rng.init(seed, stream, (uint64_t)k);
     double Ef, mu;
-    const int rc = comp_sample_iso<Variant>(c, rng, ekin[i], Ef, mu);
+    const int rc = comp_sample_iso<Variant>(c, rng, __builtin_nontemporal_load(ekin + i), Ef, mu);
     if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
-    oE[k] = Ef;
-    oMu[k] = mu;
+    __builtin_nontemporal_store(Ef, oE + k);
+    __builtin_nontemporal_store(mu, oMu + k);
   }
 }
 
