@@ -53,20 +53,18 @@ struct SabSmall {
     start = egrid + s.ne;
   }
 };
-// two neighbouring points (48 bytes) as three loads
+// two neighbouring points (48 bytes) as three loads (the vector type keeps the
+// compiler from splitting them)
+typedef double sab_double2 __attribute__((ext_vector_type(2), aligned(8)));
 NCD void load_points(const SabPt* __restrict__ p, SabPt& p0, SabPt& p1) {
-  double2 a, b, c;
-  __builtin_memcpy(&a, &p->s, 16);
-  __builtin_memcpy(&b, &p->cumul, 16);
-  __builtin_memcpy(&c, &p[1].logs, 16);
+  const sab_double2* q = reinterpret_cast<const sab_double2*>(p);
+  const sab_double2 a = q[0], b = q[1], c = q[2];
   p0 = SabPt{a.x, a.y, b.x};
   p1 = SabPt{b.y, c.x, c.y};
 }
 NCD void load_bins(const SabBin* __restrict__ p, SabBin& p0, SabBin& p1) {
-  double2 a, b, c;
-  __builtin_memcpy(&a, &p->cdf, 16);
-  __builtin_memcpy(&b, &p->y, 16);
-  __builtin_memcpy(&c, &p[1].x, 16);
+  const sab_double2* q = reinterpret_cast<const sab_double2*>(p);
+  const sab_double2 a = q[0], b = q[1], c = q[2];
   p0 = SabBin{a.x, a.y, b.x};
   p1 = SabBin{b.y, c.x, c.y};
 }
