@@ -973,7 +973,7 @@ def run_lcbragg(args):
                    "neutrons": n, "xs_ms": xs_ms, "sample_ms": samp_ms,
                    "xs_neutrons_per_s": n / (xs_ms * 1e-3)},
         "roofline": {"bound": "fp64-valu", "achieved": None, "peak": None, "unit": None, "frac": None,
-                     "traffic": None, "kernel": "k_lc0_xs (per-neutron Romberg averages over rotation ranges)",
+                     "traffic": None, "kernel": "k_lc0<false> (per-neutron Romberg averages over rotation ranges)",
                      "note": "40 B of HBM traffic per neutron; the FP64 Romberg arithmetic of each range bounds it"},
         "cpu_baseline": cpu,
     }

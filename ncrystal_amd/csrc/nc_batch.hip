@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(kBatchBlock, 2) k_batch_highe(const BatchMat* 
     rng.init(r.seed, (uint32_t)r.stream, (uint64_t)k);
     if (m.view.n > 1) rng.gen();
     double Ef, mu;
-    const int rc = sab_sample_iso<true>(m.view.sab[0], rng, ekin[m.offset + k], Ef, mu);
+    const int rc = sab_sample_iso(m.view.sab[0], rng, ekin[m.offset + k], Ef, mu);
     if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
     o1[m.offset + k] = Ef;
     o2[m.offset + k] = mu;

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <exception>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -134,7 +135,11 @@ class HostStage {
       raise("HIPError", "hipHostGetDevicePointer");
     }
   }
-  ~HostStage() { give_back(); }
+  ~HostStage() {
+    // on the way out of an error a kernel may still be writing
+    if (std::uncaught_exceptions() > unwinding_) (void)hipDeviceSynchronize();
+    give_back();
+  }
   HostStage(const HostStage&) = delete;
   HostStage& operator=(const HostStage&) = delete;
   // arrays of kHostStage values each, and one counter at the end
@@ -146,6 +151,7 @@ class HostStage {
   static constexpr size_t kArrays = 3;
   static constexpr size_t kBytes = (kArrays * kHostStage + 1) * sizeof(double);
   double *host_ = nullptr, *dev_ = nullptr;
+  const int unwinding_ = std::uncaught_exceptions();
   static std::mutex& mtx() {
     static std::mutex m;
     return m;

@@ -723,14 +723,12 @@ NCD int sab_sample_highe(const SABView& s, double E, Rng& rng, double& a_out, do
 }
 
 // SABSampler::sampleAlphaBeta (NCSABSampler.cc:158-227)
-template <bool WithHighE = true>
 NCD int sab_sample_ab(const SABView& s, double E, Rng& rng, double& a_out, double& b_out) {
   int up = egrid_upper_bound(s, E);
   bool ultra = false;
   const double ultra_e = s.egrid[0];
   int isamp;
   if (up == s.ne) {
-    if constexpr (!WithHighE) return kErrBadSampler;  // caller routes E >= Emax elsewhere
     double a, b;
     const int rc = sab_sample_highe(s, E, rng, a, b);
     if (rc) return rc;
@@ -784,10 +782,9 @@ NCD int sab_ab_to_emu(const SABView& s, Rng& rng, double E, double a, double b, 
   mu = m;
   return kOK;
 }
-template <bool WithHighE = true>
 NCD int sab_sample_iso(const SABView& s, Rng& rng, double E, double& Ef, double& mu) {
   double a, b;
-  const int rc = sab_sample_ab<WithHighE>(s, E, rng, a, b);
+  const int rc = sab_sample_ab(s, E, rng, a, b);
   if (rc) return rc;
   return sab_ab_to_emu(s, rng, E, a, b, Ef, mu);
 }

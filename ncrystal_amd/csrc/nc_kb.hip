@@ -237,7 +237,7 @@ __global__ void k_kb_queue_ab(SABView s, const double* __restrict__ ekin, uint64
     Rng rng;
     rng.init(seed, stream, (uint64_t)kk);
     double a = -1.0, b = 0.0;
-    if (sab_sample_ab<true>(s, ekin[kk], rng, a, b)) { a = -1.0; b = 0.0; }
+    if (sab_sample_ab(s, ekin[kk], rng, a, b)) { a = -1.0; b = 0.0; }
     oa[kk] = a;
     ob[kk] = b;
   }

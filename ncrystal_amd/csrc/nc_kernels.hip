@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(256, 4) k_comp_sab(SABView s, const double* __
       rng.init(seed, stream, (uint64_t)k);
       if (skip) rng.gen();
       double Ef, mu;
-      const int rc = sab_sample_iso<true>(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
+      const int rc = sab_sample_iso(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
       comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
     }
     return;
@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(256, 4) k_comp_local(CompView c, const double*
       rng.init(seed, stream, (uint64_t)k);
       if (skip) rng.gen();
       double Ef, mu;
-      const int rc = sab_sample_iso<true>(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
+      const int rc = sab_sample_iso(s, rng, ekin[(total == n) ? k : (k % n)], Ef, mu);
       comp_store<Dirs>(k, rc, Ef, mu, rng, dirs, oE, o2, nerr);
     }
   }
@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(256) k_sab_sample_iso_highe(SABView s, const d
     Rng rng;
     rng.init(seed, stream, (uint64_t)k);
     double Ef, mu;
-    const int rc = sab_sample_iso<true>(s, rng, ekin[i], Ef, mu);
+    const int rc = sab_sample_iso(s, rng, ekin[i], Ef, mu);
     if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
     oE[k] = Ef;
     oMu[k] = mu;

@@ -22,9 +22,9 @@
 // Lanes of a wavefront scan the demi-normals together: the normal index is
 // wave-uniform (the records are scalar loads shared by the 64 lanes) and a
 // lane whose families are exhausted is masked.  The rare backscattering
-// geometry that needs the Romberg circle integral is left to a second kernel
-// (AllowSlow=true) through a queue, so the main kernel carries no Romberg
-// state.
+// geometry that needs the Romberg circle integral goes through a queue to a
+// second kernel, a wave per neutron (scb_candidate<true>), so the main kernel
+// carries no Romberg state.
 #pragma once
 #include "nc_dev.hh"
 #include "nc_math.hh"
