@@ -12,11 +12,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <exception>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -63,10 +64,15 @@ struct Error : std::runtime_error {
 };
 [[noreturn]] void raise(const char* type, const std::string& msg) { throw Error(type, msg); }
 
-#define NCAMD_HIP(call)                                                                       \
-  do {                                                                                        \
-    hipError_t e_ = (call);                                                                   \
-    if (e_ != hipSuccess) raise("HIPError", std::string(#call) + ": " + hipGetErrorString(e_)); \
+// (the error is taken from HIP as it is raised: kept there as the last error, it
+// would be reported again by the next call's check of its launches)
+#define NCAMD_HIP(call)                                                         \
+  do {                                                                          \
+    hipError_t e_ = (call);                                                     \
+    if (e_ != hipSuccess) {                                                     \
+      (void)hipGetLastError();                                                  \
+      raise("HIPError", std::string(#call) + ": " + hipGetErrorString(e_));     \
+    }                                                                           \
   } while (0)
 
 #define NCAMD_TRY try {
@@ -3241,10 +3247,22 @@ void ncamd_setrngstate(ncamd_process_t h, uint64_t seed, uint64_t ctr) {
 }
 
 // ---- host pointer API
-// batches that go through a HostStage (not empty, and a repeat count that
-// cannot overflow the product)
-static bool small_call(unsigned long n, unsigned long repeat) {
-  return n > 0 && repeat > 0 && n <= kHostStage && repeat <= kHostStage / n;
+// memory that the host itself may read and write (0.1 us): not NULL, which the
+// copies of the general route refuse, nor device memory, which they take
+static bool host_memory(const void* p) {
+  if (!p) return false;
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();  // memory that HIP does not know
+    return true;
+  }
+  return a.type != hipMemoryTypeDevice && a.type != hipMemoryTypeArray;
+}
+// calls that go through a HostStage (not empty, a repeat count that cannot
+// overflow the product, arrays in host memory)
+static bool small_call(unsigned long n, unsigned long repeat, std::initializer_list<const void*> arrays) {
+  return n > 0 && repeat > 0 && n <= kHostStage && repeat <= kHostStage / n &&
+         std::all_of(arrays.begin(), arrays.end(), host_memory);
 }
 static void xs_many_impl(ncamd_process_t h, const double* ekin, unsigned long n, unsigned long repeat, double* out,
                          bool fp32) {
@@ -3252,7 +3270,7 @@ static void xs_many_impl(ncamd_process_t h, const double* ekin, unsigned long n,
   NCAMD_TRY
   Proc* p = extract(h);  // an invalid handle is a LogicError before any device check
   ensure_device();
-  if (small_call(n, repeat)) {
+  if (small_call(n, repeat, {ekin, out})) {
     const HostStage st;
     std::copy(ekin, ekin + n, st.host(0));
     xs_dispatch(p, st.dev(0), (int64_t)n, (int64_t)repeat, st.dev(1), fp32, 0);
@@ -3288,7 +3306,7 @@ void ncamd_samplescatterisotropic_many(ncamd_process_t h, const double* ekin, un
   Proc* p = extract(h);  // an invalid handle is a LogicError before any device check
   ensure_device();
   const size_t tot = (size_t)n * repeat;
-  if (small_call(n, repeat)) {
+  if (small_call(n, repeat, {ekin, oE, oMu})) {
     const HostStage st;
     std::copy(ekin, ekin + n, st.host(0));
     sample_iso_dispatch(p, st.dev(0), (int64_t)n, (int64_t)repeat, st.dev(1), st.dev(2), 0);

@@ -1,6 +1,7 @@
 """Host-array calls around the size that goes through pinned staging: the same
 values as larger calls on the same streams, repeats, poisoned outputs, and several
 threads on handles of their own."""
+import ctypes
 import threading
 
 import numpy as np
@@ -62,3 +63,28 @@ def test_threads(mat):
     for t in ts:
         t.join()
     assert all(np.array_equal(g[0], want[0]) and np.array_equal(g[1], want[1]) for g in got)
+
+
+@pytest.mark.parametrize("n", [64, 5000])  # either side of the staging size
+def test_null_and_device_arrays(mat, n):
+    """no energies are an error that poisons the outputs, and device memory in
+    place of host arrays is copied like them, at every size"""
+    from ncrystal_amd import _capi as C
+    e = synth.energies_logu(n, 1e-4, 1.0, seed=5)
+    x, oe, om = np.zeros(n), np.zeros(n), np.zeros(n)
+    with pytest.raises(C.NCAMDError, match="HIPError"):
+        C.call("ncamd_crosssection_nonoriented_many", mat.handle, None, n, 1, C.dptr(x))
+    with pytest.raises(C.NCAMDError, match="HIPError"):
+        C.call("ncamd_samplescatterisotropic_many", mat.handle, None, n, 1, C.dptr(oe), C.dptr(om))
+    assert np.all(x == -1.0) and np.all(oe == -1.0) and np.all(om == -999.0)
+    want = mat.crossSectionIsotropic(e)
+    mat.setRNGState(3, 0)
+    ws = mat.sampleScatterIsotropic(e)
+    de, dx, do, dm = C.DeviceArray.from_numpy(e), C.DeviceArray(n), C.DeviceArray(n), C.DeviceArray(n)
+    p = lambda d: ctypes.cast(d.ptr, C._dp)
+    C.call("ncamd_crosssection_nonoriented_many", mat.handle, p(de), n, 1, C.dptr(x))
+    C.call("ncamd_crosssection_nonoriented_many", mat.handle, C.dptr(e), n, 1, p(dx))
+    mat.setRNGState(3, 0)
+    C.call("ncamd_samplescatterisotropic_many", mat.handle, p(de), n, 1, p(do), p(dm))
+    assert np.array_equal(x, want) and np.array_equal(dx.numpy(), want)
+    assert np.array_equal(do.numpy(), ws[0]) and np.array_equal(dm.numpy(), ws[1])
