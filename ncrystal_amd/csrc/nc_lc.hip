@@ -676,12 +676,12 @@ static_assert(2 * kLc0Sets <= kLc0List, "a neutron's ranges of one round fit the
 // the axis (rotateToFrame) and reversed
 template <bool Sample>
 __global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, const double* __restrict__ ekin,
-                                                     const double* __restrict__ dirs, int64_t n, int nb, uint64_t seed,
-                                                     uint32_t stream, double* __restrict__ o1,
+                                                     const double* __restrict__ dirs, int64_t i0, int64_t n, int nb,
+                                                     uint64_t seed, uint32_t stream, double* __restrict__ o1,
                                                      double* __restrict__ oD) {
   __shared__ Lc0Lds S;
   const int tid = (int)threadIdx.x;
-  const int64_t i = (int64_t)blockIdx.x * nb + tid;
+  const int64_t i = i0 + (int64_t)blockIdx.x * nb + tid;
   const bool mine = tid < nb && i < n;
   double E = 0.0, ux = 0.0, uy = 0.0, uz = 0.0, wl = -1.0, c3raw = 0.0, c3 = 0.0, s3 = 0.0;
   double ox = 0.0, oy = 0.0, oz = 0.0;
@@ -760,7 +760,7 @@ __global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, co
       const int per = kLc0Threads / nb < 64 ? kLc0Threads / nb : 64;  // lanes of a neutron (a power of two)
       const int nu = tid / per, q = tid - nu * per;
       const bool on = nu < nb && S.off[nu];
-      const int64_t inu = (int64_t)blockIdx.x * nb + nu;
+      const int64_t inu = i0 + (int64_t)blockIdx.x * nb + nu;
       const double* z = par + 8 * (on ? nu : 0);
       float data[8];
       if (on) {
@@ -852,19 +852,27 @@ int lc0_group(int64_t n) {
 
 }  // namespace
 
+// at most kLc0Launch neutrons a launch: a grid holds fewer than 2^32 work-items,
+// and a workgroup takes four a neutron or more
+constexpr int64_t kLc0Launch = (int64_t)1 << 28;
+static_assert((kLc0Launch / kLc0Neutrons + 1) * kLc0Threads < ((int64_t)1 << 32), "work-items of a launch");
+template <bool Sample>
+static void launch_lc0(const LC0View& L, const SCBView& v, const double* ekin, const double* dirs, int64_t n,
+                       uint64_t seed, uint32_t stream, double* o1, double* oD, hipStream_t st) {
+  const int nb = lc0_group(n);
+  for (int64_t i0 = 0; i0 < n; i0 += kLc0Launch) {
+    const int64_t end = n - i0 < kLc0Launch ? n : i0 + kLc0Launch;
+    hipLaunchKernelGGL(k_lc0<Sample>, dim3((unsigned)((end - i0 + nb - 1) / nb)), dim3(kLc0Threads), 0, st, L, v, ekin,
+                       dirs, i0, end, nb, seed, stream, o1, oD);
+  }
+}
 void launch_lc0_xs(const LC0View& L, const SCBView& v, const double* ekin, const double* dirs, int64_t n, double* out,
                    hipStream_t st) {
-  if (n <= 0) return;
-  const int nb = lc0_group(n);
-  hipLaunchKernelGGL(k_lc0<false>, dim3((unsigned)((n + nb - 1) / nb)), dim3(kLc0Threads), 0, st, L, v, ekin, dirs, n,
-                     nb, (uint64_t)0, (uint32_t)0, out, (double*)nullptr);
+  launch_lc0<false>(L, v, ekin, dirs, n, 0, 0, out, nullptr, st);
 }
 void launch_lc0_sample(const LC0View& L, const SCBView& v, const double* ekin, const double* dirs, int64_t n,
                        uint64_t seed, uint32_t stream, double* oE, double* oD, hipStream_t st) {
-  if (n <= 0) return;
-  const int nb = lc0_group(n);
-  hipLaunchKernelGGL(k_lc0<true>, dim3((unsigned)((n + nb - 1) / nb)), dim3(kLc0Threads), 0, st, L, v, ekin, dirs, n,
-                     nb, seed, stream, oE, oD);
+  launch_lc0<true>(L, v, ekin, dirs, n, seed, stream, oE, oD, st);
 }
 
 void launch_lc_expand(const double* ekin, const double* dirs, int64_t n, int N, const LCView& L, const double2* cs,

@@ -71,3 +71,47 @@ def test_more_plane_sets_than_a_round(core, oracle):
     assert np.max(np.abs(got - want) / want) < 1e-10
     gd = large.sampleScatter(e, d)[1]
     assert np.allclose(np.linalg.norm(gd, axis=1), 1.0, atol=1e-12)
+
+
+def test_more_neutrons_than_a_grid(core):
+    """2^30 neutrons and some: beyond what one launch takes at 256 work-items
+    per 64 neutrons.  All but a few have zero energy (no scattering); the few,
+    around the places where launches meet and at the end, get the values of a
+    small call, and equal neutrons in different launches draw different numbers."""
+    from ncrystal_amd import _capi as C
+    lc = _layered(core, 0.5, 4.0)
+    n, part, k = 2 ** 30 + 65, 2 ** 28, 40
+    e, d = _neutrons(k, 0.6, 2.0, 7)
+    xs = lc.crossSection(e, d)
+    de, dd, o1, o2 = C.DeviceArray(n), C.DeviceArray(3 * n), C.DeviceArray(n), C.DeviceArray(3 * n)
+    put = lambda a, i, x: C.call("ncamd_memcpy_htod", a.ptr + 8 * i, x.ctypes.data, 8 * x.size)
+
+    def get(a, i, m):
+        x = np.empty(m)
+        C.call("ncamd_memcpy_dtoh", x.ctypes.data, a.ptr + 8 * i, 8 * m)
+        return x
+
+    zero = np.zeros(2 ** 25)
+    for i in range(0, n, zero.size):
+        put(de, i, zero[:min(zero.size, n - i)])
+    at = [0, part - k // 2, 2 * part + k, 2 ** 30 - k // 2, n - k]
+    for i in at:
+        put(de, i, e)
+        put(dd, 3 * i, d)
+    lc.dev_crossSection(de.ptr, dd.ptr, n, o1.ptr)
+    C.call("ncamd_stream_sync", None)
+    for i in at:
+        assert np.array_equal(get(o1, i, k), xs)
+    for i in (k, part - k, part + k, 3 * part, 2 ** 30 - k):  # (up to the window after it)
+        assert not get(o1, i, k // 2).any()
+    lc.setRNGState(5, 0)
+    lc.dev_sampleScatter(de.ptr, dd.ptr, n, o1.ptr, o2.ptr)
+    C.call("ncamd_stream_sync", None)
+    got = [get(o2, 3 * i, 3 * k).reshape(-1, 3) for i in at]
+    lc.setRNGState(5, 0)
+    assert np.array_equal(got[0], lc.sampleScatter(e, d)[1])
+    for a in range(len(at)):
+        assert np.array_equal(get(o1, at[a], k), e)
+        assert np.allclose(np.linalg.norm(got[a], axis=1), 1.0, atol=1e-12)
+        for b in range(a):
+            assert np.any(got[a][xs > 0] != got[b][xs > 0])
