@@ -349,7 +349,7 @@ NCD void lc0_neutron(const LC0View& L, double E, double& ux, double& uy, double&
   s3 = sqrt(fabs(1.0 - c3 * c3));
 }
 
-// Layered-crystal kernel: a workgroup takes nb neutrons and works on all
+// Layered-crystal kernel: a workgroup takes 4 to 256 neutrons and works on all
 // their rotation ranges together.
 //
 // A neutron has between none and twice the number of plane sets of ranges
@@ -358,9 +358,12 @@ NCD void lc0_neutron(const LC0View& L, double E, double& ux, double& uy, double&
 // neutron ran at the pace of the longest lane of its wave, with the nested
 // circle integral in line (256 registers, one wave per SIMD, 480 B of scratch
 // per lane): 22 ms for the cross sections of 131072 neutrons and 30 ms for
-// scattering, against 1.09 and 1.31 ms now, bound by the FP64 arithmetic of the
+// scattering, against 1.05 and 1.15 ms now, bound by the FP64 arithmetic of the
 // points (about 210 vector instructions each).  Here
-//  - the ranges are found with one lane per (neutron, 32 plane sets) and
+//  - every lane first looks at one neutron and its first plane sets; neutrons
+//    without a range are done (k_lc0), and where the first sets were all the
+//    sets in reach, the ranges are listed;
+//  - else the ranges are found with one lane per (neutron, 32 plane sets) and
 //    listed in the neutrons' order (bit masks and a prefix sum);
 //  - one lane per range integrates up to row 5 of the Romberg tableau (33
 //    points), where 90 to 97 % are accepted; row 6 of the others takes half a
@@ -374,11 +377,19 @@ NCD void lc0_neutron(const LC0View& L, double E, double& ux, double& uy, double&
 // Neutrons with more ranges than the lists hold together, and more plane sets
 // than a round's masks, are worked on in rounds; only with more than kLc0Sets
 // plane sets does sampling run them again to find its range.
+//
+// The first step is what batches with few or no ranges need, beyond the
+// wavelengths of all sets but one or two: without it 1e6 neutrons of 8 to 20 Aa
+// took 142 us (cross sections) and 349 us (scattering), with it 18 and 19 (one
+// lane per neutron: 51 and 52), of 4.3 to 6 Aa 175 and 589 us, now 63 and 156
+// (70 and 198).  Where such a batch is small (1e3 to 1e5 neutrons, 4.3 Aa and
+// beyond), the steps' latencies leave the cross sections at 7 to 43 us, 1.2 to
+// 1.8 times those of one lane per neutron.
 constexpr int kLc0Threads = 256;
-constexpr int kLc0Neutrons = 64;                  // neutrons of a workgroup at most
+constexpr int kLc0Neutrons = 128;                 // neutrons worked on together at most
 constexpr int kLc0Words = 8;                      // mask words (32 plane sets each) per neutron and round
 constexpr int kLc0Sets = 32 * kLc0Words;
-constexpr int kLc0Units = kLc0Neutrons * kLc0Words;
+constexpr int kLc0Units = 512;                    // mask words of those neutrons at most
 constexpr int kLc0List = 1536;
 constexpr int kLc0Redo = 28;                      // listed ranges redone together: 28 x 9 groups of 4 points
 constexpr int kLc0RedoPts = 33;
@@ -387,14 +398,17 @@ struct Lc0Lds {
   uint64_t mask[kLc0Units];
   double wl[kLc0Neutrons], c3[kLc0Neutrons], s3[kLc0Neutrons];
   double val[kLc0List];
-  double sv[kLc0Redo * kLc0RedoPts];
-  double row[kLc0Redo * 16];
+  double sv[kLc0Redo * (kLc0RedoPts + 16)];  // points of the ranges redone, then their rows (the rotation step takes all)
   int off[kLc0Units + 1];
   uint16_t item[kLc0List];   // neutron << 9 | set of the round << 1 | side
   uint16_t redo[kLc0List];   // ranges not done by their one lane: not accepted at row 6 from the front, slow from the back
-  int nredo, nslow, nact;
+  int nredo, nslow, nact, nwork, nlisted, more;
   uint8_t act[kLc0Redo];
+  uint8_t work[kLc0Threads];   // neutrons of the workgroup that may have ranges
+  uint8_t turn[kLc0Neutrons];  // neutrons of the rotation step
 };
+static_assert(kLc0Redo * (kLc0RedoPts + 16) >= 10 * kLc0Neutrons && kLc0List >= 8 * kLc0Neutrons, "rotation step");
+static_assert(kLc0Neutrons <= 128 && 2 * kLc0Sets <= 512 && kLc0Words <= kLc0Units, "bits of item");
 
 // integrates the ranges listed in S.item[0..n) (plane sets k0 + .. of this
 // round) into S.val; the whole workgroup calls it
@@ -538,7 +552,7 @@ NCD void lc0_values(const LC0View& L, const SCBView& v, Lc0Lds& S, int k0, int n
         const LC0Roi roi = lc0_roi(L, L.sets[k0 + (int)((it >> 1) & 255u)], S.wl[nu], S.c3[nu], S.s3[nu],
                                    (it & 1u) ? -1.0 : 1.0);
         const double len = roi.r1 - roi.r0;
-        double* row = S.row + 16 * tid;
+        double* row = S.sv + kLc0Redo * kLc0RedoPts + 16 * tid;
         bool done = true;
         double x;
         if (roi.kind != 2) {
@@ -579,68 +593,78 @@ NCD void lc0_values(const LC0View& L, const SCBView& v, Lc0Lds& S, int k0, int n
 // (plane set << 1 | side) the first range at which the sum exceeds target, or
 // the last range.  kLc0SumPick, for plane sets that fit one round's masks, does
 // both at once: the sum of a round's neutrons is complete and their values are
-// still in S, so the target is drawn from r and the values walked again.
+// still in S, so the target is drawn (the first number of neutron i's stream) and
+// the values walked again.  listed >= 0: that many ranges are in S.item already, all
+// there are, with S.mask and S.off per neutron.
 enum : int { kLc0Sum, kLc0SumPick, kLc0Find };
 template <int Mode>
-NCD void lc0_pass(const LC0View& L, const SCBView& v, Lc0Lds& S, int nb, bool valid, Rng& r, double target,
-                  double& tot, int64_t& pick) {
+NCD void lc0_pass(const LC0View& L, const SCBView& v, Lc0Lds& S, int nb, int listed, bool valid, uint64_t seed,
+                  uint32_t stream, int64_t i, double target, double& tot, int64_t& pick) {
   const int tid = (int)threadIdx.x;
   bool found = false;
   for (int k0 = 0; k0 < L.nsets; k0 += kLc0Sets) {
     const int nk = L.nsets - k0 < kLc0Sets ? L.nsets - k0 : kLc0Sets;
-    const int nw = (nk + 31) >> 5;
+    const int nw = listed < 0 ? (nk + 31) >> 5 : 1;
     const int units = nb * nw;  // unit u: mask word u % nw of neutron u / nw
-    for (int u = tid; u < units; u += kLc0Threads) {
-      const int nu = u / nw;
-      const int ka = k0 + 32 * (u - nu * nw), kb = ka + 32 < k0 + nk ? ka + 32 : k0 + nk;
-      const double wl = S.wl[nu], c3 = S.c3[nu], s3 = S.s3[nu];
-      uint64_t m = 0;
-      if (wl >= 0.0)
+    if (listed < 0) {
+      for (int u = tid; u < units; u += kLc0Threads) {
+        const int nu = u / nw;
+        const int ka = k0 + 32 * (u - nu * nw), kb = ka + 32 < k0 + nk ? ka + 32 : k0 + nk;
+        const double wl = S.wl[nu], c3 = S.c3[nu], s3 = S.s3[nu];
+        uint64_t m = 0;
         for (int k = ka; k < kb; ++k) {
           const LC0Set ps = L.sets[k];
           if (wl > ps.twodsp) break;
           m |= (uint64_t)lc0_sides(L, ps, wl, c3, s3) << (2 * (k - ka));
         }
-      S.mask[u] = m;
-    }
-    __syncthreads();
-    if (tid < 64) {  // prefix sum of the units' counts
-      const int per = (units + 63) >> 6;
-      int s = 0;
-      for (int u = tid * per; u < (tid + 1) * per && u < units; ++u) s += __popcll(S.mask[u]);
-      int run = s;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(run, o, 64);
-        if (tid >= o) run += y;
-      }
-      int at = run - s;
-      for (int u = tid * per; u < (tid + 1) * per && u < units; ++u) {
-        S.off[u] = at;
-        at += __popcll(S.mask[u]);
-      }
-      if (tid == 63) S.off[units] = run;
-    }
-    __syncthreads();
-    for (int n0 = 0; n0 < nb;) {
-      // neutrons n0 .. n1 - 1: as many as the lists hold (one always fits)
-      const int base = S.off[n0 * nw];
-      int n1 = n0 + 1;
-      while (n1 < nb && S.off[(n1 + 1) * nw] - base <= kLc0List) ++n1;
-      const int n = S.off[n1 * nw] - base;
-      for (int u = n0 * nw + tid; u < n1 * nw; u += kLc0Threads) {
-        const int nu = u / nw;
-        uint64_t m = S.mask[u];
-        for (int p = S.off[u] - base; m; ++p) {
-          const int b = __builtin_ctzll(m);
-          m &= m - 1ull;
-          S.item[p] = (uint16_t)((nu << 9) | (64 * (u - nu * nw) + b));
-        }
+        S.mask[u] = m;
       }
       __syncthreads();
+      if (tid < 64) {  // prefix sum of the units' counts
+        const int per = (units + 63) >> 6;
+        int s = 0;
+        for (int u = tid * per; u < (tid + 1) * per && u < units; ++u) s += __popcll(S.mask[u]);
+        int run = s;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int y = __shfl_up(run, o, 64);
+          if (tid >= o) run += y;
+        }
+        int at = run - s;
+        for (int u = tid * per; u < (tid + 1) * per && u < units; ++u) {
+          S.off[u] = at;
+          at += __popcll(S.mask[u]);
+        }
+        if (tid == 63) S.off[units] = run;
+      }
+      __syncthreads();
+    }
+    for (int n0 = 0; n0 < nb;) {
+      // neutrons n0 .. n1 - 1: as many as the lists hold (one always fits)
+      int base = 0, n1 = nb, n = listed;
+      if (listed < 0) {
+        base = S.off[n0 * nw];
+        if (S.off[units] - base > kLc0List) {
+          n1 = n0 + 1;
+          while (S.off[(n1 + 1) * nw] - base <= kLc0List) ++n1;
+        }
+        n = S.off[n1 * nw] - base;
+        if (n == 0) break;  // none in reach: n1 is nb
+        for (int u = n0 * nw + tid; u < n1 * nw; u += kLc0Threads) {
+          const int nu = u / nw;
+          uint64_t m = S.mask[u];
+          for (int p = S.off[u] - base; m; ++p) {
+            const int b = __builtin_ctzll(m);
+            m &= m - 1ull;
+            S.item[p] = (uint16_t)((nu << 9) | (64 * (u - nu * nw) + b));
+          }
+        }
+        __syncthreads();
+      }
       lc0_values(L, v, S, k0, n);
       if (valid && tid >= n0 && tid < n1) {
-        const int p0 = S.off[tid * nw] - base, e = S.off[(tid + 1) * nw] - base;
+        const int p0 = S.off[tid * nw] - base;
+        const int e = listed < 0 ? S.off[(tid + 1) * nw] - base : p0 + __popcll(S.mask[tid]);
         for (int p = p0; p < e; ++p) {
           tot += S.val[p];
           if (Mode == kLc0Find && !found) {
@@ -649,6 +673,8 @@ NCD void lc0_pass(const LC0View& L, const SCBView& v, Lc0Lds& S, int nb, bool va
           }
         }
         if (Mode == kLc0SumPick && tot > 0.0) {
+          Rng r;
+          r.init(seed, stream, (uint64_t)i);
           target = r.gen() * tot;
           double run = 0.0;
           for (int p = p0; p < e && !found; ++p) {
@@ -661,6 +687,7 @@ NCD void lc0_pass(const LC0View& L, const SCBView& v, Lc0Lds& S, int nb, bool va
       n0 = n1;
       if (n0 < nb) __syncthreads();  // the lists are rewritten
     }
+    if (listed >= 0) break;  // all
     if (k0 + kLc0Sets < L.nsets) __syncthreads();
   }
 }
@@ -673,94 +700,89 @@ static_assert(2 * kLc0Sets <= kLc0List, "a neutron's ranges of one round fit the
 // along the axis; a random sign of sin(phi); the Gaussian-mosaic scattering of
 // the reversed neutron (-s3, 0, -c3) off that normal in the frame of the axis
 // (LCStdFrame::genScat, :755-772), taken to the lab frame by the neutron and
-// the axis (rotateToFrame) and reversed
+// the axis (rotateToFrame) and reversed.  For the workgroup's neutrons base +
+// S.work[r0 .. r0 + nb); listed: see lc0_pass.
 template <bool Sample>
-__global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, const double* __restrict__ ekin,
-                                                     const double* __restrict__ dirs, int64_t i0, int64_t n, int nb,
-                                                     uint64_t seed, uint32_t stream, double* __restrict__ o1,
-                                                     double* __restrict__ oD) {
-  __shared__ Lc0Lds S;
+NCD void lc0_round(const LC0View& L, const SCBView& v, Lc0Lds& S, const double* __restrict__ ekin,
+                   const double* __restrict__ dirs, int64_t base, int r0, int nb, int listed,
+                   uint64_t seed, uint32_t stream, double* __restrict__ o1, double* __restrict__ oD) {
   const int tid = (int)threadIdx.x;
-  const int64_t i = i0 + (int64_t)blockIdx.x * nb + tid;
-  const bool mine = tid < nb && i < n;
-  double E = 0.0, ux = 0.0, uy = 0.0, uz = 0.0, wl = -1.0, c3raw = 0.0, c3 = 0.0, s3 = 0.0;
-  double ox = 0.0, oy = 0.0, oz = 0.0;
-  if (mine) {
-    E = ekin[i];
-    ox = ux = dirs[3 * i]; oy = uy = dirs[3 * i + 1]; oz = uz = dirs[3 * i + 2];
-    if (E > 0.0) lc0_neutron(L, E, ux, uy, uz, wl, c3raw, c3, s3);
+  const bool valid = tid < nb;
+  const int64_t i = base + (valid ? S.work[r0 + tid] : 0);
+  // (nothing of a neutron but its place stays in registers through the
+  // integrals: it is read again)
+  if (listed < 0) {
+    if (valid) {
+      double ux = dirs[3 * i], uy = dirs[3 * i + 1], uz = dirs[3 * i + 2], c3raw;
+      lc0_neutron(L, ekin[i], ux, uy, uz, S.wl[tid], c3raw, S.c3[tid], S.s3[tid]);
+    }
+    __syncthreads();
   }
-  if (tid < nb) {
-    S.wl[tid] = wl;  // -1: nothing to do
-    S.c3[tid] = c3;
-    S.s3[tid] = s3;
-  }
-  __syncthreads();
-  const bool valid = mine && E > 0.0;
   double tot = 0.0;
   int64_t pick = 0;
-  Rng r;
   if constexpr (!Sample) {
-    lc0_pass<kLc0Sum>(L, v, S, nb, valid, r, -1.0, tot, pick);
-    if (mine) o1[i] = L.xsfact * tot;
+    lc0_pass<kLc0Sum>(L, v, S, nb, listed, valid, seed, stream, i, -1.0, tot, pick);
+    if (valid) o1[i] = L.xsfact * tot;
   } else {
-    if (valid) r.init(seed, stream, (uint64_t)i);
     if (L.nsets <= kLc0Sets) {
-      lc0_pass<kLc0SumPick>(L, v, S, nb, valid, r, -1.0, tot, pick);
+      lc0_pass<kLc0SumPick>(L, v, S, nb, listed, valid, seed, stream, i, -1.0, tot, pick);
     } else {
-      lc0_pass<kLc0Sum>(L, v, S, nb, valid, r, -1.0, tot, pick);
+      lc0_pass<kLc0Sum>(L, v, S, nb, listed, valid, seed, stream, i, -1.0, tot, pick);
       double target = 0.0, run = 0.0;
-      if (valid && tot > 0.0) target = r.gen() * tot;
+      if (valid && tot > 0.0) {
+        Rng r;
+        r.init(seed, stream, (uint64_t)i);
+        target = r.gen() * tot;
+      }
       __syncthreads();
-      lc0_pass<kLc0Find>(L, v, S, nb, valid && tot > 0.0, r, target, run, pick);
+      lc0_pass<kLc0Find>(L, v, S, nb, listed, valid && tot > 0.0, seed, stream, i, target, run, pick);
     }
     const bool scat = valid && tot > 0.0;
-    if (mine) o1[i] = E;
     // The rotation in the picked range, with the workgroup's lanes shared out
-    // among its neutrons: the envelope's 9 points, then `per` tries at a time
-    // (each try takes the next three numbers of the neutron's stream, so a
-    // lane can draw try t without the ones before; the first accepted one
-    // counts).  One lane per neutron made a wave wait for its longest
-    // rejection, 0.8 ms more for 131072 neutrons than the ranges' own 1.05 ms;
-    // shared out it is 0.2 ms.
+    // among the neutrons that need one: the envelope's 9 points, then `per`
+    // tries at a time (each try takes the next three numbers of the neutron's
+    // stream, so a lane can draw try t without the ones before; the first
+    // accepted one counts).  One lane per neutron made a wave wait for its
+    // longest rejection, 0.8 ms more for 131072 neutrons than the ranges' own
+    // 1.05 ms; shared out it is 0.2 ms.
+    if (tid == 0) S.nact = 0;
     __syncthreads();  // S.val and S.sv change their use
     LC0Set ps{};
     double sg = 1.0;
-    int kind = 0;
-    double* par = S.val;                   // [nb][8] k1, k0, r0, length, sinpt, cospt, Q, fixed
-    double* env = S.sv;                    // [nb][9]
-    double* got = S.sv + 9 * kLc0Neutrons; // [nb] cos(phi); then the number of tries
-    if (tid < nb) {
-      S.off[tid] = 0;
-      if (scat) {
-        ps = L.sets[pick >> 1];
-        sg = (pick & 1) ? -1.0 : 1.0;
-        const LC0Roi roi = lc0_roi(L, ps, wl, c3, s3, sg);
-        kind = roi.kind;
-        if (kind == 2) {
-          const LC0Raw raw = lc0_raw_setup(wl, ps.inv2d, ps.fsq);
-          double* q = par + 8 * tid;
-          q[0] = roi.k1; q[1] = roi.k0; q[2] = roi.r0; q[3] = roi.r1 - roi.r0;
-          q[4] = raw.sinpt; q[5] = raw.cospt; q[6] = raw.Q; q[7] = raw.fixed;
-          S.off[tid] = 1;
-        }
+    int kind = 0, mine = 0;                // mine: place among those neutrons
+    double* par = S.val;                   // [nact][8] k1, k0, r0, length, sinpt, cospt, Q, fixed
+    double* env = S.sv;                    // [nact][9]
+    double* got = S.sv + 9 * kLc0Neutrons; // [nact] cos(phi), with the number of tries in S.off
+    if (scat) {
+      ps = L.sets[pick >> 1];
+      sg = (pick & 1) ? -1.0 : 1.0;
+      const LC0Roi roi = lc0_roi(L, ps, S.wl[tid], S.c3[tid], S.s3[tid], sg);
+      kind = roi.kind;
+      if (kind == 2) {
+        mine = atomicAdd(&S.nact, 1);
+        S.turn[mine] = (uint8_t)tid;
+        const LC0Raw raw = lc0_raw_setup(S.wl[tid], ps.inv2d, ps.fsq);
+        double* q = par + 8 * mine;
+        q[0] = roi.k1; q[1] = roi.k0; q[2] = roi.r0; q[3] = roi.r1 - roi.r0;
+        q[4] = raw.sinpt; q[5] = raw.cospt; q[6] = raw.Q; q[7] = raw.fixed;
       }
     }
     __syncthreads();
+    const int ns = S.nact;
     bool dummy = false;
-    for (int q = tid; q < 9 * nb; q += kLc0Threads) {
+    for (int q = tid; q < 9 * ns; q += kLc0Threads) {
       const int nu = q / 9, j = q - 9 * nu;
-      if (!S.off[nu]) continue;
       const double* z = par + 8 * nu;
       const LC0Raw raw{z[4], z[5], z[6], z[7]};
       env[q] = lc0_raw<true>(v, raw, z[0] * lc0_cos(z[2] + j * (z[3] * 0.125)) + z[1], dummy);
     }
     __syncthreads();
-    {
-      const int per = kLc0Threads / nb < 64 ? kLc0Threads / nb : 64;  // lanes of a neutron (a power of two)
+    if (ns > 0) {
+      int per = 64;  // lanes of a neutron (a power of two)
+      while (per * ns > kLc0Threads) per >>= 1;
       const int nu = tid / per, q = tid - nu * per;
-      const bool on = nu < nb && S.off[nu];
-      const int64_t inu = i0 + (int64_t)blockIdx.x * nb + nu;
+      const bool on = nu < ns;
+      const int64_t inu = base + S.work[r0 + S.turn[on ? nu : 0]];
       const double* z = par + 8 * (on ? nu : 0);
       float data[8];
       if (on) {
@@ -807,34 +829,35 @@ __global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, co
       }
     }
     __syncthreads();
-    if (scat) {
-      const V3 indir_std{-s3, 0.0, -c3};
-      V3 normal{0.0, 0.0, sg};
-      if (kind != 0) {
-        double cosphi;
-        if (kind == 1) {
-          cosphi = cos(r.gen() * kPi);
-        } else {
-          cosphi = got[tid];
-          const int d = 1 + 3 * (S.off[tid] - 1);  // numbers drawn so far
-          r.c0 = (uint32_t)d >> 1;
-          r.nleft = 0;
-          if (d & 1) (void)r.gen();
+    if (valid) {
+      const double E = ekin[i];
+      double ox = dirs[3 * i], oy = dirs[3 * i + 1], oz = dirs[3 * i + 2];
+      if (scat) {
+        double ux = ox, uy = oy, uz = oz, wl, c3raw, c3, s3;
+        lc0_neutron(L, E, ux, uy, uz, wl, c3raw, c3, s3);
+        const V3 indir_std{-s3, 0.0, -c3};
+        V3 normal{0.0, 0.0, sg};
+        const int d = kind == 2 ? 1 + 3 * (S.off[mine] - 1) : 1;  // numbers drawn so far
+        Rng r;
+        r.init(seed, stream, (uint64_t)i);
+        r.c0 = (uint32_t)d >> 1;
+        if (d & 1) (void)r.gen();
+        if (kind != 0) {
+          const double cosphi = kind == 1 ? cos(r.gen() * kPi) : got[mine];
+          const double sgn = r.gen() < 0.5 ? 1.0 : -1.0;
+          const double sinphi = sgn * sqrt(dmax(0.0, 1.0 - cosphi * cosphi));
+          const double ns1 = sg * ps.s1;
+          normal = V3{ns1 * cosphi, ns1 * sinphi, sg * ps.c1};
         }
-        const double sgn = r.gen() < 0.5 ? 1.0 : -1.0;
-        const double sinphi = sgn * sqrt(dmax(0.0, 1.0 - cosphi * cosphi));
-        const double ns1 = sg * ps.s1;
-        normal = V3{ns1 * cosphi, ns1 * sinphi, sg * ps.c1};
+        const V3 w = gm_genscat(v, r, normal, gm_round(ps.inv2d), wl, indir_std);
+        const double isg = c3raw >= 0.0 ? 1.0 : -1.0;
+        const V3 a{ux, uy, uz}, b{L.ax * isg, L.ay * isg, L.az * isg};
+        const V3 o = rotate_to_frame(s3, c3, a, b, w, r);
+        ox = -o.x;
+        oy = -o.y;
+        oz = -o.z;
       }
-      const V3 w = gm_genscat(v, r, normal, gm_round(ps.inv2d), wl, indir_std);
-      const double isg = c3raw >= 0.0 ? 1.0 : -1.0;
-      const V3 a{ux, uy, uz}, b{L.ax * isg, L.ay * isg, L.az * isg};
-      const V3 o = rotate_to_frame(s3, c3, a, b, w, r);
-      ox = -o.x;
-      oy = -o.y;
-      oz = -o.z;
-    }
-    if (mine) {
+      o1[i] = E;
       oD[3 * i] = ox;
       oD[3 * i + 1] = oy;
       oD[3 * i + 2] = oz;
@@ -842,20 +865,112 @@ __global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, co
   }
 }
 
-// neutrons of a workgroup: 64 where that gives every CU two workgroups,
-// fewer for small batches, so that a batch still spreads over the chip
+// the ranges of the first plane sets (two bits each, lc0_sides); all: there are
+// no others in reach
+constexpr int kLc0Look = 4;
+NCD unsigned lc0_look(const LC0View& L, double wl, double c3, double s3, bool& all) {
+  unsigned m = 0;
+  all = true;
+  for (int k = 0; k < kLc0Look && k < L.nsets; ++k) {
+    const LC0Set ps = L.sets[k];
+    if (wl > ps.twodsp) return m;
+    m |= lc0_sides(L, ps, wl, c3, s3) << (2 * k);
+  }
+  all = L.nsets <= kLc0Look;
+  return m;
+}
+static_assert(2 * kLc0Look * kLc0Neutrons <= kLc0List, "listed ranges");
+
+// A workgroup's `per` neutrons, one per lane first: those that have no range
+// (all beyond the first plane sets' wavelengths, and there most others: 0.5-7
+// Aa about half of a batch) are done at once, the others in rounds.
+template <bool Sample>
+__global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, const double* __restrict__ ekin,
+                                                     const double* __restrict__ dirs, int64_t i0, int64_t n, int per,
+                                                     uint64_t seed, uint32_t stream, double* __restrict__ o1,
+                                                     double* __restrict__ oD) {
+  __shared__ Lc0Lds S;
+  const int tid = (int)threadIdx.x;
+  const int64_t base = i0 + (int64_t)blockIdx.x * per;
+  if (tid == 0) { S.nwork = 0; S.nlisted = 0; S.more = 0; }
+  __syncthreads();
+  {
+    const int64_t i = base + tid;
+    const bool mine = tid < per && i < n;
+    bool work = false, all = true;
+    unsigned m = 0;
+    double wl = 0.0, c3 = 0.0, s3 = 0.0;
+    double E = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
+    if (mine) {
+      E = ekin[i];
+      dx = dirs[3 * i]; dy = dirs[3 * i + 1]; dz = dirs[3 * i + 2];
+      if (E > 0.0) {
+        double ux = dx, uy = dy, uz = dz, c3raw;
+        lc0_neutron(L, E, ux, uy, uz, wl, c3raw, c3, s3);
+        m = lc0_look(L, wl, c3, s3, all);
+        work = m || !all;
+      }
+    }
+    const uint64_t B = __ballot(work);
+    int at = 0;
+    if ((tid & 63) == 0 && B) at = atomicAdd(&S.nwork, __popcll(B));
+    at = __builtin_amdgcn_readfirstlane(at) + __popcll(B & ((1ull << (tid & 63)) - 1ull));
+    if (work) S.work[at] = (uint8_t)tid;
+    if (__any(!all)) {
+      S.more = 1;
+    } else if (work && at < kLc0Neutrons) {
+      // listed here already, which counts if it holds for the whole workgroup
+      S.wl[at] = wl;
+      S.c3[at] = c3;
+      S.s3[at] = s3;
+      S.mask[at] = m;
+      int p = atomicAdd(&S.nlisted, __popc(m));
+      S.off[at] = p;
+      for (unsigned q = m; q; q &= q - 1u) S.item[p++] = (uint16_t)((at << 9) | __builtin_ctz(q));
+    }
+    if (mine && !work) {
+      if constexpr (Sample) {
+        o1[i] = E;
+        oD[3 * i] = dx;
+        oD[3 * i + 1] = dy;
+        oD[3 * i + 2] = dz;
+      } else {
+        o1[i] = 0.0;
+      }
+    }
+  }
+  __syncthreads();
+  const int nwork = S.nwork;
+  if (nwork == 0) return;
+  const bool ready = !S.more && nwork <= kLc0Neutrons;
+  const int nw = ready ? 1 : (L.nsets < kLc0Sets ? (L.nsets + 31) >> 5 : kLc0Words);
+  const int most = kLc0Units / nw < kLc0Neutrons ? kLc0Units / nw : kLc0Neutrons;
+  const int rounds = (nwork + most - 1) / most, nb = (nwork + rounds - 1) / rounds;
+  for (int r0 = 0; r0 < nwork; r0 += nb) {
+    if (r0) __syncthreads();
+    lc0_round<Sample>(L, v, S, ekin, dirs, base, r0, nwork - r0 < nb ? nwork - r0 : nb, ready ? S.nlisted : -1, seed, stream,
+                      o1, oD);
+  }
+}
+
+// neutrons of a workgroup: 64 where that gives every CU two workgroups, fewer
+// for small batches, so that a batch still spreads over the chip; 128 and 256
+// where that leaves the chip filled 2 and 4 times.  Many share the steps' latencies
+// where few have ranges (3e5 neutrons, 4.3-6 Aa, cross sections: 60 us with 64, 25
+// with 128, 21 with 256), but even out worse where most have (0.5-7 Aa: 131072
+// neutrons 2.20 ms with 64 and 2.30 with 128 for both calls, 3e5 1.96 with 64, 2.05
+// with 128 and 2.54 with 256, 1e6 5.59 with 128 and 6.08 with 256).
 int lc0_group(int64_t n) {
-  int nb = kLc0Neutrons;
-  while (nb > 4 && n < (int64_t)512 * nb) nb >>= 1;
+  int nb = kLc0Threads;
+  while (nb > 4 && n < (int64_t)(nb > 128 ? 4096 : (nb > 64 ? 2048 : 512)) * nb) nb >>= 1;
   return nb;
 }
 
 }  // namespace
 
-// at most kLc0Launch neutrons a launch: a grid holds fewer than 2^32 work-items,
-// and a workgroup takes four a neutron or more
+// at most kLc0Launch neutrons a launch: a grid holds fewer than 2^32 work-items
 constexpr int64_t kLc0Launch = (int64_t)1 << 28;
-static_assert((kLc0Launch / kLc0Neutrons + 1) * kLc0Threads < ((int64_t)1 << 32), "work-items of a launch");
+static_assert((kLc0Launch / kLc0Threads + 1) * kLc0Threads < ((int64_t)1 << 32), "work-items of a launch");
 template <bool Sample>
 static void launch_lc0(const LC0View& L, const SCBView& v, const double* ekin, const double* dirs, int64_t n,
                        uint64_t seed, uint32_t stream, double* o1, double* oD, hipStream_t st) {

@@ -53,6 +53,29 @@ def test_batch_size_changes_nothing(core, lo, hi, mosaic):
         assert np.array_equal(lc.sampleScatter(e[:m], d[:m])[1], od[:m])
 
 
+# workgroups of 128 and 256 neutrons: all beyond the last wavelength, around it,
+# with the first plane set alone, with a few, and every kind mixed
+@pytest.mark.parametrize("n", [262147, 1048581])
+@pytest.mark.parametrize("lo,hi", [(6.9, 9.0), (6.6, 6.8), (4.3, 6.0), (3.0, 4.0), (1.0, 9.0)])
+def test_sparse_batches(core, n, lo, hi):
+    lc = _layered(core, 0.5, 4.0)
+    e, d = _neutrons(n, lo, hi, 11)
+    d[:64] = [0.0, 0.0, 1.0]  # along the axis
+    e[100:110] = [0.0, -1.0, np.inf, np.nan, 1e-9, 1e3, 0.0, np.nan, -0.0, 1e-300]
+    xs = lc.crossSection(e, d)
+    lc.setRNGState(17, 0)
+    oe, od = lc.sampleScatter(e, d)
+    assert np.array_equal(oe, e, equal_nan=True)
+    none = ~(e > WL2EKIN / 6.8 ** 2)  # the largest 2d is 6.71 Aa
+    assert np.all(xs[none] == 0.0) and np.array_equal(od[none], d[none])
+    for m in (130, 4999, 40000):  # 4, 8 and 64 neutrons per workgroup
+        assert np.array_equal(lc.crossSection(e[:m], d[:m]), xs[:m], equal_nan=True)
+        lc.setRNGState(17, 0)
+        assert np.array_equal(lc.sampleScatter(e[:m], d[:m])[1], od[:m], equal_nan=True)
+    k = n - 4000  # the batch's end
+    assert np.array_equal(lc.crossSection(e[k:], d[k:]), xs[k:], equal_nan=True)
+
+
 def test_more_plane_sets_than_a_round(core, oracle):
     """dcutoff 0.2 Aa gives the crystal over 256 plane sets; neutrons that
     reach only those down to 0.5 Aa see the same crystal as without the rest
