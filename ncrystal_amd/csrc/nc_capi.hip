@@ -1824,7 +1824,7 @@ Proc* create_scb(double v0n, int64_t nfam, const double* dsp, const double* fsq,
   const double T = trunc * (1.0 + 1e-6);
   v.band_hT2 = (float)(0.5 * T * T);
   v.band_T2 = (float)(T * T);
-  v.band_T2c = (float)(T * T * (1.0 + 1e-6));
+  v.band_T2c = (float)(T * T * (1.0 + 1e-6) + 2.0 * T * kScbBandEps + (double)kScbBandEps * kScbBandEps);
   {
     const double w = maxd * 2.0, w2 = w * w;
     v.threshold = w2 ? kWl2Ekin / w2 : __builtin_huge_val();

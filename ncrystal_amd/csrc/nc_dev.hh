@@ -177,6 +177,13 @@ NCD unsigned long long block_append2(unsigned long long* counter, int stride, bo
   return pos;
 }
 
+// LDS that lanes of one wave exchange through: what they wrote is there for the
+// others (they run in step; this holds back the compiler)
+NCD void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---------------------------------------------------------------------------
 // Position of this lane's entry in a queue that the active lanes with `want`
 // append to: one atomic per wave (the first such lane adds their count) and

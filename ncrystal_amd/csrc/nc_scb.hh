@@ -23,8 +23,7 @@
 // wave-uniform (the records are scalar loads shared by the 64 lanes) and a
 // lane whose families are exhausted is masked.  The rare backscattering
 // geometry that needs the Romberg circle integral goes through a queue to a
-// second kernel, a wave per neutron (scb_candidate<true>), so the main kernel
-// carries no Romberg state.
+// second kernel (nc_scb.hip), so the main kernel carries no Romberg state.
 #pragma once
 #include "nc_dev.hh"
 #include "nc_math.hh"
@@ -53,7 +52,7 @@ struct SCBView {
   const double2* __restrict__ nfx;      // [nnormals + kScbPad] (family xsf, family index) of each demi-normal
   double threshold;                     // ekin below which nothing reflects
   double cta, k1, k2, numacc;           // GaussOnSphere: cos(truncation), fast-path bounds, Romberg accuracy
-  // pre-filter: T^2/2, T^2 and T^2 (1 + 1e-6) with T the truncation angle + 1e-6 of it
+  // pre-filter: T^2/2, T^2 and T^2 (1 + 1e-6) + 2 T eps + eps^2 with T the truncation angle + 1e-6 of it
   float band_hT2, band_T2, band_T2c;
   SplineView lt_evalcosx, lt_sofcosd;
 };
@@ -117,6 +116,10 @@ struct CSGrid {
   }
 };
 
+NCD double readlane_d(double x, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
 struct GCI {
   double sasg, cacg, acc;
 };
@@ -133,63 +136,104 @@ NCD double gci_sum(const SCBView& v, const GCI& g, unsigned n, double off, doubl
   do { sum += gci_f(v, g, gr.c); } while (gr.step());
   return sum;
 }
-// Romberg integration of the mosaic density along the circle, t in [a,b].
-// The 17 points of the first five rows are added to their groups (ends, eighth
+// The same with the points of up to 64 on the lanes of the wave (all 64 call it
+// with the same arguments), added in the same order
+NCD double gci_sum_wave(const SCBView& v, const GCI& g, unsigned n, double off, double delta) {
+  if (n > 64) return gci_sum(v, g, n, off, delta);
+  const int lane = (int)__lane_id();
+  CSGrid gr;
+  gr.init(n, off, delta);
+#pragma nounroll
+  for (int i = 0; i + 1 < (int)n; ++i)
+    if (i < lane) gr.step();
+  const double f = gci_f(v, g, gr.c);
+  double sum = 0.0;
+  for (int i = 0; i < (int)n; ++i) sum += readlane_d(f, i);
+  return sum;
+}
+// The 17 points of the first five rows, added to their groups: ends, eighth
 // point, quarters, eighths, sixteenths; pairwise, in the order of the
-// reference's expressions) as they come: an array of them would hold 34
-// registers in every kernel that can meet this integral.
+// reference's expressions
+struct GCIRows {
+  double end, mid, q, e, s;
+};
+// one lane: added as they come, an array of them would hold 34 registers in
+// every kernel that can meet this integral
+NCD GCIRows gci_rows(const SCBView& v, const GCI& g, double a, double h) {
+  GCIRows o{0.0, 0.0, 0.0, 0.0, 0.0};
+  CSGrid gr;
+  gr.init(17, a, h * 0.0625);
+  double x0 = 0.0, e0 = 0.0;
+#pragma nounroll
+  for (int k = 0; k < 4; ++k) {  // points 4k .. 4k+3
+    const double p = gci_f(v, g, gr.c);
+    if (k == 0) o.end = p;
+    else if (k == 2) o.mid = p;
+    else o.q = k == 1 ? p : o.q + p;
+    gr.step();
+    double x = gci_f(v, g, gr.c);
+    gr.step();
+    double e = gci_f(v, g, gr.c);
+    gr.step();
+    x += gci_f(v, g, gr.c);
+    gr.step();
+    if (k & 1) {
+      x = x0 + x;
+      e = e0 + e;
+      o.s = k == 1 ? x : o.s + x;
+      o.e = k == 1 ? e : o.e + e;
+    }
+    x0 = x;
+    e0 = e;
+  }
+  o.end += gci_f(v, g, gr.c);  // 16
+  return o;
+}
+// a wave: a point per lane
+NCD GCIRows gci_rows_wave(const SCBView& v, const GCI& g, double a, double h) {
+  const int lane = (int)__lane_id();
+  CSGrid gr;
+  gr.init(17, a, h * 0.0625);
+#pragma nounroll
+  for (int i = 0; i < 16; ++i)
+    if (i < lane) gr.step();
+  const double f = gci_f(v, g, gr.c);
+  const auto p = [f](int i) { return readlane_d(f, i); };
+  GCIRows o;
+  o.end = p(0) + p(16);
+  o.mid = p(8);
+  o.q = p(4) + p(12);
+  o.e = (p(2) + p(6)) + (p(10) + p(14));
+  o.s = ((p(1) + p(3)) + (p(5) + p(7))) + ((p(9) + p(11)) + (p(13) + p(15)));
+  return o;
+}
+// Romberg integration of the mosaic density along the circle, t in [a,b], by a
+// lane or by a wave (all lanes with the same arguments)
+template <bool Wave>
 NCD double gci_integrate(const SCBView& v, const GCI& g, double a, double b) {
   double h = (b - a);
-  double s_end = 0.0, s_mid = 0.0, s_q = 0.0, s_e = 0.0, s_s = 0.0;
-  {
-    CSGrid gr;
-    gr.init(17, a, h * 0.0625);
-    double x0 = 0.0, e0 = 0.0;
-#pragma nounroll
-    for (int k = 0; k < 4; ++k) {  // points 4k .. 4k+3
-      const double p = gci_f(v, g, gr.c);
-      if (k == 0) s_end = p;
-      else if (k == 2) s_mid = p;
-      else s_q = k == 1 ? p : s_q + p;
-      gr.step();
-      double x = gci_f(v, g, gr.c);
-      gr.step();
-      double e = gci_f(v, g, gr.c);
-      gr.step();
-      x += gci_f(v, g, gr.c);
-      gr.step();
-      if (k & 1) {
-        x = x0 + x;
-        e = e0 + e;
-        s_s = k == 1 ? x : s_s + x;
-        s_e = k == 1 ? e : s_e + e;
-      }
-      x0 = x;
-      e0 = e;
-    }
-    s_end += gci_f(v, g, gr.c);  // 16
-  }
+  const GCIRows p = Wave ? gci_rows_wave(v, g, a, h) : gci_rows(v, g, a, h);
   h *= 0.5;
-  const double R00 = s_end * h;
-  const double R10 = h * s_mid + 0.5 * R00;
+  const double R00 = p.end * h;
+  const double R10 = h * p.mid + 0.5 * R00;
   const double R11 = (4. / 3.) * R10 + (-1. / 3.) * R00;
   h *= 0.5;
-  const double R20 = h * s_q + 0.5 * R10;
+  const double R20 = h * p.q + 0.5 * R10;
   const double R21 = (4. / 3.) * R20 + (-1. / 3.) * R10;
   const double R22 = (16. / 15.) * R21 + (-1. / 15.) * R11;
   h *= 0.5;
-  const double R30 = h * s_e + 0.5 * R20;
+  const double R30 = h * p.e + 0.5 * R20;
   const double R31 = (4. / 3.) * R30 + (-1. / 3.) * R20;
   const double R32 = (16. / 15.) * R31 + (-1. / 15.) * R21;
   const double R33 = (64. / 63.) * R32 + (-1. / 63.) * R22;
   h *= 0.5;
-  const double R40 = h * s_s + 0.5 * R30;
+  const double R40 = h * p.s + 0.5 * R30;
   const double R41 = (4. / 3.) * R40 + (-1. / 3.) * R30;
   const double R42 = (16. / 15.) * R41 + (-1. / 15.) * R31;
   const double R43 = (64. / 63.) * R42 + (-1. / 63.) * R32;
   const double R44 = (256. / 255.) * R43 + (-1. / 255.) * R33;
   if (gci_accept(g, 4, R33, R44)) return R44;
-  const double c5 = gci_sum(v, g, 16, a + h * 0.5, h);
+  const double c5 = Wave ? gci_sum_wave(v, g, 16, a + h * 0.5, h) : gci_sum(v, g, 16, a + h * 0.5, h);
   h *= 0.5;
   const double R50 = h * c5 + 0.5 * R40;
   const double R51 = (4. / 3.) * R50 + (-1. / 3.) * R40;
@@ -208,7 +252,7 @@ NCD double gci_integrate(const SCBView& v, const GCI& g, double a, double b) {
     const double hh = h;
     h *= 0.5;
     nj *= 2;
-    const double cc = gci_sum(v, g, nj, a + h, hh);
+    const double cc = Wave ? gci_sum_wave(v, g, nj, a + h, hh) : gci_sum(v, g, nj, a + h, hh);
     double* row_prev = rows[ip];
     double* row = rows[ip ^ 1];
     row[0] = h * cc + 0.5 * row_prev[0];
@@ -223,6 +267,7 @@ NCD double gci_integrate(const SCBView& v, const GCI& g, double a, double b) {
   return rows[ip][maxlevel - 1];
 }
 
+template <bool Wave = false>
 NCD double gos_circle_slow(const SCBView& v, double cg, double sg, double ca, double sa) {
   const double sasg = sa * sg;
   const double cacg = ca * cg;
@@ -242,7 +287,7 @@ NCD double gos_circle_slow(const SCBView& v, double cg, double sg, double ca, do
     }
   }
   GCI g{sasg, cacg, intacc};
-  return 2.0 * sa * gci_integrate(v, g, 0.0, tmax);
+  return 2.0 * sa * gci_integrate<Wave>(v, g, 0.0, tmax);
 }
 
 // true if the fast spline evaluation applies (NCGaussOnSphere.hh:194-211)
@@ -412,16 +457,21 @@ NCD float readlane_f(float x, int l) { return __int_as_float(__builtin_amdgcn_re
 // not reflect (NCSCBragg.cc:263-300 with GaussMos::calcCrossSections).  The
 // reference evaluates Q and cos(theta) lazily once per family; both depend
 // on the family alone (sin(theta) = w / 2d), so evaluating them per
-// demi-normal gives the same values.  Returns false, without AllowSlow, if a
-// side needs the Romberg circle integral.
+// demi-normal gives the same values.  Returns false, without Defer, if a side
+// needs the Romberg circle integral; with it such sides are left in slow, with
+// what the integral takes.
 //
 // A demi-normal usually reflects on one side only, and lanes of a wave
 // differ in which: the sides that pass the cone test are evaluated by one
 // loop, so that a wave runs the circle integral once per candidate rather
 // than once per side.
-template <bool AllowSlow>
+struct ScbSlow {
+  unsigned sides;
+  double dot, sinpt, cospt, Q;
+};
+template <bool Defer>
 NCD bool scb_candidate(const SCBView& v, const double4& r, double xsf, double w, double wl3, double ux, double uy,
-                       double uz, double& xs0, double& xs1) {
+                       double uz, double& xs0, double& xs1, ScbSlow* slow = nullptr) {
   xs0 = 0.0;
   xs1 = 0.0;
   const double cta = v.cta;
@@ -453,13 +503,28 @@ NCD bool scb_candidate(const SCBView& v, const double4& r, double xsf, double w,
     const double sc2 = sqrt(1.0 - cc * cc);
     double ci;
     if (!gos_circle_fast_ok(v, cc, sc2, sinpt, cospt, ci)) {
-      if constexpr (AllowSlow) ci = gos_circle_slow(v, cc, sc2, sinpt, cospt);
-      else return false;
+      if constexpr (!Defer) return false;
+      slow->sides |= 1u << side;
+      slow->dot = dot; slow->sinpt = sinpt; slow->cospt = cospt; slow->Q = Q;
+      continue;
     }
     if (side == 0) xs0 = Q * ci;
     else xs1 = Q * ci;
   }
   return true;
+}
+
+// the deferred sides, a lane its own
+NCD void scb_slow_sides(const SCBView& v, ScbSlow& slow, double& xs0, double& xs1) {
+#pragma nounroll
+  while (slow.sides) {
+    const int side = __builtin_ctz(slow.sides);
+    slow.sides &= slow.sides - 1u;
+    const double cc = dclamp(side == 0 ? slow.dot : -slow.dot, -1.0, 1.0);
+    const double ci = gos_circle_slow(v, cc, sqrt(1.0 - cc * cc), slow.sinpt, slow.cospt);
+    if (side == 0) xs0 = slow.Q * ci;
+    else xs1 = slow.Q * ci;
+  }
 }
 
 // Candidate lists: a wave keeps, per lane, the demi-normals that passed the
@@ -496,7 +561,7 @@ struct ScbLane {
 // order and accumulates them; all lanes of the wave call this together.
 // Select=false: count and cumulative total.  Select=true: stop at the
 // contribution picked by pickRandIdxByWeight for (n_select, target).
-template <bool Select>
+template <bool Select, bool AllowSlow>
 NCD void scb_eval_list(const SCBView& v, ScbLane& L, ScbAcc& a, bool& alive, const uint16_t* __restrict__ list,
                        int base, int n, double w, double wl3, int n_select, double target) {
   const int lane = (int)__lane_id();
@@ -513,7 +578,11 @@ NCD void scb_eval_list(const SCBView& v, ScbLane& L, ScbAcc& a, bool& alive, con
       a.xssum = 0.0;
     }
     double xs2[2];
-    if (!scb_candidate<false>(v, r, fx.x, w, wl3, L.u.x, L.u.y, L.u.z, xs2[0], xs2[1])) {
+    if constexpr (AllowSlow) {
+      ScbSlow slow{0u, 0.0, 0.0, 0.0, 0.0};
+      scb_candidate<true>(v, r, fx.x, w, wl3, L.u.x, L.u.y, L.u.z, xs2[0], xs2[1], &slow);
+      scb_slow_sides(v, slow, xs2[0], xs2[1]);
+    } else if (!scb_candidate<false>(v, r, fx.x, w, wl3, L.u.x, L.u.y, L.u.z, xs2[0], xs2[1])) {
       L.slow = true;
       alive = false;
       continue;
@@ -545,8 +614,8 @@ NCD void scb_eval_list(const SCBView& v, ScbLane& L, ScbAcc& a, bool& alive, con
 //   |sin(phi) - sin(theta)| = 2 sin(|phi - theta| / 2) cos((phi + theta) / 2)
 //                           < T cos(theta - T/2) <= T cos(theta) + T^2/2 sin(theta)
 // (for theta < T/2 the last form is above T).  kScbBandEps (FP32 normals and
-// products: below 1e-6) and 1e-6 under the root of cos(theta) cover the
-// rounding.  The test against T alone let 1.7 times as many through (cos(theta)
+// products: below 1e-6), taken in under the root of cos(theta) as 2 T eps + eps^2,
+// and 1e-6 of T^2 there cover the rounding.  The test against T alone let 1.7 times as many through (cos(theta)
 // averages 3 pi / 16 over the planes in reach, their density growing as
 // 1/d^4), each a step of the FP64 evaluation for the whole wave: cross sections
 // of 2e6 neutrons, 1 to 6 Aa, 237382 families: 1.61 -> 1.28 ms.
@@ -555,7 +624,7 @@ NCD bool scb_prefilter(const SCBView& v, float rx, float ry, float rz, float rw,
                        float fw) {
   const float d32 = __fmaf_rn(rz, fz, __fmaf_rn(ry, fy, rx * fx));
   const float s32 = fw * rw;
-  const float x = __fmaf_rn(-v.band_hT2, s32, fabsf(fabsf(d32) - s32) - kScbBandEps);
+  const float x = __fmaf_rn(-v.band_hT2, s32, fabsf(fabsf(d32) - s32));
   return x * fabsf(x) < __fmaf_rn(-v.band_T2 * s32, s32, v.band_T2c);
 }
 
@@ -563,6 +632,38 @@ NCD bool scb_prefilter(const SCBView& v, float rx, float ry, float rz, float rw,
 // within this chord of their mean direction (beyond it too few demi-normals
 // are ruled out to pay for the second test)
 constexpr double kScbCoarseChord = 0.2;
+// bounds of the neutrons (direction u, FP32 wavelength fw) of the wave's lanes
+// with `alive`: mean direction, chord, wavelength range; all lanes call this.  ok
+// is false where the chord is wider, or NaN (e.g. directions that cancel).
+struct ScbBounds {
+  bool ok;
+  float R0, gx, gy, gz, fwlo, fwhi;
+};
+NCD ScbBounds scb_bounds(const V3& u, float fw, bool alive) {
+  ScbBounds B{false, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  const double mx0 = wave_sum_d(alive ? u.x : 0.0), my0 = wave_sum_d(alive ? u.y : 0.0),
+               mz0 = wave_sum_d(alive ? u.z : 0.0);
+  const double mn = sqrt(mx0 * mx0 + my0 * my0 + mz0 * mz0);
+  const double mx = mx0 / mn, my = my0 / mn, mz = mz0 / mn;
+  const double cmin = wave_min_d(alive ? u.x * mx + u.y * my + u.z * mz : 1.0);
+  const double rho = sqrt(dmax(0.0, 2.0 - 2.0 * cmin));
+  if (mn > 0.0 && rho < kScbCoarseChord) {
+    B.ok = true;
+    B.R0 = (float)rho + kScbBandEps + 1e-5f;
+    B.gx = (float)mx; B.gy = (float)my; B.gz = (float)mz;
+    B.fwlo = wave_min_f(alive ? fw : __builtin_huge_valf());
+    B.fwhi = wave_max_f(alive ? fw : -__builtin_huge_valf());
+  }
+  return B;
+}
+// false: demi-normal r fails the pre-filter for every neutron within the bounds
+NCD bool scb_bounds_pass(const SCBView& v, const ScbBounds& B, const float4& r) {
+  const float D = fabsf(__fmaf_rn(r.z, B.gz, __fmaf_rn(r.y, B.gy, r.x * B.gx)));
+  const float slo = B.fwlo * r.w, shi = B.fwhi * r.w;
+  const float R = __fmaf_rn(v.band_hT2, shi, B.R0) +
+                  1.000001f * __builtin_amdgcn_sqrtf(fmaxf(0.0f, __fmaf_rn(-v.band_T2 * slo, slo, v.band_T2c)));
+  return (slo < D + R) && (shi > D - R);
+}
 
 // Scan of all (family, demi-normal, side) contributions in the reference's
 // order (families by decreasing d, normals in family order, anti-normal side
@@ -591,7 +692,7 @@ constexpr double kScbCoarseChord = 0.2;
 //  - dense: every lane pre-filters every normal, in groups of kScbGroup with
 //    a wave-uniform index (scalar loads of the FP32 records).
 // All lanes of the wavefront must call this together.
-template <bool Select>
+template <bool Select, bool AllowSlow = false>
 NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uint16_t* __restrict__ list) {
   L.count = 0;
   L.total = 0.0;
@@ -605,35 +706,20 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
   const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
   ScbAcc a{-1, 0.0, 0.0, 0.0};
   int n = 0, base = 0;
-  // bounds of the wave: mean direction, chord, wavelength range
-  const double mx0 = wave_sum_d(alive ? L.u.x : 0.0), my0 = wave_sum_d(alive ? L.u.y : 0.0),
-               mz0 = wave_sum_d(alive ? L.u.z : 0.0);
-  const double mn = sqrt(mx0 * mx0 + my0 * my0 + mz0 * mz0);
-  const double mx = mx0 / mn, my = my0 / mn, mz = mz0 / mn;
-  const double cmin = wave_min_d(alive ? L.u.x * mx + L.u.y * my + L.u.z * mz : 1.0);
-  const double rho = sqrt(dmax(0.0, 2.0 - 2.0 * cmin));
-  // (a NaN in the bounds, e.g. from directions that cancel, selects the dense scan)
-  if (jmax > 0 && mn > 0.0 && rho < kScbCoarseChord) {
-    const float R0 = (float)rho + kScbBandEps + 1e-5f;
-    const float gx = (float)mx, gy = (float)my, gz = (float)mz;
-    const float fwlo = wave_min_f(alive ? fw : __builtin_huge_valf());
-    const float fwhi = wave_max_f(alive ? fw : -__builtin_huge_valf());
+  const ScbBounds B = scb_bounds(L.u, fw, alive);
+  if (jmax > 0 && B.ok) {
     for (int jb = 0; jb < jmax; jb += 64) {
       const int jl = jb + lane;
       float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
       bool pass = false;
       if (jl < jmax) {
         r = v.nrec32[jl];
-        const float D = fabsf(__fmaf_rn(r.z, gz, __fmaf_rn(r.y, gy, r.x * gx)));
-        const float slo = fwlo * r.w, shi = fwhi * r.w;
-        const float R = __fmaf_rn(v.band_hT2, shi, R0) +
-                        1.000001f * __builtin_amdgcn_sqrtf(fmaxf(0.0f, __fmaf_rn(-v.band_T2 * slo, slo, v.band_T2c)));
-        pass = (slo < D + R) && (shi > D - R);
+        pass = scb_bounds_pass(v, B, r);
       }
       uint64_t M = __ballot(pass);
       if (!M) continue;
       if (__any(n + __popcll(M) > kScbListCap) || jb + 64 - base > kScbListSpan) {
-        scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
+        scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
         n = 0;
         base = jb;
         if (!__any(alive)) break;
@@ -653,7 +739,7 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
   } else {
     for (int jb = 0; jb < jmax; jb += kScbGroup) {
       if (__any(n > kScbListCap - kScbGroup) || jb + kScbGroup - base > kScbListSpan) {
-        scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
+        scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
         n = 0;
         base = jb;
         if (!__any(alive)) break;
@@ -675,7 +761,7 @@ NCD void scb_walk(const SCBView& v, ScbLane& L, int n_select, double target, uin
       }
     }
   }
-  scb_eval_list<Select>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
+  scb_eval_list<Select, AllowSlow>(v, L, a, alive, list, base, n, w, wl3, n_select, target);
   L.total = a.commul_last;
 }
 

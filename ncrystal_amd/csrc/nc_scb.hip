@@ -12,9 +12,10 @@
 // Each kernel pair is a main kernel without the Romberg circle integral and
 // a queue kernel that redoes, with it, the neutrons whose scan met a
 // contribution outside the spline's validity (backscattering within the
-// mosaic spread), one wave per neutron.  Cross sections involve no random numbers and sampling
-// draws from the neutron's own Philox stream from its first draw, so the
-// split does not change any result either.
+// mosaic spread), one wave per neutron or, for long queues of a narrow beam,
+// several or one lane (scb_wave_group).  Cross sections involve no random numbers
+// and sampling draws from the neutron's own Philox stream from its first draw, so
+// the split does not change any result either.
 //
 // Reference: ncrystal_core/src/scbragg/NCSCBragg.cc:233-323 (crossSection,
 // sampleScatter), ncrystal_core/src/cinterface/ncrystal.cc:1248-1282 (batched
@@ -46,17 +47,90 @@ NCD void scb_xs_one(const SCBView& v, bool valid, int64_t i, const double* __res
 
 // Contributions of one neutron evaluated by a whole wave, with the Romberg
 // circle integral: lane t tests demi-normal jb + t; the candidates collect in
-// order in the wave's list and are evaluated 64 at a time, one per lane; every
-// lane then adds up the contributions in order (the sums and the selection of
-// scb_eval_list).  The queue holds few neutrons (0.2 % of a beam on a 30
-// arcmin crystal), each with a long scan and some integrals: one lane per
-// neutron left 60 waves to run 0.8 ms (cross sections of 2e6 neutrons) and 1.8
-// ms (two passes, sampling).
+// order in the wave's list and are evaluated 64 at a time, one per lane, but for
+// their Romberg integrals: a few take the whole wave one after the other, a point
+// per lane (on its own lane each would hold the wave for its 17 points and more);
+// the contributions are then added up in order (the sums and
+// the selection of scb_eval_list) from the lanes' registers.  The queue usually
+// holds few neutrons (0.2 % of a beam on a 30 arcmin crystal), each with a long
+// scan and some integrals: one lane per neutron left 60 waves to run 0.8 ms
+// (cross sections of 2e6 neutrons) and 1.8 ms (two passes, sampling).
 // The scan keeps four loads in flight (a scan of 15000 demi-normals, 1 Aa, is
 // otherwise one load's latency per 64 of them), and the selection reads the
 // candidates from the list where it held them all.
 constexpr int kScbWaveList = 1024;
 constexpr int kScbWaveLoads = 4;
+static_assert(2 * kScbWaveList * sizeof(int) >= kScbListWave * sizeof(uint16_t), "a wave's lists, of either kind");
+// integrals of a batch that the wave does together; more are done a lane each
+// (5 degree crystal, dozens in a batch, 30000 isotropic neutrons: 15 ms together,
+// 4.8 a lane each)
+constexpr int kScbWaveSlow = 2;
+// A narrow beam near backscattering puts most of a batch in the queue.  Then a
+// wave takes several neutrons in a row and, where their directions are as close
+// as for the wave-level filter (scb_walk), scans the demi-normals once for all of
+// them: the ones left are the list that each neutron tests.
+constexpr int kScbWaveGroup = 32;
+constexpr int kScbWaveShare = 3;  // from this many neutrons on
+// lists of a wave in LDS: the neutron's candidates, the group's demi-normals (n
+// of them, or -1: scan all)
+struct ScbWaveLists {
+  int* cand;
+  int* near;
+  int n;
+};
+// neutrons of a wave at a time, of a queue of nq: several if 64 of them, from all
+// over the queue, are close (every wave finds the same), and 64 of these, one per
+// lane, if there are enough to fill the chip that way: lanes with the same
+// candidates cost one evaluation for 64 neutrons, and add up side by side.
+// Otherwise one, and the next a launch's waves on: the queue is sorted by scan
+// length, and neighbours would all be the long ones.
+// Cross sections / sampling, all neutrons queued, narrow beam: 20000 at
+// backscattering off a 0.2 degree crystal 0.33 / 0.59 ms with one per wave, 0.26 /
+// 0.44 several, 0.26 / 0.38 in lanes; off a 5 degree crystal 2.28 / 4.51, 2.07 / 3.54
+// and 3.23 / 5.90; 100000 of 1.5 Aa, 5 degrees: 9.8 / 21.2, 7.7 / 15.2 and 3.1 / 5.5.
+constexpr int64_t kScbLaneQueue = 65536;
+NCD int scb_wave_group(const SCBView& v, const double* __restrict__ ekin, const double* __restrict__ dirs,
+                       const int64_t* __restrict__ queue, int64_t nq, int64_t nwaves) {
+  const int64_t g = (nq + nwaves - 1) / nwaves;
+  if (g < kScbWaveShare) return 1;
+  const int64_t i = queue[(int64_t)((double)__lane_id() * ((double)nq * 0x1.0p-6))];
+  ScbLane L;
+  L.wl = 1.0;
+  L.u = V3{0.0, 0.0, 1.0};
+  scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
+  if (!scb_bounds(L.u, (float)gm_round(L.wl), true).ok) return 1;
+  if (nq >= kScbLaneQueue) return 64;
+  return (int)(g < kScbWaveGroup ? g : kScbWaveGroup);
+}
+NCD void scb_wave_near(const SCBView& v, const double* __restrict__ ekin, const double* __restrict__ dirs,
+                       const int64_t* __restrict__ queue, int ng, ScbWaveLists& W) {
+  W.n = -1;
+  if (ng < kScbWaveShare) return;
+  const int lane = (int)__lane_id();
+  const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
+  ScbLane L;
+  L.wl = 1.0;
+  L.u = V3{0.0, 0.0, 1.0};
+  L.jlim = 0;
+  if (lane < ng) {
+    const int64_t i = queue[lane];
+    scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
+  }
+  const ScbBounds B = scb_bounds(L.u, (float)gm_round(L.wl), L.jlim > 0);
+  const int jmax = wave_max_i(L.jlim);
+  if (!B.ok) return;
+  int n = 0;
+  for (int jb = 0; jb < jmax; jb += 64) {
+    const int j = jb + lane;
+    const bool pass = j < jmax && scb_bounds_pass(v, B, v.nrec32[j < jmax ? j : jmax - 1]);
+    const uint64_t M = __ballot(pass);
+    if (n + __popcll(M) > kScbWaveList) return;
+    if (pass) W.near[n + __popcll(M & below)] = j;
+    n += __popcll(M);
+  }
+  wave_lds_fence();
+  W.n = n;
+}
 template <bool Select>
 NCD bool scb_wave_eval(const SCBView& v, ScbLane& L, ScbAcc& a, int n_select, double target, double w, double wl3,
                        const int* __restrict__ list, int n) {
@@ -64,15 +138,36 @@ NCD bool scb_wave_eval(const SCBView& v, ScbLane& L, ScbAcc& a, int n_select, do
   for (int b = 0; b < n; b += 64) {
     double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
     double xs0 = 0.0, xs1 = 0.0;
+    ScbSlow slow{0u, 0.0, 0.0, 0.0, 0.0};
     int f = 0;
     if (b + lane < n) {
       const int j = list[b + lane];
       r = v.nrec[j];
       const double2 nf = v.nfx[j];
       f = (int)nf.y;
-      scb_candidate<true>(v, r, nf.x, w, wl3, L.u.x, L.u.y, L.u.z, xs0, xs1);
+      scb_candidate<true>(v, r, nf.x, w, wl3, L.u.x, L.u.y, L.u.z, xs0, xs1, &slow);
     }
-    uint64_t C = __ballot(xs0 != 0.0 || xs1 != 0.0);
+    const uint64_t S0 = __ballot(slow.sides & 1u), S1 = __ballot(slow.sides & 2u);
+    if (__popcll(S0) + __popcll(S1) > kScbWaveSlow) {
+      scb_slow_sides(v, slow, xs0, xs1);
+    } else {
+#pragma nounroll
+      for (int side = 0; side < 2; ++side) {
+        uint64_t S = side ? S1 : S0;
+#pragma nounroll
+        while (S) {
+          const int t = __builtin_ctzll(S);
+          S &= S - 1ull;
+          const double dot = readlane_d(slow.dot, t);
+          const double cc = dclamp(side == 0 ? dot : -dot, -1.0, 1.0);
+          const double ci = gos_circle_slow<true>(v, cc, sqrt(1.0 - cc * cc), readlane_d(slow.sinpt, t),
+                                                  readlane_d(slow.cospt, t));
+          if (lane == t) (side == 0 ? xs0 : xs1) = slow.Q * ci;
+        }
+      }
+    }
+    const uint64_t B0 = __ballot(xs0 != 0.0), B1 = __ballot(xs1 != 0.0);
+    uint64_t C = B0 | B1;
     while (C) {
       const int t = __builtin_ctzll(C);
       C &= C - 1ull;
@@ -83,16 +178,16 @@ NCD bool scb_wave_eval(const SCBView& v, ScbLane& L, ScbAcc& a, int n_select, do
         a.xssum = 0.0;
       }
       for (int side = 0; side < 2; ++side) {
-        const double xs = __shfl(side ? xs1 : xs0, t, 64);
-        if (!xs) continue;
+        if (!(((side ? B1 : B0) >> t) & 1ull)) continue;
+        const double xs = readlane_d(side ? xs1 : xs0, t);
         const double cm = a.xsoffset + (a.xssum += xs);
         a.commul_last = cm;
         if constexpr (Select) {
           const bool hit = n_select < 5 ? (cm > target) : !(cm < target);
           if (hit || L.count == n_select - 1) {
-            const double nx = __shfl(r.x, t, 64), ny = __shfl(r.y, t, 64), nz = __shfl(r.z, t, 64);
+            const double nx = readlane_d(r.x, t), ny = readlane_d(r.y, t), nz = readlane_d(r.z, t);
             L.found = true;
-            L.sel_inv2d_r = __shfl(r.w, t, 64);
+            L.sel_inv2d_r = readlane_d(r.w, t);
             L.sel_normal = side == 0 ? V3{-nx, -ny, -nz} : V3{nx, ny, nz};
             return true;
           }
@@ -106,10 +201,11 @@ NCD bool scb_wave_eval(const SCBView& v, ScbLane& L, ScbAcc& a, int n_select, do
 // complete: the list holds all candidates (set by the first pass and taken by
 // the second); nlist: their number
 template <bool Select>
-NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target, int* __restrict__ list, int& nlist,
+NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target, const ScbWaveLists& W, int& nlist,
                        bool& complete) {
   const int lane = (int)__lane_id();
   const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
+  int* list = W.cand;
   L.count = 0;
   L.total = 0.0;
   L.slow = false;
@@ -124,30 +220,32 @@ NCD void scb_wave_walk(const SCBView& v, ScbLane& L, int n_select, double target
   const float fx = (float)L.u.x, fy = (float)L.u.y, fz = (float)L.u.z, fw = (float)w;
   int n = 0;
   complete = true;
-  for (int jb = 0; jb < L.jlim; jb += 64 * kScbWaveLoads) {
+  const int end = L.jlim > 0 && W.n >= 0 ? W.n : L.jlim;
+  for (int jb = 0; jb < end; jb += 64 * kScbWaveLoads) {
     if (n > kScbWaveList - 64 * kScbWaveLoads) {
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_fence();
       if (scb_wave_eval<Select>(v, L, a, n_select, target, w, wl3, list, n)) return;
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_fence();
       n = 0;
       complete = false;
     }
+    int js[kScbWaveLoads];
     float4 r[kScbWaveLoads];
 #pragma unroll
     for (int q = 0; q < kScbWaveLoads; ++q) {
-      const int j = jb + 64 * q + lane;
-      r[q] = v.nrec32[j < L.jlim ? j : L.jlim - 1];
+      const int at = jb + 64 * q + lane;
+      js[q] = at < end ? (W.n >= 0 ? W.near[at] : at) : L.jlim;
+      r[q] = v.nrec32[js[q] < L.jlim ? js[q] : L.jlim - 1];
     }
 #pragma unroll
     for (int q = 0; q < kScbWaveLoads; ++q) {
-      const int j = jb + 64 * q + lane;
-      const bool cand = j < L.jlim && scb_prefilter(v, r[q].x, r[q].y, r[q].z, r[q].w, fx, fy, fz, fw);
+      const bool cand = js[q] < L.jlim && scb_prefilter(v, r[q].x, r[q].y, r[q].z, r[q].w, fx, fy, fz, fw);
       const uint64_t M = __ballot(cand);
-      if (cand) list[n + __popcll(M & below)] = j;
+      if (cand) list[n + __popcll(M & below)] = js[q];
       n += __popcll(M);
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   nlist = n;
   if (scb_wave_eval<Select>(v, L, a, n_select, target, w, wl3, list, n)) return;
   L.total = a.commul_last;
@@ -257,17 +355,36 @@ __global__ void __launch_bounds__(256) k_scb_xs_slow(SCBView v, const double* __
                                                      const double* __restrict__ dirs, double* __restrict__ out,
                                                      const int64_t* __restrict__ queue,
                                                      const unsigned long long* __restrict__ qcount) {
-  __shared__ int lists[4 * kScbWaveList];
-  int* list = lists + (threadIdx.x >> 6) * kScbWaveList;
+  __shared__ __align__(16) int lists[4][2][kScbWaveList];
+  ScbWaveLists W{lists[threadIdx.x >> 6][0], lists[threadIdx.x >> 6][1], -1};
   const int64_t nq = (int64_t)*qcount;
   const int64_t nwaves = (int64_t)gridDim.x * 4;
-  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < nq; q += nwaves) {
+  const int group = scb_wave_group(v, ekin, dirs, queue, nq, nwaves);
+  const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * group;
+  if (group == 64) {
+    for (int64_t q0 = first; q0 < nq; q0 += nwaves * 64) {
+      const int64_t q = q0 + (threadIdx.x & 63);
+      const int64_t i = queue[q < nq ? q : nq - 1];
+      ScbLane L;
+      L.wl = 1.0;
+      L.u = V3{0.0, 0.0, 1.0};
+      L.jlim = 0;
+      const bool can = q < nq && scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
+      scb_walk<false, true>(v, L, 0, 0.0, reinterpret_cast<uint16_t*>(W.cand));
+      if (q < nq) out[i] = (can && L.count) ? L.total : 0.0;
+    }
+    return;
+  }
+  // (every lane of a wave has the same q)
+  for (int64_t q0 = first; q0 < nq; q0 += nwaves * group)
+  for (int64_t q = q0; q < nq && q < q0 + group; ++q) {
+    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(nq - q0 < group ? nq - q0 : group), W);
     const int64_t i = queue[q];
     ScbLane L;
     const bool can = scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
     int nlist = 0;
     bool complete = false;
-    scb_wave_walk<false>(v, L, 0, 0.0, list, nlist, complete);
+    scb_wave_walk<false>(v, L, 0, 0.0, W, nlist, complete);
     if ((threadIdx.x & 63) == 0) out[i] = (can && L.count) ? L.total : 0.0;
   }
 }
@@ -396,11 +513,49 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
                                                          double* __restrict__ oD, const int64_t* __restrict__ queue,
                                                          const unsigned long long* __restrict__ qcount,
                                                          const int64_t* __restrict__ idmap, int skip) {
-  __shared__ int lists[4 * kScbWaveList];
-  int* list = lists + (threadIdx.x >> 6) * kScbWaveList;
+  __shared__ __align__(16) int lists[4][2][kScbWaveList];
+  ScbWaveLists W{lists[threadIdx.x >> 6][0], lists[threadIdx.x >> 6][1], -1};
   const int64_t nq = (int64_t)*qcount;
   const int64_t nwaves = (int64_t)gridDim.x * 4;
-  for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < nq; q += nwaves) {
+  const int group = scb_wave_group(v, ekin, dirs, queue, nq, nwaves);
+  const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * group;
+  if (group == 64) {
+    uint16_t* list = reinterpret_cast<uint16_t*>(W.cand);
+    for (int64_t q0 = first; q0 < nq; q0 += nwaves * 64) {
+      const int64_t q = q0 + (threadIdx.x & 63);
+      const int64_t i = queue[q < nq ? q : nq - 1];
+      const double E = ekin[i];
+      const V3 din{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
+      ScbLane L;
+      L.wl = 1.0;
+      L.u = V3{0.0, 0.0, 1.0};
+      L.jlim = 0;
+      const bool can = q < nq && scb_lane_setup(v, E, din.x, din.y, din.z, L);
+      scb_walk<false, true>(v, L, 0, 0.0, list);
+      const bool scatter = can && L.count > 0 && L.total > 0.0;
+      const int64_t o = idmap ? idmap[i] : i;
+      Rng rng;
+      rng.init(seed, stream, (uint64_t)o);
+      for (int s = 0; s < skip; ++s) (void)rng.gen();
+      const int n = L.count;
+      const double target = scatter && n > 1 ? L.total * rng.gen() : 0.0;
+      if (!scatter) L.jlim = 0;
+      scb_walk<true, true>(v, L, n, target, list);
+      V3 d = din;
+      if (scatter && L.found) d = gm_genscat(v, rng, L.sel_normal, L.sel_inv2d_r, L.wl, L.u);
+      if (q < nq) {
+        oE[o] = E;
+        oD[3 * o] = d.x;
+        oD[3 * o + 1] = d.y;
+        oD[3 * o + 2] = d.z;
+      }
+    }
+    return;
+  }
+  // (every lane of a wave has the same q)
+  for (int64_t q0 = first; q0 < nq; q0 += nwaves * group)
+  for (int64_t q = q0; q < nq && q < q0 + group; ++q) {
+    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(nq - q0 < group ? nq - q0 : group), W);
     const int64_t i = queue[q];
     const double E = ekin[i];
     const V3 din{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
@@ -408,7 +563,7 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
     const bool can = scb_lane_setup(v, E, din.x, din.y, din.z, L);
     int nlist = 0;
     bool complete = false;
-    scb_wave_walk<false>(v, L, 0, 0.0, list, nlist, complete);
+    scb_wave_walk<false>(v, L, 0, 0.0, W, nlist, complete);
     const int64_t o = idmap ? idmap[i] : i;  // output slot and Philox index
     V3 d = din;
     if (can && L.count > 0 && L.total > 0.0) {  // the same for every lane
@@ -417,7 +572,7 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
       for (int s = 0; s < skip; ++s) (void)rng.gen();
       const int n = L.count;
       const double target = n > 1 ? L.total * rng.gen() : 0.0;
-      scb_wave_walk<true>(v, L, n, target, list, nlist, complete);
+      scb_wave_walk<true>(v, L, n, target, W, nlist, complete);
       if (L.found) d = gm_genscat(v, rng, L.sel_normal, L.sel_inv2d_r, L.wl, L.u);
     }
     if ((threadIdx.x & 63) == 0) {

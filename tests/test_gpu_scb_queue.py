@@ -1,5 +1,5 @@
-"""SCBragg's Romberg queue (one wave per neutron), its candidate lists and the
-family guide, at the sizes where they can go wrong, against the checker: cross
+"""SCBragg's Romberg queue (one wave per neutron, several of a narrow beam, or
+one lane), its candidate lists and the family guide, at the sizes where they can go wrong, against the checker: cross
 sections and samples on the same Philox streams."""
 import math
 
@@ -31,14 +31,14 @@ def _crystal(core, oracle, cr, mosaic_deg):
 
 
 def _compare(g, o, e, d, label):
-    x, y = g.crossSection(e, d), o.xs_dir(e, d)
+    x, y = g.crossSection(e, d), o.xs_dir(e, d, nthreads=8)
     # the same arithmetic with the device's acos, sqrt and cosine in the circle
     # integral; its density has a logarithmic slope of 1/sigma^2 <= 2e4 here
     assert np.max(np.abs(x - y) / np.maximum(y, 1e-300)) < 1e-10
     assert np.array_equal(x == 0, y == 0)
     g.setRNGState(9, 0)
     ge, gd = g.sampleScatter(e, d)
-    _, od, nerr = o.sample_dir(e, d, seed=9)
+    _, od, nerr = o.sample_dir(e, d, seed=9, nthreads=8)
     assert nerr == 0 and np.array_equal(ge, e)
     assert_streams_match(np.max(np.abs(gd - od), axis=1) > 1e-9, label)
     return x
@@ -56,6 +56,30 @@ def test_backscattering_along_normals(core, oracle, n):
     e = WL2EKIN / ((1.0 - 10.0 ** rng.uniform(-8, -4, n)) / t["inv2d"][f]) ** 2
     x = _compare(g, o, e, d, f"backscattering {n}")
     assert np.mean(x > 0) > 0.9
+
+
+# a narrow beam near backscattering from one family: waves that take three
+# neutrons and more, and lanes from 65536 queued ones on; wide: single ones at the
+# same sizes.  5 degrees: more integrals in a batch of candidates than the wave
+# does together.
+@pytest.mark.parametrize("n,mosaic,spread", [(9001, 0.5, 0.3), (9001, 5.0, 0.3), (80001, 0.5, 0.3), (80001, 5.0, 0.3),
+                                             (13001, 0.5, None)])
+def test_many_queued(core, oracle, n, mosaic, spread):
+    g, o, dsp = _crystal(core, oracle, synth.fcc_powder(dcutoff=0.7), mosaic)
+    t = g.tables()
+    rng = np.random.default_rng(n)
+    f = rng.integers(0, len(t["inv2d"]), n) if spread is None else np.full(n, len(t["inv2d"]) // 3)
+    d = t["normals"][t["off"][f]] + rng.normal(scale=(spread or 0.3) * math.radians(mosaic), size=(n, 3))
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    e = WL2EKIN / ((1.0 - 10.0 ** rng.uniform(-8, -4, n)) / t["inv2d"][f]) ** 2
+    x = _compare(g, o, e, d, f"queued {n} {mosaic}")
+    assert np.mean(x > 0) > 0.95
+    g.setRNGState(9, 0)
+    od = g.sampleScatter(e, d)[1]
+    for m in (1, 700):  # a wave each: the same sums and integrals in the same order
+        assert np.array_equal(g.crossSection(e[:m], d[:m]), x[:m])
+        g.setRNGState(9, 0)
+        assert np.array_equal(g.sampleScatter(e[:m], d[:m])[1], od[:m])
 
 
 def test_long_lists(core, oracle):
