@@ -137,12 +137,11 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_sab(const BatchMat* __res
     const int skip = m.view.n > 1 ? 1 : 0;
     const SABView& view = m.view.sab[0];
     const SabSmall<Lds> small(view, lds);
-    int64_t begin, end;
-    sab_share(cnt, threadIdx.x >> 6, kBatchBlock / 64, begin, end);
+    const SabShare<kBatchBlock / 64> share(cnt, threadIdx.x >> 6, kBatchBlock / 64);
     sab_stream<false>(
-        view, small, r.seed, (uint32_t)r.stream, skip, begin, end,
-        [&](int64_t p, int64_t& k, double& E) {
-          k = sab[m.offset + tile.begin + p];
+        view, small, r.seed, (uint32_t)r.stream, skip, share,
+        [&](int64_t i, int64_t& k, double& E) {
+          k = sab[m.offset + tile.begin + share.at(i)];
           E = ekin[m.offset + k];
           return true;
         },

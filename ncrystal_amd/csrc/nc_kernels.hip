@@ -220,12 +220,12 @@ __global__ void __launch_bounds__(256, 4) k_comp_sab(SABView s, const double* __
   const int64_t m = queue_count(count, 0, total);
   if (m == 0) return;
   const SabSmall<Lds> small(s, lds);
-  int64_t begin, end;
-  sab_share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4, begin, end);
+  const SabShare<> share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4,
+                       share_shift(m));
   sab_stream<Dirs>(
-      s, small, seed, stream, skip, begin, end,
-      [&](int64_t p, int64_t& k, double& E) {
-        k = q[p];
+      s, small, seed, stream, skip, share,
+      [&](int64_t i, int64_t& k, double& E) {
+        k = q[share.at(i)];
         E = ekin[(total == n) ? k : (k % n)];
         return true;
       },
@@ -337,12 +337,11 @@ __global__ void __launch_bounds__(256, 4) k_comp_local(CompView c, const double*
     const SABView& s = c.sab[sl];
     if (low > 0) {
       const SabSmall<Lds> small(s, lds);
-      int64_t begin, end;
-      sab_share(low, tid >> 6, 4, begin, end, 32);
+      const SabShare<4> share(low, tid >> 6, 4, 5);
       sab_stream<Dirs>(
-          s, small, seed, stream, skip, begin, end,
-          [&](int64_t p, int64_t& k, double& E) {
-            k = k0 + list[sl][p];
+          s, small, seed, stream, skip, share,
+          [&](int64_t i, int64_t& k, double& E) {
+            k = k0 + list[sl][share.at(i)];
             E = ekin[(total == n) ? k : (k % n)];
             return true;
           },
@@ -406,23 +405,25 @@ __global__ void __launch_bounds__(256, 4) k_sab_sample_iso_main(SABView s, const
                                                                 unsigned long long* __restrict__ qcount,
                                                                 int domain_check) {
   __shared__ double lds[Lds ? kSabLds : 1];
-  // neutrons for the high-energy queue, kept until there is a wave of them:
-  // one atomic each would pace a batch that has many
-  __shared__ int64_t bufs[4][128];
+  // places in the share of neutrons for the high-energy queue, kept until there are
+  // four waves of them: appends to it run one after the other, 13 ns each, and
+  // would pace a batch that has many (5e6 of 1e7, in order: 1.85 ms with one
+  // append per wave of them)
+  constexpr int kKeep = 256;
+  __shared__ uint32_t bufs[4][kKeep + 64];
   __shared__ int counts[4];
   const int lane = (int)(threadIdx.x & 63);
-  int64_t* buf = bufs[threadIdx.x >> 6];
+  uint32_t* buf = bufs[threadIdx.x >> 6];
   int* have = counts + (threadIdx.x >> 6);
   if (lane == 0) *have = 0;
   __syncthreads();
   const SabSmall<Lds> small(s, lds);
-  int64_t begin, end;
-  sab_share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4, begin, end);
+  const SabShare<> share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4, share_shift(total));
   const double emax = s.egrid[s.ne - 1];
   sab_stream<false>(
-      s, small, seed, stream, 0, begin, end,
-      [&](int64_t p, int64_t& k, double& E) {
-        k = p;
+      s, small, seed, stream, 0, share,
+      [&](int64_t i, int64_t& k, double& E) {
+        k = share.at(i);
         E = ekin[(total == n) ? k : (k % n)];
         if (domain_check && !(E >= 0.0 && E <= __builtin_huge_val())) {
           // a composition outside its energy domain does not scatter
@@ -432,20 +433,20 @@ __global__ void __launch_bounds__(256, 4) k_sab_sample_iso_main(SABView s, const
         }
         if (E < emax) return true;
         // the free-gas kernel, and the sampler's own handling of non-finite E
-        buf[atomicAdd(have, 1)] = k;
+        buf[atomicAdd(have, 1)] = (uint32_t)i;
         return false;
       },
-      [&](bool last) {  // at most 63 kept and 64 new ones
-        __builtin_amdgcn_wave_barrier();
-        const int c = *(volatile int*)have;
-        if (c < (last ? 1 : 64)) return;
+      [&](bool last) {  // at most kKeep - 1 kept and 64 new ones
+        wave_lds_fence();
+        const int c = *have;
+        if (c < (last ? 1 : kKeep)) return;
         unsigned long long at = 0ull;
         if (lane == 0) at = atomicAdd(qcount, (unsigned long long)c);
         at = __shfl(at, 0, 64);
-        for (int j = lane; j < c; j += 64) queue[at + j] = buf[j];
-        __builtin_amdgcn_wave_barrier();
-        if (lane == 0) *(volatile int*)have = 0;
-        __builtin_amdgcn_wave_barrier();
+        for (int j = lane; j < c; j += 64) queue[at + j] = share.at(buf[j]);
+        wave_lds_fence();
+        if (lane == 0) *have = 0;
+        wave_lds_fence();
       },
       [&](int64_t k, int rc, double Ef, double mu) {
         if (rc) atomicAdd(nerr, 1ull);

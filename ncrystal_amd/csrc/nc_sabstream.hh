@@ -176,17 +176,44 @@ NCD int egrid_sampler(const SABView& s, const double* egrid, double E) {
   return lo;
 }
 
-// Samples the neutrons at positions [next, end) of a list, all lanes of the
-// wave together.  take(pos, k, E): the neutron there (index k, which is also its
-// Philox index; E below the table's Emax), or false if there is nothing to
+// A wave's share of a list of n among nw waves: every nw-th piece of 1 << shift
+// places.  Pieces, because a list in the order of its energies has the tries of cold
+// neutrons, or nothing but neutrons above Emax, side by side (1e7 neutrons of 1 meV
+// to 1 eV, ordered: 660 us with one run of the list per wave, 590 in pieces).
+// share_shift: 64 places fill a wave before the next one is begun; of long lists
+// larger ones cost less (3e7 neutrons: 2.56 ms with 64, 2.52 with 256; one run each:
+// 2.55).
+NCD int share_shift(int64_t n) { return n > (1 << 24) ? 8 : 6; }
+template <int NW = 0>  // nw, where it is fixed
+struct SabShare {
+  uint32_t nw;
+  int shift;
+  int64_t w, size;
+  NCD SabShare(int64_t n, int64_t wave, int64_t nwaves, int sh = 6)
+      : nw(NW ? NW : (uint32_t)nwaves), shift(sh), w(wave), size(0) {
+    const int64_t pieces = (n + (1 << sh) - 1) >> sh;
+    if (w >= pieces) return;
+    size = ((pieces - w + nw - 1) / nw) << sh;
+    if ((pieces - 1 - w) % nw == 0) size -= (pieces << sh) - n;  // the list's last piece
+  }
+  // (a wave's pieces are fewer than 2^32)
+  NCD int64_t at(int64_t i) const {
+    const uint64_t piece = (uint64_t)(uint32_t)(i >> shift) * (NW ? NW : nw) + (uint64_t)w;
+    return (int64_t)(piece << shift) | (i & ((1 << shift) - 1));
+  }
+};
+
+// Samples the neutrons of a wave's share of a list, all lanes of the wave
+// together.  take(i, k, E): the neutron at place i of the share (index k, which is
+// also its Philox index; E below the table's Emax), or false if there is nothing to
 // sample; put(k, rc, Ef, mu) for an isotropic outcome or an error, and with Dirs
-// put_dir(k, Ef, ox, oy, oz) for the outcome about the incoming direction that dir(k, ix, iy, iz)
-// gives.  after(last) runs, the whole wave together, when lanes have taken
+// put_dir(k, Ef, ox, oy, oz) for the outcome about the incoming direction that
+// dir(k, ix, iy, iz) gives.  after(last) runs, the whole wave together, when lanes have taken
 // neutrons and once at the end.  skip: numbers of the stream already used.
-template <bool Dirs, class Small, class Take, class After, class Put, class PutDir, class Dir>
-NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_t stream, int skip, int64_t next, int64_t end,
-                    const Take& take, const After& after, const Put& put, const PutDir& put_dir,
-                    const Dir& dir) {
+template <bool Dirs, class Small, class Share, class Take, class After, class Put, class PutDir, class Dir>
+NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_t stream, int skip,
+                    const Share& share, const Take& take, const After& after, const Put& put,
+                    const PutDir& put_dir, const Dir& dir) {
   // kTry: the next try (nv >= 0: from the sampler; -1: alpha = beta = 0; -2: no
   // sampler); kFirst: an inner try of the first-bin rule; kDir: a try of the
   // outgoing direction
@@ -201,6 +228,7 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
   bool ultra = false;
   // the neutron's stream: index of its next number; the last block made (its
   // number and halves), whose second half is kept while the index is odd
+  int64_t next = 0;
   uint32_t drawn = 0, blk = 0;
   uint64_t h0 = 0, h1 = 0;
   const auto block = [&](uint32_t b) {
@@ -225,8 +253,8 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
   };
   while (true) {
     uint64_t idle = __ballot(mode == kIdle);
-    while (idle && next < end) {
-      const int64_t room = end - next;
+    while (idle && next < share.size) {
+      const int64_t room = share.size - next;
       const int cnt = room < (int64_t)__popcll(idle) ? (int)room : __popcll(idle);
       if (mode == kIdle) {
         const int rank = __popcll(idle & below);
@@ -399,15 +427,6 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
     }
   }
   after(true);
-}
-
-// positions of a wave's share of a list of n among nw waves: at least `fill`
-// each (64: a wave is filled before the next one is begun)
-NCD void sab_share(int64_t n, int64_t w, int64_t nw, int64_t& begin, int64_t& end, int fill = 64) {
-  int64_t per = (n + nw - 1) / nw;
-  per = per < fill ? fill : per;
-  begin = w * per < n ? w * per : n;
-  end = begin + per < n ? begin + per : n;
 }
 
 }  // namespace ncamd

@@ -78,6 +78,21 @@ def test_composition(core, oracle, sab, n):
     _check((ge, *gd.T), (oe, *np.asarray(od).reshape(-1, 3).T), f"oriented {n}")
 
 
+@pytest.mark.parametrize("n", [300001, 1200001])  # pieces of 64 and of 256 places per wave
+def test_ordered_energies(core, sab, n):
+    """a list in the order of its energies, most of it above Emax: whole waves keep
+    neutrons for the high-energy queue"""
+    g, o = sab
+    emax = g.egrid()[0][-1]
+    e = np.concatenate([np.sort(_energies(n - n // 2, emax, n)), emax * np.linspace(1.0, 5.0, n // 2)])
+    for x in (e, e[::-1].copy()):
+        g.setRNGState(5, 0)
+        ge, gm = g.sampleScatterIsotropic(x)
+        oe, om, nerr = o.sample_iso(x, seed=5, nthreads=8)
+        assert nerr == 0
+        _check((ge, gm), (oe, om), f"ordered {n}")
+
+
 def test_repeat_and_batch(core, oracle, sab):
     g, o = sab
     gc = core.create_composition([core.create_elincscatter([0.01], [1.0], [1.0]), g], [1.0, 1.0])
