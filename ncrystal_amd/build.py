@@ -13,7 +13,8 @@ HERE = pathlib.Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 OUT = HERE / "libncrystal_amd.so"
 BUILD = HERE / "_build"
-SOURCES = ["nc_kernels.hip", "nc_sab_build.hip", "nc_hkl.hip", "nc_scb.hip", "nc_batch.hip", "nc_kb.hip", "nc_mlp.hip", "nc_vdos.hip", "nc_mmc.hip", "nc_lc.hip", "nc_capi.hip"]
+SOURCES = ["nc_kernels.hip", "nc_sab_build.hip", "nc_hkl.hip", "nc_scb.hip", "nc_batch.hip", "nc_kb.hip",
+           "nc_kb_build.hip", "nc_mlp.hip", "nc_vdos.hip", "nc_mmc.hip", "nc_lc.hip", "nc_capi.hip"]
 ARCH = os.environ.get("NCAMD_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -34,7 +35,8 @@ HIPCC_FLAGS = [
 # 100 of them: S(alpha,beta) sampler 148 -> 109 registers (3 -> 4 waves per
 # SIMD, 5.32 -> 4.68 ms per 3e7 neutrons), composition pick 163 -> 77, envelope
 # sampler 110 -> 84 (4.92 -> 4.60 ms per 1e8), cross sections 100 -> 30.  The
-# kernels that build tables gain nothing by it.
+# kernels that build tables gain nothing by it or lose (envelope bounds 8.6 ->
+# 11.9 ms), and are in files of their own.
 PER_NEUTRON = {"nc_kernels.hip", "nc_scb.hip", "nc_batch.hip", "nc_kb.hip", "nc_mmc.hip", "nc_lc.hip"}
 PER_NEUTRON_FLAGS = ["-mllvm", "-disable-machine-licm"]
 
