@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(kCumulBlock) k_fp32_cumul_scan(const double* _
 // the threshold search (the number of planes up to E grows as E^1.5, so their
 // density changes little along it) and of the cumulative sum for the plane
 // pick.  A bucket holds the planes that a plain binary search can end at.
-// kPBBuckets buckets per plane at most, and bounded where a finer guide would
+// kPBBuckets buckets per plane (64 at least), and bounded where a finer guide would
 // take more of a die's L2 cache than its shorter searches give back: at 262k
 // planes (figures at PBView's lookups) 2^17 energy buckets cost 1.38 ms for
 // 1.27 with 2^18, and 2^19 the same as 2^18; 2^18 cumulative ones 1.14 ms for 1.12
@@ -499,37 +499,36 @@ constexpr int kPBGuideE = 1 << 18, kPBGuideC = 1 << 16, kPBBuckets = 16;
 
 void pb_guides(Proc* p, const std::vector<double>& e2d, const std::vector<double>& fdm) {
   const int n = (int)e2d.size();
-  // lo, hi of every bucket: the planes in buckets below it and up to it
-  auto guide = [n](const std::vector<double>& x, int nb, double scale, std::vector<PBGuide>& out) {
-    out.resize((size_t)nb);
-    for (int g = 0, i = 0; g < nb; ++g) {
+  // every bucket from the numbers lo, hi of planes in buckets below it and up to it
+  const auto guide = [n](const std::vector<double>& x, int nb, double scale, const auto& bucket) {
+    std::unique_ptr<PBGuide[]> out(new PBGuide[(size_t)nb]);  // (not cleared first: up to 4 MB)
+    for (int g = 0, i = 0, next = pb_bucket(x[0], scale, nb); g < nb; ++g) {
       const int lo = i;
-      while (i < n && pb_bucket(x[(size_t)i], scale, nb) <= g) ++i;
-      out[(size_t)g] = {lo, i, 0.0};
+      while (i < n && next <= g)
+        if (++i < n) next = pb_bucket(x[(size_t)i], scale, nb);
+      out[(size_t)g] = bucket(lo, i);
     }
+    return out;
   };
-  std::vector<PBGuide> eg, cg;
   PBView& v = p->pb;
   const long long want = std::max<long long>(64, (long long)kPBBuckets * n);
   v.e_n = (int)std::min<long long>(kPBGuideE, want);
   v.c_n = (int)std::min<long long>(kPBGuideC, want);
   v.e_scale = (double)v.e_n / v.top;
   v.c_scale = (double)v.c_n / v.all;
-  guide(e2d, v.e_n, v.e_scale, eg);
-  for (PBGuide& g : eg) {  // E >= the first energy: a plane before is always there
-    const int lo = std::max(1, g.lo), hi = std::max(1, g.cnt);
-    g = {lo, hi - lo, fdm[(size_t)lo - 1]};
-  }
-  guide(fdm, v.c_n, v.c_scale, cg);
-  for (PBGuide& g : cg) {  // a target is at most the last value: its plane is below n
-    const int lo = std::min(g.lo, n - 1), hi = std::min(g.cnt, n - 1);
-    g = {lo, hi - lo, e2d[(size_t)lo]};
-  }
+  const auto eg = guide(e2d, v.e_n, v.e_scale, [&](int lo, int hi) {
+    lo = std::max(1, lo);  // E >= the first energy: a plane before is always there
+    return PBGuide{lo, std::max(1, hi) - lo, fdm[(size_t)lo - 1]};
+  });
+  const auto cg = guide(fdm, v.c_n, v.c_scale, [&](int lo, int hi) {
+    lo = std::min(lo, n - 1);  // a target is at most the last value: its plane is below n
+    return PBGuide{lo, std::min(hi, n - 1) - lo, e2d[(size_t)lo]};
+  });
   DevBuf* be = p->newbuf();
-  be->upload(eg.data(), eg.size());
+  be->upload(eg.get(), (size_t)v.e_n);
   v.eg = be->as<PBGuide>();
   DevBuf* bc = p->newbuf();
-  bc->upload(cg.data(), cg.size());
+  bc->upload(cg.get(), (size_t)v.c_n);
   v.cg = bc->as<PBGuide>();
 }
 
@@ -999,23 +998,36 @@ Proc* create_sab(int na, int nb, const double* alpha, const double* beta, const 
 
   const int ne = (int)egrid.size();
   s.ne = ne;
-  DevBuf* beg = p->newbuf(); beg->upload(egrid.data(), egrid.size());
-  DevBuf* bxs = p->newbuf(); bxs->alloc(sizeof(double) * ne);
-  DevBuf* bhdr = p->newbuf(); bhdr->alloc(sizeof(int4) * ne);
-  DevBuf* bfst = p->newbuf(); bfst->alloc(sizeof(double) * ne);
-  DevBuf* bcdf = p->newbuf(); bcdf->alloc(sizeof(double) * (size_t)ne * (nb + 1));
-  DevBuf* bxy = p->newbuf(); bxy->alloc(sizeof(double2) * (size_t)ne * (nb + 1));
-  DevBuf* binf = p->newbuf(); binf->alloc(sizeof(AInfo) * (size_t)ne * nb);
-  NCAMD_HIP(hipMemset(bcdf->p, 0, bcdf->bytes));
-  NCAMD_HIP(hipMemset(bxy->p, 0, bxy->bytes));
-  NCAMD_HIP(hipMemset(binf->p, 0, binf->bytes));
-  launch_sab_analyse(B, beg->as<double>(), ne, bxs->as<double>(), bhdr->as<int4>(), bfst->as<double>(),
-                     bcdf->as<double>(), bxy->as<double2>(), binf->as<AInfo>(), 0);
+  if (nb + 1 > 65535) raise("BadInput", "beta grid too large (at most 65534 points)");
+  // one allocation for the energy grid's tables, the search guides and the
+  // sampler's layout: a material is set up in 0.4 to 1.4 ms, and an allocation and
+  // its release take 10 to 20 us of it
+  size_t at = 0;
+  const auto part = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) / 256 * 256; return o; };
+  const size_t n_cg = (size_t)ne * (kCdfGuide + 1), n_rg = (size_t)nb * (kRowGuide + 1);
+  const size_t o_eg = part(sizeof(double) * ne), o_xs = part(sizeof(double) * ne), o_hdr = part(sizeof(int4) * ne),
+               o_fst = part(sizeof(double) * ne), o_cdf = part(sizeof(double) * (size_t)ne * (nb + 1)),
+               o_xy = part(sizeof(double2) * (size_t)ne * (nb + 1)), o_inf = part(sizeof(AInfo) * (size_t)ne * nb),
+               o_head = part(sizeof(SabHead) * (size_t)ne * nb), o_pt = part(sizeof(SabPt) * (size_t)nb * na),
+               o_bin = part(sizeof(SabBin) * (size_t)ne * (nb + 1)), o_rs = part(sizeof(double) * (size_t)nb),
+               o_small = part(sizeof(double) * (size_t)(na + 2 * nb + 3 * ne)),
+               o_cg = part(sizeof(unsigned short) * n_cg), o_rg = part(sizeof(unsigned short) * n_rg);
+  DevBuf* blk = p->newbuf();
+  blk->alloc(at);
+  char* base = blk->as<char>();
+  const auto dbl = [base](size_t o) { return reinterpret_cast<double*>(base + o); };
+  double *d_eg = dbl(o_eg), *d_xs = dbl(o_xs), *d_fst = dbl(o_fst), *d_cdf = dbl(o_cdf);
+  int4* d_hdr = reinterpret_cast<int4*>(base + o_hdr);
+  double2* d_xy = reinterpret_cast<double2*>(base + o_xy);
+  AInfo* d_inf = reinterpret_cast<AInfo*>(base + o_inf);
+  NCAMD_HIP(hipMemcpy(d_eg, egrid.data(), sizeof(double) * ne, hipMemcpyHostToDevice));
+  NCAMD_HIP(hipMemset(d_cdf, 0, o_head - o_cdf));
+  launch_sab_analyse(B, d_eg, ne, d_xs, d_hdr, d_fst, d_cdf, d_xy, d_inf, 0);
   NCAMD_HIP(hipGetLastError());
   std::vector<double> xs(ne);
-  NCAMD_HIP(hipMemcpy(xs.data(), bxs->p, sizeof(double) * ne, hipMemcpyDeviceToHost));
+  NCAMD_HIP(hipMemcpy(xs.data(), d_xs, sizeof(double) * ne, hipMemcpyDeviceToHost));
   std::vector<int4> hdr(ne);
-  NCAMD_HIP(hipMemcpy(hdr.data(), bhdr->p, sizeof(int4) * ne, hipMemcpyDeviceToHost));
+  NCAMD_HIP(hipMemcpy(hdr.data(), d_hdr, sizeof(int4) * ne, hipMemcpyDeviceToHost));
   for (int i = 0; i < ne; ++i)
     if (hdr[i].x < 0) raise("CalcError", "S(alpha,beta) beta distribution has no area");
   // high-E constants (NCSABXSProvider.cc:35-51, NCSABSampler.cc:40-57)
@@ -1066,28 +1078,17 @@ Proc* create_sab(int na, int nb, const double* alpha, const double* beta, const 
   s.beta = bb->as<double>();
   s.sl = bsl->as<double2>();
   s.cumul = bcu->as<double>();
-  s.egrid = beg->as<double>();
-  s.xs = bxs->as<double>();
-  s.shdr = bhdr->as<int4>();
-  s.sfirst = bfst->as<double>();
-  s.scdf = bcdf->as<double>();
-  s.sxy = bxy->as<double2>();
-  s.sinfo = binf->as<AInfo>();
+  s.egrid = d_eg;
+  s.xs = d_xs;
+  s.shdr = d_hdr;
+  s.sfirst = d_fst;
+  s.scdf = d_cdf;
+  s.sxy = d_xy;
+  s.sinfo = d_inf;
   {
-    if (nb + 1 > 65535) raise("BadInput", "beta grid too large (at most 65534 points)");
-    // one allocation for the search guides and the sampler's layout
-    const size_t n_cg = (size_t)ne * (kCdfGuide + 1), n_rg = (size_t)nb * (kRowGuide + 1);
-    size_t at = 0;
-    const auto part = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) / 256 * 256; return o; };
-    const size_t o_head = part(sizeof(SabHead) * (size_t)ne * nb), o_pt = part(sizeof(SabPt) * (size_t)nb * na),
-                 o_bin = part(sizeof(SabBin) * (size_t)ne * (nb + 1)), o_rs = part(sizeof(double) * (size_t)nb),
-                 o_small = part(sizeof(double) * (size_t)(na + 2 * nb + 3 * ne)),
-                 o_cg = part(sizeof(unsigned short) * n_cg), o_rg = part(sizeof(unsigned short) * n_rg);
-    DevBuf* blk = p->newbuf();
-    blk->alloc(at);
-    char* base = blk->as<char>();
-    unsigned short *cg = reinterpret_cast<unsigned short*>(base + o_cg), *rg = reinterpret_cast<unsigned short*>(base + o_rg);
-    double* rs = reinterpret_cast<double*>(base + o_rs);
+    unsigned short* cg = reinterpret_cast<unsigned short*>(base + o_cg);
+    unsigned short* rg = reinterpret_cast<unsigned short*>(base + o_rg);
+    double* rs = dbl(o_rs);
     launch_sab_guides(s, cg, rg, rs, 0);
     NCAMD_HIP(hipGetLastError());
     s.cdf_guide = cg;
@@ -1096,7 +1097,7 @@ Proc* create_sab(int na, int nb, const double* alpha, const double* beta, const 
     SabPt* pt = reinterpret_cast<SabPt*>(base + o_pt);
     SabHead* head = reinterpret_cast<SabHead*>(base + o_head);
     SabBin* bin = reinterpret_cast<SabBin*>(base + o_bin);
-    double* small = reinterpret_cast<double*>(base + o_small);
+    double* small = dbl(o_small);
     launch_sab_pack(s, pt, head, bin, small, 0);
     NCAMD_HIP(hipGetLastError());
     NCAMD_HIP(hipDeviceSynchronize());
