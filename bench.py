@@ -458,7 +458,7 @@ def run_powderbragg(args):
                    "neutrons_per_step": n, "families": int(len(dsp)), "planes": nplanes,
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": ach / HBM_PEAK_GBS, "traffic": None, "kernel": "k_sample_iso<kCompPBOnly>",
+                     "frac": ach / HBM_PEAK_GBS, "traffic": None, "kernel": "k_sample_iso<kCompPBOnly, true>",
                      "kernel_ms": ts, "xs_fp64_ms": t64, "xs_fp32_ms": t32,
                      "xs_fp64_GBs": 16 * n / (t64 * 1e-3) / 1e9, "xs_fp32_GBs": 16 * n / (t32 * 1e-3) / 1e9},
         "cpu_baseline": cpu,

@@ -8,30 +8,48 @@
 #include "nc_kernels.hh"
 #include "nc_sabstream.hh"
 #include <algorithm>
+#include <type_traits>
 
 namespace ncamd {
 
+// Neutrons and results of a batch that the last-level cache (256 MB) cannot hold
+// pass by the caches, which are left to the tables: 3e7 neutrons, PowderBragg, 5000
+// and 262k planes, cross sections 189 -> 177 and 250 -> 234 us, sampling 347 -> 326
+// and 459 -> 430.  Smaller ones are often still there from the step that made
+// them: 1e7 neutrons, past the caches against through them, cross sections 56 and
+// 35 us (5000 planes), 76 and 58 (262k), sampling 104 and 64, 140 and 112.
+// (A variant of the kernels: of a branch at run time the compiler makes one access.)
+static inline bool past_caches(int64_t bytes) { return bytes > ((int64_t)256 << 20); }
+template <bool Past>
+NCD double load_stream(const double* __restrict__ p) {
+  if constexpr (Past) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool Past>
+NCD void store_stream(double x, double* __restrict__ p) {
+  if constexpr (Past) __builtin_nontemporal_store(x, p);
+  else *p = x;
+}
+
 // Variant kCompPBOnly: a single PowderBragg component (the same sum as
-// comp_xs: 0 + scale * xs); kCompFG: FreeGas / absorption components.  The
-// neutrons and results pass by the caches, which are left to the tables
-// (PowderBragg, 262k planes, 5e7 neutrons, both kernels: 1341 -> 1279 us)
-template <bool FP32PB, int Variant>
+// comp_xs: 0 + scale * xs); kCompFG: FreeGas / absorption components
+template <bool FP32PB, int Variant, bool Past>
 __global__ void __launch_bounds__(256) k_xs_iso(CompView c, const double* __restrict__ ekin,
                                                 int64_t n, int64_t repeat, double* __restrict__ out) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const double E = __builtin_nontemporal_load(ekin + i);
+    const double E = load_stream<Past>(ekin + i);
     double xs;
     if constexpr (Variant == kCompPBOnly) {
       xs = comp_outside(c, E) ? 0.0 : 0.0 + c.scale[0] * (pb_active(c.pb, E) ? pb_xs_sel<FP32PB>(c.pb, E) : 0.0);
     } else {
       xs = comp_xs<FP32PB, Variant == kCompFG>(c, E, nullptr);  // kCompFG: any composition with gas components
     }
-    for (int64_t r = 0; r < repeat; ++r) __builtin_nontemporal_store(xs, out + r * n + i);
+    for (int64_t r = 0; r < repeat; ++r) store_stream<Past>(xs, out + r * n + i);
   }
 }
 
-template <int Variant>
+template <int Variant, bool Past>
 __global__ void __launch_bounds__(256) k_sample_iso(CompView c, const double* __restrict__ ekin,
                                                     int64_t n, int64_t total, uint64_t seed,
                                                     uint32_t stream, double* __restrict__ oE,
@@ -43,10 +61,10 @@ __global__ void __launch_bounds__(256) k_sample_iso(CompView c, const double* __
     Rng rng;
     rng.init(seed, stream, (uint64_t)k);
     double Ef, mu;
-    const int rc = comp_sample_iso<Variant>(c, rng, __builtin_nontemporal_load(ekin + i), Ef, mu);
+    const int rc = comp_sample_iso<Variant>(c, rng, load_stream<Past>(ekin + i), Ef, mu);
     if (rc) { Ef = -1.0; mu = -999.0; atomicAdd(nerr, 1ull); }
-    __builtin_nontemporal_store(Ef, oE + k);
-    __builtin_nontemporal_store(mu, oMu + k);
+    store_stream<Past>(Ef, oE + k);
+    store_stream<Past>(mu, oMu + k);
   }
 }
 
@@ -665,35 +683,37 @@ void launch_xs_iso(const CompView& c, const double* ekin, int64_t n, int64_t rep
                    bool fp32, hipStream_t st) {
   if (n <= 0 || repeat <= 0) return;
   const dim3 g(grid_for(n, 256)), b(256);
+  const bool past = past_caches(8 * n * (1 + repeat));
   const int v = comp_variant(c);
-  if (v == kCompPBOnly) {
-    if (fp32) hipLaunchKernelGGL((k_xs_iso<true, kCompPBOnly>), g, b, 0, st, c, ekin, n, repeat, out);
-    else hipLaunchKernelGGL((k_xs_iso<false, kCompPBOnly>), g, b, 0, st, c, ekin, n, repeat, out);
-  } else if (v == kCompFG || comp_has_gas(c)) {
-    if (fp32) hipLaunchKernelGGL((k_xs_iso<true, kCompFG>), g, b, 0, st, c, ekin, n, repeat, out);
-    else hipLaunchKernelGGL((k_xs_iso<false, kCompFG>), g, b, 0, st, c, ekin, n, repeat, out);
-  } else {
-    if (fp32) hipLaunchKernelGGL((k_xs_iso<true, kCompNoSAB>), g, b, 0, st, c, ekin, n, repeat, out);
-    else hipLaunchKernelGGL((k_xs_iso<false, kCompNoSAB>), g, b, 0, st, c, ekin, n, repeat, out);
-  }
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, st, c, ekin, n, repeat, out); };
+  const auto variant = [&](auto kind) {
+    constexpr int V = decltype(kind)::value;
+    if (fp32) past ? go(k_xs_iso<true, V, true>) : go(k_xs_iso<true, V, false>);
+    else past ? go(k_xs_iso<false, V, true>) : go(k_xs_iso<false, V, false>);
+  };
+  if (v == kCompPBOnly) variant(std::integral_constant<int, kCompPBOnly>{});
+  else if (v == kCompFG || comp_has_gas(c)) variant(std::integral_constant<int, kCompFG>{});
+  else variant(std::integral_constant<int, kCompNoSAB>{});
 }
 void launch_sample_iso(const CompView& c, const double* ekin, int64_t n, int64_t repeat, uint64_t seed,
                        uint32_t stream, double* oE, double* oMu, unsigned long long* nerr, int64_t* queues,
                        unsigned long long* qcount, hipStream_t st) {
   const int64_t total = n * repeat;
   if (total <= 0) return;
+  const bool past = past_caches(8 * n + 16 * total);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid_for(total, 256)), dim3(256), 0, st, c, ekin, n, total, seed, stream, oE, oMu,
+                       nerr);
+  };
   switch (comp_variant(c)) {
     case kCompPBOnly:
-      hipLaunchKernelGGL(k_sample_iso<kCompPBOnly>, dim3(grid_for(total, 256)), dim3(256), 0, st, c, ekin, n, total,
-                         seed, stream, oE, oMu, nerr);
+      past ? go(k_sample_iso<kCompPBOnly, true>) : go(k_sample_iso<kCompPBOnly, false>);
       break;
     case kCompNoSAB:
-      hipLaunchKernelGGL(k_sample_iso<kCompNoSAB>, dim3(grid_for(total, 256)), dim3(256), 0, st, c, ekin, n, total,
-                         seed, stream, oE, oMu, nerr);
+      past ? go(k_sample_iso<kCompNoSAB, true>) : go(k_sample_iso<kCompNoSAB, false>);
       break;
     case kCompFG:
-      hipLaunchKernelGGL(k_sample_iso<kCompFG>, dim3(grid_for(total, 256)), dim3(256), 0, st, c, ekin, n, total,
-                         seed, stream, oE, oMu, nerr);
+      past ? go(k_sample_iso<kCompFG, true>) : go(k_sample_iso<kCompFG, false>);
       break;
     default:
       launch_staged<false>(c, ekin, nullptr, n, total, seed, stream, oE, oMu, nerr, queues, qcount, st, nullptr,

@@ -48,3 +48,20 @@ def test_lookup_and_pick(core, oracle, n, kind):
     pick = np.searchsorted(fdm, u * fdm[idx])
     ref = np.where(on, 1.0 - 2.0 * (e2d[np.minimum(pick, len(e2d) - 1)] / np.where(on, e, 1.0)), 1.0)
     assert np.array_equal(ge, e) and np.array_equal(mu, ref)
+
+
+def test_batches_beyond_the_last_level_cache(core):
+    """17e6 neutrons, 272 MB and 408 MB of arrays, pass by the caches: the values of
+    smaller calls"""
+    rng = np.random.default_rng(1)
+    p = core.create_powderbragg(3000.0, *_planes(5000, "dense", rng), fp32_tables=False)
+    n, m = 17_000_001, 9_000_000
+    e = 10.0 ** rng.uniform(-4, 0, n)
+    xs = p.crossSectionIsotropic(e)
+    assert np.array_equal(xs[:m], p.crossSectionIsotropic(e[:m]))
+    assert np.array_equal(xs[m:], p.crossSectionIsotropic(e[m:]))
+    p.setRNGState(5, 0)
+    ge, mu = p.sampleScatterIsotropic(e)
+    p.setRNGState(5, 0)
+    assert np.array_equal(mu[:m], p.sampleScatterIsotropic(e[:m])[1])
+    assert np.array_equal(ge, e) and np.all(np.abs(mu) <= 1.0)
