@@ -69,8 +69,10 @@ def _dynamics(case):
     return [(f, {"freegas": HELIUM} if e == "gas" else _table(*e)) for f, e in CASES[case]]
 
 
+# staged within workgroups up to 131072 neutrons, through queues above
+@pytest.mark.parametrize("n", [5003, 150000])
 @pytest.mark.parametrize("case", list(CASES))
-def test_compound_matches_checker(amd, oracle, case):
+def test_compound_matches_checker(amd, oracle, case, n):
     C, core, materials = amd
     dyn = _dynamics(case)
     m = materials.Material(synth.fcc_powder(dcutoff=0.3), dynamics=dyn)
@@ -78,7 +80,6 @@ def test_compound_matches_checker(amd, oracle, case):
     g = m.scatter
     parts = core.composition_components(g)
     assert [s for _, s in parts] == [1.0, 1.0] + [f for f, _ in dyn]
-    n = 150000
     e = synth.energies_logu(n, 1e-5, 10.0, seed=5)
     assert np.max(_rel(g.crossSectionIsotropic(e), o.xs(e, nthreads=8))) <= 1e-12
     g.setRandomSeed(77)
@@ -101,13 +102,14 @@ def test_compound_matches_checker(amd, oracle, case):
         assert np.mean(f * c.crossSectionIsotropic(e) / tot) > 1e-2
 
 
-def test_repeat_matches_tiled_checker(amd, oracle):
-    """repeat > 1 (n x repeat queue entries per staged component)"""
+@pytest.mark.parametrize("n", [20001, 50001])  # 60003: within workgroups; 150003: queues
+def test_repeat_matches_tiled_checker(amd, oracle, n):
+    """repeat > 1 (n x repeat neutrons of n energies, queue entries per staged component)"""
     C, core, materials = amd
     dyn = _dynamics("three S(alpha,beta)")
     m = materials.Material(synth.fcc_powder(dcutoff=0.3), dynamics=dyn)
     o = _checker(oracle, materials, m, dyn)
-    e = synth.energies_logu(20001, 1e-4, 3.0, seed=6)
+    e = synth.energies_logu(n, 1e-4, 3.0, seed=6)
     m.scatter.setRandomSeed(5)
     ge, gm = m.scatter.sampleScatterIsotropic(e, repeat=3)
     oe, om, nerr = o.sample_iso(e, repeat=3, seed=5, nthreads=8)

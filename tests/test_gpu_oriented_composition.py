@@ -78,11 +78,12 @@ def _rel(a, b):
 
 @pytest.mark.parametrize("with_sab,only_scb,gas", [(True, False, False), (False, False, False), (False, True, False),
                                                    (True, False, True), (False, False, True)])
-def test_oriented_composition_matches_checker(amd, oracle, with_sab, only_scb, gas):
+# staged within workgroups up to 131072 neutrons, through queues above
+@pytest.mark.parametrize("n", [40000, 140001])
+def test_oriented_composition_matches_checker(amd, oracle, with_sab, only_scb, gas, n):
     C, core = amd
     g, o = _material(core, oracle, with_sab, only_scb, gas)
     assert C.call("ncamd_isoriented", g._h) == 1
-    n = 40000
     wl = synth.wavelengths_uniform(n, 0.5, 6.0, seed=4)
     e = 0.081804209605330899 / wl ** 2
     dirs = synth.cone_dirs(n, synth.random_unit_vector(2), 5 * math.pi / 180, seed=6)
