@@ -294,7 +294,7 @@ def run_c1(args):
                    "neutrons_per_step": n, "families": int(len(m.pb_inputs[1])), "setup_s": t_setup},
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "oriented sampling call (k_comp_pick + k_comp_sab + high-energy queue)",
+                     "kernel": "oriented sampling call (k_comp_pick + k_comp_sab)",
                      "kernel_ms": samp_ms, "bytes_per_neutron": 64, "xs_call_ms": xs_ms,
                      "xs_GBs": 16 * n / (xs_ms * 1e-3) / 1e9},
         "cpu_baseline": cpu,

@@ -2583,8 +2583,9 @@ void sample_dirs_dispatch(Proc* p, const double* ekin, const double* dirs, int64
 
 // isotropic sampling dispatch: S(alpha,beta)-only handles take the split
 // main/high-energy kernels, everything else the composition kernel
-// ext_q / ext_qc: caller-provided queue (2 x n x repeat entries) and 2
-// kMaxStaged counters; then no device memory is allocated here
+// ext_q / ext_qc: caller-provided queues (n x repeat entries per staged
+// component, n x repeat for a single S(alpha,beta)) and 2 kMaxStaged counters;
+// then no device memory is allocated here
 void sample_iso_dispatch(Proc* p, const double* ekin, int64_t n, int64_t repeat, double* oE, double* oMu,
                          hipStream_t st, int64_t* ext_q = nullptr, unsigned long long* ext_qc = nullptr) {
   if (p->oriented_comp) raise("BadInput", "oriented process: use the calls with neutron directions");
@@ -2626,7 +2627,7 @@ void sample_iso_dispatch(Proc* p, const double* ekin, int64_t n, int64_t repeat,
 }
 
 // ------------------------------------------ allocation-free sampling call ---
-// Fixed scratch for ncamd_dev_samplescatterisotropic_many_noalloc: two
+// Fixed scratch for ncamd_dev_samplescatterisotropic_many_noalloc: the
 // counters (in the first 256 bytes) and the sampling queues (two int64
 // entries per neutron) for at most kNoAllocMaxNeutrons neutrons per call,
 // 32 MiB + 256 B, held by every GPU the library runs on until the process
@@ -2634,6 +2635,7 @@ void sample_iso_dispatch(Proc* p, const double* ekin, int64_t n, int64_t repeat,
 // array's name.
 constexpr int64_t kNoAllocMaxNeutrons = int64_t(1) << 21;
 constexpr size_t kNoAllocCounterBytes = 256;
+static_assert(2 * kMaxStaged * sizeof(unsigned long long) <= kNoAllocCounterBytes, "counters of the staged queues");
 constexpr size_t kNoAllocBytes = kNoAllocCounterBytes + 2 * sizeof(int64_t) * (size_t)kNoAllocMaxNeutrons;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -3460,8 +3462,8 @@ void ncamd_dev_samplescatterisotropic_many_noalloc(ncamd_process_t h, const doub
   NCAMD_TRY
   Proc* p = extract(h);
   ensure_device();
-  // queue entries the call needs: n x repeat per staged component plus the
-  // high-energy queue (two queues for a single S(alpha,beta) stage)
+  // the documented limits: room for n x repeat entries per staged component and
+  // once more (the queues, filled from both ends, need the former)
   const uint64_t nq = is_absorption(p) || p->kind == kKindFG ? 2 : (uint64_t)make_view(p).nstaged + 1;
   const uint64_t cap = 2 * (uint64_t)kNoAllocMaxNeutrons;
   if (repeat && (n > cap / repeat || (uint64_t)n * repeat > cap / std::max<uint64_t>(nq, 2)))

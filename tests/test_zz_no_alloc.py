@@ -85,3 +85,20 @@ def test_noalloc_refuses_oversized_calls(env):
     with pytest.raises(C.NCBadInput):
         C.check()
     assert pb.getRNGState() == before  # refused before any launch
+
+
+def test_two_components_at_the_limit(env):
+    """two staged components: 2/3 of the limit, and one more is refused"""
+    C, core, materials = env
+    t, t2 = synth.small_sab_table(mass_amu=26.98), synth.small_sab_table(seed=5, mass_amu=15.999, amax=60.0)
+    parts = [core.create_sabscatter(x["alpha"], x["beta"], x["sab"], x["temperature"], x["mass"], x["sigma_bound"])
+             for x in (t, t2)]
+    proc = core.create_composition(parts, [0.5, 0.5])
+    n = (1 << 22) // 3
+    st = C.Stream()
+    de = C.DeviceArray.from_numpy(synth.energies_logu(n + 1, 1e-5, 5.0, seed=3))
+    a, b = (_run(C, proc, fn, de, n, 1, st) for fn in ("alloc", "noalloc"))
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    C.lib().ncamd_dev_samplescatterisotropic_many_noalloc(proc.handle, de.ptr, n + 1, 1, de.ptr, de.ptr, st.ptr)
+    with pytest.raises(C.NCBadInput):
+        C.check()
