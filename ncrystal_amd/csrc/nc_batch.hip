@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(kBatchBlock) k_batch_sab(const BatchMat* __res
     const int skip = m.view.n > 1 ? 1 : 0;
     const SABView& view = m.view.sab[0];
     const SabSmall<Lds> small(view, lds);
-    const SabShare<kBatchBlock / 64> share(cnt, threadIdx.x >> 6, kBatchBlock / 64);
+    const SabRun share(cnt, threadIdx.x >> 6, kBatchBlock / 64, 64);
     sab_stream<false>(
         view, small, r.seed, (uint32_t)r.stream, skip, share,
         [&](int64_t i, int64_t& k, double& E) {

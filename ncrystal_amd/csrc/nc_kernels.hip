@@ -238,8 +238,7 @@ __global__ void __launch_bounds__(256, 4) k_comp_sab(SABView s, const double* __
   const int64_t m = queue_count(count, 0, total);
   if (m == 0) return;
   const SabSmall<Lds> small(s, lds);
-  const SabShare<> share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4,
-                       share_shift(m));
+  const SabShare share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4);
   sab_stream<Dirs>(
       s, small, seed, stream, skip, share,
       [&](int64_t i, int64_t& k, double& E) {
@@ -355,7 +354,7 @@ __global__ void __launch_bounds__(256, 4) k_comp_local(CompView c, const double*
     const SABView& s = c.sab[sl];
     if (low > 0) {
       const SabSmall<Lds> small(s, lds);
-      const SabShare<4> share(low, tid >> 6, 4, 5);
+      const SabRun share(low, tid >> 6, 4, 32);
       sab_stream<Dirs>(
           s, small, seed, stream, skip, share,
           [&](int64_t i, int64_t& k, double& E) {
@@ -436,7 +435,7 @@ __global__ void __launch_bounds__(256, 4) k_sab_sample_iso_main(SABView s, const
   if (lane == 0) *have = 0;
   __syncthreads();
   const SabSmall<Lds> small(s, lds);
-  const SabShare<> share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4, share_shift(total));
+  const SabShare share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4);
   const double emax = s.egrid[s.ne - 1];
   sab_stream<false>(
       s, small, seed, stream, 0, share,

@@ -184,23 +184,34 @@ NCD int egrid_sampler(const SABView& s, const double* egrid, double E) {
 // larger ones cost less (3e7 neutrons: 2.56 ms with 64, 2.52 with 256; one run each:
 // 2.55).
 NCD int share_shift(int64_t n) { return n > (1 << 24) ? 8 : 6; }
-template <int NW = 0>  // nw, where it is fixed
 struct SabShare {
   uint32_t nw;
   int shift;
   int64_t w, size;
-  NCD SabShare(int64_t n, int64_t wave, int64_t nwaves, int sh = 6)
-      : nw(NW ? NW : (uint32_t)nwaves), shift(sh), w(wave), size(0) {
-    const int64_t pieces = (n + (1 << sh) - 1) >> sh;
+  NCD SabShare(int64_t n, int64_t wave, int64_t nwaves)
+      : nw((uint32_t)nwaves), shift(share_shift(n)), w(wave), size(0) {
+    const int64_t pieces = (n + (1 << shift) - 1) >> shift;
     if (w >= pieces) return;
-    size = ((pieces - w + nw - 1) / nw) << sh;
-    if ((pieces - 1 - w) % nw == 0) size -= (pieces << sh) - n;  // the list's last piece
+    size = ((pieces - w + nw - 1) / nw) << shift;
+    if ((pieces - 1 - w) % nw == 0) size -= (pieces << shift) - n;  // the list's last piece
   }
   // (a wave's pieces are fewer than 2^32)
   NCD int64_t at(int64_t i) const {
-    const uint64_t piece = (uint64_t)(uint32_t)(i >> shift) * (NW ? NW : nw) + (uint64_t)w;
+    const uint64_t piece = (uint64_t)(uint32_t)(i >> shift) * nw + (uint64_t)w;
     return (int64_t)(piece << shift) | (i & ((1 << shift) - 1));
   }
+};
+// The same of a workgroup's own short list: one run, at least `fill` places
+struct SabRun {
+  int64_t begin, size;
+  NCD SabRun(int n, int wave, int nwaves, int fill) {
+    int per = (n + nwaves - 1) / nwaves;
+    per = per < fill ? fill : per;
+    const int b = wave * per < n ? wave * per : n;
+    begin = b;
+    size = b + per < n ? per : n - b;
+  }
+  NCD int64_t at(int64_t i) const { return begin + i; }
 };
 
 // Samples the neutrons of a wave's share of a list, all lanes of the wave
