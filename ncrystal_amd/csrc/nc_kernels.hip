@@ -611,11 +611,14 @@ void launch_stages(const CompView& c, const double* ekin, const double* dirs, in
 }
 
 
-// Batches of at most 512 workgroups of 256 neutrons are staged within workgroups
-// (rock salt, two S(alpha,beta) components, isotropic call of 100003 neutrons: 67
-// against 99 us through the queues; powder, 1000 neutrons: 31 against 52 us; rock
-// salt, 1e6: 227 against 195 us, where full waves count more).
-constexpr int64_t kLocalMax = 512 * 256;
+// Batches of at most 1024 workgroups of 256 neutrons, what the chip holds at once
+// (four to a CU), are staged within workgroups; beyond, the second round's
+// workgroups cost more than the queues.  Within workgroups against through queues
+// [us], isotropic calls, powder (one S(alpha,beta)) and rock salt (two):
+//   neutrons      1000     100000     200000     260000     300000     1000000
+//   powder      27   43   48   58    63   65    66   70    95   81   208  151
+//   rock salt   39   76   67  101    78  106    81  110   119  126   261  194
+constexpr int64_t kLocalMax = 1024 * 256;
 bool staged_locally(int64_t total) { return total <= kLocalMax; }
 template <bool Dirs>
 void launch_staged(const CompView& c, const double* ekin, const double* dirs, int64_t n, int64_t total, uint64_t seed,

@@ -69,8 +69,8 @@ def _dynamics(case):
     return [(f, {"freegas": HELIUM} if e == "gas" else _table(*e)) for f, e in CASES[case]]
 
 
-# staged within workgroups up to 131072 neutrons, through queues above
-@pytest.mark.parametrize("n", [5003, 150000])
+# staged within workgroups up to 262144 neutrons, through queues above
+@pytest.mark.parametrize("n", [5003, 150000, 270001])
 @pytest.mark.parametrize("case", list(CASES))
 def test_compound_matches_checker(amd, oracle, case, n):
     C, core, materials = amd
@@ -102,7 +102,7 @@ def test_compound_matches_checker(amd, oracle, case, n):
         assert np.mean(f * c.crossSectionIsotropic(e) / tot) > 1e-2
 
 
-@pytest.mark.parametrize("n", [20001, 50001])  # 60003: within workgroups; 150003: queues
+@pytest.mark.parametrize("n", [20001, 90001])  # 60003: within workgroups; 270003: queues
 def test_repeat_matches_tiled_checker(amd, oracle, n):
     """repeat > 1 (n x repeat neutrons of n energies, queue entries per staged component)"""
     C, core, materials = amd

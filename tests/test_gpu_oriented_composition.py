@@ -78,8 +78,8 @@ def _rel(a, b):
 
 @pytest.mark.parametrize("with_sab,only_scb,gas", [(True, False, False), (False, False, False), (False, True, False),
                                                    (True, False, True), (False, False, True)])
-# staged within workgroups up to 131072 neutrons, through queues above
-@pytest.mark.parametrize("n", [40000, 140001])
+# staged within workgroups up to 262144 neutrons, through queues above
+@pytest.mark.parametrize("n", [40000, 270001])
 def test_oriented_composition_matches_checker(amd, oracle, with_sab, only_scb, gas, n):
     C, core = amd
     g, o = _material(core, oracle, with_sab, only_scb, gas)

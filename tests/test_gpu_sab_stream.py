@@ -57,10 +57,10 @@ def test_single_process(core, sab, n):
     _check((ge, gm), (oe, om), f"single {n}")
 
 
-@pytest.mark.parametrize("n", [1, 65, 1025, 40000, 131072, 131073])
+@pytest.mark.parametrize("n", [1, 65, 1025, 40000, 131072, 131073, 262144, 262145])
 def test_composition(core, oracle, sab, n):
     """two S(alpha,beta) components beside incoherent elastic: both ends of two
-    lists, within workgroups up to 131072 neutrons and in queues above"""
+    lists, within workgroups up to 262144 neutrons and in queues above"""
     g, o = sab
     t = synth.small_sab_table(seed=5, mass_amu=12.0)
     args = (t["alpha"], t["beta"], t["sab"], t["temperature"], t["mass"], t["sigma_bound"])
