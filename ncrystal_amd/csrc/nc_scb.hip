@@ -375,10 +375,10 @@ __global__ void __launch_bounds__(256) k_scb_xs_slow(SCBView v, const double* __
     }
     return;
   }
-  // (every lane of a wave has the same q)
-  for (int64_t q0 = first; q0 < nq; q0 += nwaves * group)
-  for (int64_t q = q0; q < nq && q < q0 + group; ++q) {
-    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(nq - q0 < group ? nq - q0 : group), W);
+  // (every lane of a wave has the same q; from the end, where the longest scans are)
+  for (int64_t q1 = nq - first; q1 > 0; q1 -= nwaves * group)
+  for (int64_t q0 = q1 > group ? q1 - group : 0, q = q0; q < q1; ++q) {
+    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(q1 - q0), W);
     const int64_t i = queue[q];
     ScbLane L;
     const bool can = scb_lane_setup(v, ekin[i], dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2], L);
@@ -552,10 +552,10 @@ __global__ void __launch_bounds__(256) k_scb_sample_slow(SCBView v, const double
     }
     return;
   }
-  // (every lane of a wave has the same q)
-  for (int64_t q0 = first; q0 < nq; q0 += nwaves * group)
-  for (int64_t q = q0; q < nq && q < q0 + group; ++q) {
-    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(nq - q0 < group ? nq - q0 : group), W);
+  // (every lane of a wave has the same q; from the end, where the longest scans are)
+  for (int64_t q1 = nq - first; q1 > 0; q1 -= nwaves * group)
+  for (int64_t q0 = q1 > group ? q1 - group : 0, q = q0; q < q1; ++q) {
+    if (q == q0) scb_wave_near(v, ekin, dirs, queue + q0, (int)(q1 - q0), W);
     const int64_t i = queue[q];
     const double E = ekin[i];
     const V3 din{dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
