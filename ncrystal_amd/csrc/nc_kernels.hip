@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(256, 4) k_comp_sab(SABView s, const double* __
   const int64_t m = queue_count(count, 0, total);
   if (m == 0) return;
   const SabSmall<Lds> small(s, lds);
-  const SabShare share(m, (int64_t)(blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (int64_t)(gridDim.x - nhigh) * 4);
+  const SabShare share(m, (blockIdx.x - nhigh) * 4 + (threadIdx.x >> 6), (gridDim.x - nhigh) * 4);
   sab_stream<Dirs>(
       s, small, seed, stream, skip, share,
       [&](int64_t i, int64_t& k, double& E) {
@@ -435,7 +435,7 @@ __global__ void __launch_bounds__(256, 4) k_sab_sample_iso_main(SABView s, const
   if (lane == 0) *have = 0;
   __syncthreads();
   const SabSmall<Lds> small(s, lds);
-  const SabShare share(total, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), (int64_t)gridDim.x * 4);
+  const SabShare share(total, blockIdx.x * 4 + (threadIdx.x >> 6), gridDim.x * 4);
   const double emax = s.egrid[s.ne - 1];
   sab_stream<false>(
       s, small, seed, stream, 0, share,

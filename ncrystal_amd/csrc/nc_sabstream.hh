@@ -184,16 +184,18 @@ NCD int egrid_sampler(const SABView& s, const double* egrid, double E) {
 // larger ones cost less (3e7 neutrons: 2.56 ms with 64, 2.52 with 256; one run each:
 // 2.55).
 NCD int share_shift(int64_t n) { return n > (1 << 24) ? 8 : 6; }
+// Places are numbered from begin to end, at(i) is the one in the list.
 struct SabShare {
   uint32_t nw;
   int shift;
-  int64_t w, size;
-  NCD SabShare(int64_t n, int64_t wave, int64_t nwaves)
-      : nw((uint32_t)nwaves), shift(share_shift(n)), w(wave), size(0) {
+  int64_t w, end;
+  static constexpr int64_t begin = 0;
+  NCD SabShare(int64_t n, unsigned wave, unsigned nwaves)
+      : nw(nwaves), shift(share_shift(n)), w(__builtin_amdgcn_readfirstlane(wave)), end(0) {
     const int64_t pieces = (n + (1 << shift) - 1) >> shift;
     if (w >= pieces) return;
-    size = ((pieces - w + nw - 1) / nw) << shift;
-    if ((pieces - 1 - w) % nw == 0) size -= (pieces << shift) - n;  // the list's last piece
+    end = ((pieces - w + nw - 1) / nw) << shift;
+    if ((pieces - 1 - w) % nw == 0) end -= (pieces << shift) - n;  // the list's last piece
   }
   // (a wave's pieces are fewer than 2^32)
   NCD int64_t at(int64_t i) const {
@@ -203,15 +205,15 @@ struct SabShare {
 };
 // The same of a workgroup's own short list: one run, at least `fill` places
 struct SabRun {
-  int64_t begin, size;
-  NCD SabRun(int n, int wave, int nwaves, int fill) {
+  int64_t begin, end;
+  NCD SabRun(int n, int w, int nwaves, int fill) {
+    const int wave = __builtin_amdgcn_readfirstlane(w);
     int per = (n + nwaves - 1) / nwaves;
     per = per < fill ? fill : per;
-    const int b = wave * per < n ? wave * per : n;
-    begin = b;
-    size = b + per < n ? per : n - b;
+    begin = wave * per < n ? wave * per : n;
+    end = begin + per < n ? begin + per : n;
   }
-  NCD int64_t at(int64_t i) const { return begin + i; }
+  NCD int64_t at(int64_t i) const { return i; }
 };
 
 // Samples the neutrons of a wave's share of a list, all lanes of the wave
@@ -239,7 +241,7 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
   bool ultra = false;
   // the neutron's stream: index of its next number; the last block made (its
   // number and halves), whose second half is kept while the index is odd
-  int64_t next = 0;
+  int64_t next = share.begin;
   uint32_t drawn = 0, blk = 0;
   uint64_t h0 = 0, h1 = 0;
   const auto block = [&](uint32_t b) {
@@ -264,8 +266,8 @@ NCD void sab_stream(const SABView& s, const Small& small, uint64_t seed, uint32_
   };
   while (true) {
     uint64_t idle = __ballot(mode == kIdle);
-    while (idle && next < share.size) {
-      const int64_t room = share.size - next;
+    while (idle && next < share.end) {
+      const int64_t room = share.end - next;
       const int cnt = room < (int64_t)__popcll(idle) ? (int)room : __popcll(idle);
       if (mode == kIdle) {
         const int rank = __popcll(idle & below);
