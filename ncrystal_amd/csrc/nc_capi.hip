@@ -152,6 +152,7 @@ class HostStage {
   double* host(int i) const { return host_ + i * kHostStage; }
   double* dev(int i) const { return dev_ + i * kHostStage; }
   unsigned long long* count() const { return reinterpret_cast<unsigned long long*>(host_ + kArrays * kHostStage); }
+  unsigned long long* dev_count() const { return reinterpret_cast<unsigned long long*>(dev_ + kArrays * kHostStage); }
 
  private:
   static constexpr size_t kArrays = 3;
@@ -3313,8 +3314,8 @@ void ncamd_samplescatterisotropic_many(ncamd_process_t h, const double* ekin, un
     const HostStage st;
     std::copy(ekin, ekin + n, st.host(0));
     sample_iso_dispatch(p, st.dev(0), (int64_t)n, (int64_t)repeat, st.dev(1), st.dev(2), 0);
+    launch_copy_u64(p->d_err.as<unsigned long long>(), st.dev_count(), 0);
     NCAMD_HIP(hipGetLastError());
-    NCAMD_HIP(hipMemcpyAsync(st.count(), p->d_err.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, 0));
     NCAMD_HIP(hipStreamSynchronize(0));
     const unsigned long long nerr = *st.count();
     if (nerr) {

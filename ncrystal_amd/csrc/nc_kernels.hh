@@ -216,6 +216,7 @@ void launch_kb_sample_ab(const SABView&, const KBView&, const double* ekin, int6
                          int maxtries, hipStream_t);
 // helpers shared with the S(alpha,beta) kernels (nc_kernels.hip)
 void launch_zero_u64(unsigned long long* p, hipStream_t);
+void launch_copy_u64(const unsigned long long* from, unsigned long long* to, hipStream_t);
 // drains a queue of neutron indices with the plain sampler (from draw 0)
 void launch_sab_queue(const SABView&, const double* ekin, int64_t n, int64_t total, uint64_t seed, uint32_t stream,
                       double* oE, double* oMu, unsigned long long* nerr, const int64_t* queue,

@@ -779,6 +779,12 @@ void launch_sab_sample_iso(const SABView& s, const double* ekin, int64_t n, int6
   hipLaunchKernelGGL(k_sab_sample_iso_highe, dim3(grid_for(total, 256)), dim3(256), 0, st, s, ekin, n, total, seed,
                      stream, oE, oMu, nerr, queue, qcount);
 }
+__global__ void k_copy_u64(const unsigned long long* __restrict__ from, unsigned long long* __restrict__ to) {
+  *to = *from;
+}
+void launch_copy_u64(const unsigned long long* from, unsigned long long* to, hipStream_t st) {
+  hipLaunchKernelGGL(k_copy_u64, dim3(1), dim3(1), 0, st, from, to);
+}
 void launch_zero_u64(unsigned long long* p, hipStream_t st) {
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, p);
 }
