@@ -955,14 +955,14 @@ __global__ void __launch_bounds__(kLc0Threads, 4) k_lc0(LC0View L, SCBView v, co
 
 // neutrons of a workgroup: 64 where that gives every CU two workgroups, fewer
 // for small batches, so that a batch still spreads over the chip; 128 and 256
-// where that leaves the chip filled 2 and 4 times.  Many share the steps' latencies
-// where few have ranges (3e5 neutrons, 4.3-6 Aa, cross sections: 60 us with 64, 25
-// with 128, 21 with 256), but even out worse where most have (0.5-7 Aa: 131072
-// neutrons 2.20 ms with 64 and 2.30 with 128 for both calls, 3e5 1.96 with 64, 2.05
-// with 128 and 2.54 with 256, 1e6 5.59 with 128 and 6.08 with 256).
+// where that leaves the chip filled 2 and 8 times.  Many share the steps' latencies
+// where few have ranges (4.3-6 Aa, cross sections: 3e5 neutrons 25 us with 128, 21
+// with 256; 2^21 126 and 73), but even out worse where most have (0.5-7 Aa, both
+// calls of 131072 neutrons 2.20 ms with 64, 2.30 with 128; cross sections of 2^20
+// 6.06 ms with 128, 6.35 with 256; of 2^21 11.6 and 12.0).
 int lc0_group(int64_t n) {
   int nb = kLc0Threads;
-  while (nb > 4 && n < (int64_t)(nb > 128 ? 4096 : (nb > 64 ? 2048 : 512)) * nb) nb >>= 1;
+  while (nb > 4 && n < (int64_t)(nb > 128 ? 8192 : (nb > 64 ? 2048 : 512)) * nb) nb >>= 1;
   return nb;
 }
 

@@ -55,7 +55,7 @@ def test_batch_size_changes_nothing(core, lo, hi, mosaic):
 
 # workgroups of 128 and 256 neutrons: all beyond the last wavelength, around it,
 # with the first plane set alone, with a few, and every kind mixed
-@pytest.mark.parametrize("n", [262147, 1048581])
+@pytest.mark.parametrize("n", [262147, 2097157])
 @pytest.mark.parametrize("lo,hi", [(6.9, 9.0), (6.6, 6.8), (4.3, 6.0), (3.0, 4.0), (1.0, 9.0)])
 def test_sparse_batches(core, n, lo, hi):
     lc = _layered(core, 0.5, 4.0)
