@@ -266,7 +266,7 @@ struct PBView {
   double c_scale;       // c_n / all
 };
 // The lookups are bound by their loads, each lane's at a place of its own: the
-// address unit is busy 85% of the time.  So a bucket carries the value that
+// address unit is busy 82% of the time.  So a bucket carries the value that
 // belongs to its first answer, which most lanes need nothing beyond, a search
 // keeps the partner of the value it ends at, and each is one 16-byte load (the
 // vector types: of a struct the compiler makes two).  262k planes, 5e7 neutrons,

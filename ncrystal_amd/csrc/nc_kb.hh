@@ -58,7 +58,7 @@ struct alignas(64) KBSlot {
 };
 // Its 16-byte quarters, each one load, both of the head at once (of struct
 // members the compiler makes one load each, the head's in turn).  What bounds
-// the sampler is the lines that miss the dies' L2 caches, 2.3 a neutron, 6.6 TB/s:
+// the sampler is the lines that miss the dies' L2 caches, 2.0 a neutron, 5.6 TB/s:
 // the records of 256 intervals x 4096 boxes are 67 MB.  Half-size records, with
 // the w-edges and cell ranges in tables of their own, miss as often and add
 // accesses.  1e8 neutrons: 4603 -> 4469 us (half-size: 4768).

@@ -162,8 +162,10 @@ NCD LC0Raw lc0_raw_setup(double wl, double inv2d, double fsq) {
   return r;
 }
 // cos(phi) for phi in [0, pi]: phi = j pi/2 + r + rl with |r| <= pi/4 and the
-// Taylor series of sine and cosine at r.  Half the instructions of the general
-// cosine, whose argument may be of any size.
+// Taylor series of sine and cosine at r, the cosine's 1 - r^2/2 + .. with the
+// rounding of its first two terms added back (the usual compensated tail) and rl's
+// share.  Half the instructions of the general cosine, whose argument may be of any
+// size.
 NCD double lc0_cos(double phi) {
   const double j = rint(phi * 0.63661977236758134308);
   const double t = fma(-j, kPiHalf, phi);  // exact

@@ -22,12 +22,11 @@ namespace ncamd {
 // What bounds it is the cache: a wave's lanes sit at unrelated places of the
 // tables, so a load costs one access per lane whatever its width (up to 16
 // bytes), and the accesses per neutron set the pace (the address unit is busy
-// about 80 % of the time, the FP64 units 30 %).  So what is used together lies
-// together (SabPt, SabHead, SabBin), a guide's two ends are one load, guides are
-// fine enough that few searches need a probe, and the tables of one value per
-// grid point are kept in LDS.  3e7 neutrons, 200 x 800 table: 4.68 ms with one
-// lane per neutron, 3.88 ms streamed (44 accesses per neutron), 2.53 ms with this
-// layout (27).
+// three quarters of the time).  So what is used together lies together (SabPt,
+// SabHead, SabBin), a guide's two ends are one load, guides are fine enough that few
+// searches need a probe, and the tables of one value per grid point are kept in
+// LDS.  3e7 neutrons, 200 x 800 table: 4.68 ms with one lane per neutron, 3.88 ms
+// streamed (44 accesses per neutron), 2.50 ms with this layout (26).
 
 // The small tables (SABView::small), in LDS where they fit.  The constructor
 // fills lds; the whole workgroup calls it.
